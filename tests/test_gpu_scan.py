@@ -202,3 +202,37 @@ def test_optimised_scan_matches_reference_kernel_at_production_shape(gpu):
     y2, s2 = gdn.gated_delta_scan(*t, use_kernel=False)
     assert max_rel(y1.cpu().numpy(), y2.cpu().numpy()) < 1e-5
     assert max_rel(s1.cpu().numpy(), s2.cpu().numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Dk, Dv, offset", [(32, 8, 0), (64, 17, 1), (128, 128, 0), (128, 9, 3), (256, 40, 0),
+                                            (256, 40, 2)])
+def test_scan_blocks_of_tokens_match_the_reference_kernel(gpu, dtype, Dk, Dv, offset):
+    """Runs of 0 to 49 tokens around the scan's 16-token blocks, partial row
+    tiles, and q and k starting `offset` elements into their storage (rows
+    that no wide load may assume aligned), against the per-row kernel. Both
+    take the same inputs and sum in float32, at most 256 products of size
+    ~1/Dk a sum: 1e-5 of the largest value."""
+
+    rng = np.random.default_rng(3)
+    lens = [1, 15, 0, 16, 17, 32, 33, 49]
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    T, Hk, Hv, N = int(cu[-1]), 2, 4, len(lens)
+
+    def rows(*shape, unit=False):
+        x = rng.standard_normal(shape)
+        if unit:
+            x /= np.linalg.norm(x, axis=-1, keepdims=True)
+        flat = torch.zeros(x.size + offset, dtype=dtype, device=gpu)
+        flat[offset:] = torch.tensor(x.ravel(), device=gpu)
+        return flat[offset:].view(*shape)
+
+    q, k, v = rows(T, Hk, Dk, unit=True), rows(T, Hk, Dk, unit=True), rows(T, Hv, Dv)
+    a, b = rows(T, Hv), rows(T, Hv)
+    A_log, dt = (torch.tensor(rng.uniform(-1, 1, Hv), dtype=torch.float32, device=gpu) for _ in range(2))
+    s0 = torch.tensor(rng.standard_normal((N, Hv, Dv, Dk)) * 0.05, dtype=torch.float32, device=gpu)
+    y1, s1 = gdn.gated_delta_update(q, k, v, a, b, A_log, dt, s0, cu_seqlens=cu)
+    y2, s2 = gdn.gated_delta_update(q, k, v, a, b, A_log, dt, s0, cu_seqlens=cu, use_kernel=False)
+    assert max_rel(y1.cpu().numpy(), y2.cpu().numpy()) < 1e-5
+    assert max_rel(s1.cpu().numpy(), s2.cpu().numpy()) < 1e-5
+    assert torch.equal(s1[2], s0[2])  # the empty run's
