@@ -2,7 +2,7 @@
 // q/k scaling, for N packed token runs (linear_attention.py:61-79,103-113).
 //
 // Two kernels. The tiled one covers the production shape (Dk = Dv = 128,
-// K = 4, bf16 activations, 16-byte aligned operands): a wave holds four
+// K = 4, 16-byte aligned operands): a wave holds four
 // 128-channel groups (q, k or v heads) of one token, 8 channels a lane, and
 // walks a tile of 4-16 tokens with the previous three input rows in registers, so
 // each qkv row is read once per tile plus a three-row halo, with 16-byte
@@ -114,6 +114,96 @@ __global__ __launch_bounds__(kFrontThreads) void frontend_kernel(
 }
 
 
+// A lane's 8 channels of a 128-channel group held by 16 lanes, in the tiled
+// kernel's activation type: the loads and stores of a token's row, the conv
+// state and taps as the general kernel rounds them, and its conv, SiLU and
+// scaled norm. bf16: channels 8l .. 8l + 7 (16 bytes). float32: channels
+// 4l .. 4l + 3 and 64 + 4l .. (two 16-byte pieces, each 256 contiguous bytes
+// over the 16 lanes); SiLU from expf and an IEEE divide and the norm in
+// double, each value rounded once, as the decode step does.
+template <class Act>
+struct Lane8;
+
+template <>
+struct Lane8<ActBF16> {
+    using Raw = uint4;
+    static constexpr int kAhead = 8;  // rows in flight
+    static GDN_DEV int first(int l16) { return 8 * l16; }
+    static GDN_DEV Raw load(const uint16_t* p) { return *reinterpret_cast<const uint4*>(p); }
+    static GDN_DEV void unpack(const Raw& r, float (&x)[8]) { unpack8(r, x); }
+    static GDN_DEV void store(uint16_t* p, const float (&o)[8]) { *reinterpret_cast<uint4*>(p) = pack8(o); }
+    template <int kConvDt>
+    static GDN_DEV void state(const void* p, int64_t at, float (&x)[8]) { load_state8<kConvDt>(p, at, x); }
+    static GDN_DEV void taps(const float* w, int64_t c0, float (&wr)[8][4]) { load_conv_w8(w, c0, wr); }
+    static GDN_DEV void conv_silu(const float (&wr)[8][4], const float (&win)[3][8], const float (&x)[8],
+                                  float (&o)[8]) {
+        conv_silu8(wr, win, x, o);
+    }
+    static GDN_DEV void norm(const float (&o)[8], float sc, float (&n)[8]) {
+        rms_norm8(o, n);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n[e] = sc * n[e];
+    }
+};
+
+template <>
+struct Lane8<ActF32> {
+    struct Raw {
+        float4 a, b;
+    };
+    static constexpr int kAhead = 4;
+    static GDN_DEV int first(int l16) { return 4 * l16; }
+    static GDN_DEV Raw load(const float* p) {
+        return {*reinterpret_cast<const float4*>(p), *reinterpret_cast<const float4*>(p + 64)};
+    }
+    static GDN_DEV void unpack(const Raw& r, float (&x)[8]) {
+        const float v[8] = {r.a.x, r.a.y, r.a.z, r.a.w, r.b.x, r.b.y, r.b.z, r.b.w};
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = v[e];
+    }
+    static GDN_DEV void store(float* p, const float (&o)[8]) {
+        *reinterpret_cast<float4*>(p) = make_float4(o[0], o[1], o[2], o[3]);
+        *reinterpret_cast<float4*>(p + 64) = make_float4(o[4], o[5], o[6], o[7]);
+    }
+    template <int kConvDt>
+    static GDN_DEV void state(const void* p, int64_t at, float (&x)[8]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (kConvDt == GDN_F32) {
+                const float4 v = *reinterpret_cast<const float4*>(static_cast<const float*>(p) + at + 64 * h);
+                x[4 * h] = v.x, x[4 * h + 1] = v.y, x[4 * h + 2] = v.z, x[4 * h + 3] = v.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[4 * h + e] = load_any(p, at + 64 * h + e, kConvDt);
+            }
+        }
+    }
+    static GDN_DEV void taps(const float* w, int64_t c0, float (&wr)[8][4]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float4 v = *reinterpret_cast<const float4*>(w + (c0 + (e & 3) + 64 * (e >> 2)) * 4);
+            wr[e][0] = v.x, wr[e][1] = v.y, wr[e][2] = v.z, wr[e][3] = v.w;
+        }
+    }
+    static GDN_DEV void conv_silu(const float (&wr)[8][4], const float (&win)[3][8], const float (&x)[8],
+                                  float (&o)[8]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float xs[4] = {win[0][e], win[1][e], win[2][e], x[e]};
+            o[e] = conv_chain(4, [&](int j) { return float2{wr[e][j], xs[j]}; });
+        }
+        silu_act<GDN_F32>(o);
+    }
+    static GDN_DEV void norm(const float (&o)[8], float sc, float (&n)[8]) {
+        double ss = 0.0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss = fma(double(o[e]), double(o[e]), ss);
+        const double rr = rms_rr(group_sum<16>(ss), 128);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n[e] = sc * float(double(o[e]) * rr);
+    }
+};
+
 constexpr int kMaxTileTokens = 16;  // tokens a wave walks, at most
 constexpr int kTileWaves = 4;    // waves a block, four channel groups each
 
@@ -130,12 +220,18 @@ constexpr int kStateChunk = kTileWaves * kWave * 8;  // conv-state elements a bl
 // run's tokens) for the token t in hand: it is loaded so at the tile's first
 // token and reloaded from the conv state where a run starts inside the tile,
 // and each token shifts itself in.
-template <int kConvDt, int kTileTokens>
+//
+// float32, T = 1531, C = 8192 (50 MB in, 50 MB out): 25 us (3.9 TB/s) against
+// 117 us on the general kernel (a block per token, scalar loads, every tap's
+// row read again); what is left over the copy's 20 us is the expf and divide
+// of SiLU.
+template <class Act, int kConvDt, int kTileTokens>
 __global__ __launch_bounds__(kTileWaves * kWave) void frontend_tiled_kernel(
-    const uint16_t* __restrict__ qkv, int64_t qs, const void* __restrict__ cs_in,
-    uint16_t* __restrict__ cs_out, const float* __restrict__ w, const int32_t* __restrict__ cu,
-    int N, int64_t T, int64_t L_uniform, int n_state, uint16_t* __restrict__ qo,
-    uint16_t* __restrict__ ko, uint16_t* __restrict__ vo, int Hk, int Hv) {
+    const typename Act::storage* __restrict__ qkv, int64_t qs, const void* __restrict__ cs_in,
+    typename Act::storage* __restrict__ cs_out, const float* __restrict__ w, const int32_t* __restrict__ cu,
+    int N, int64_t T, int64_t L_uniform, int n_state, typename Act::storage* __restrict__ qo,
+    typename Act::storage* __restrict__ ko, typename Act::storage* __restrict__ vo, int Hk, int Hv) {
+    using Lane = Lane8<Act>;
     constexpr int D = 128, K = 4, S = K - 1;
     const int G = 2 * Hk + Hv;
     const int C = G * D;
@@ -151,14 +247,14 @@ __global__ __launch_bounds__(kTileWaves * kWave) void frontend_tiled_kernel(
                 const int j = int(e / C % S), c = int(e % C);
                 const int64_t start = cu ? cu[run] : run * L_uniform;
                 const int64_t idx = (cu ? cu[run + 1] - cu[run] : L_uniform) + j;  // in concat(state, run)
-                x[i] = idx < S ? round_bf16(load_any(cs_in, (int64_t(run) * S + idx) * C + c, kConvDt))
-                               : ActBF16::load(qkv, (start + idx - S) * qs + c);
+                x[i] = idx < S ? Act::round(load_any(cs_in, (int64_t(run) * S + idx) * C + c, kConvDt))
+                               : Act::load(qkv, (start + idx - S) * qs + c);
             }
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int64_t e = first + int64_t(i) * kTileWaves * kWave;
-            if (e < total) ActBF16::store(cs_out, e, x[i]);
+            if (e < total) Act::store(cs_out, e, x[i]);
         }
         return;
     }
@@ -167,17 +263,17 @@ __global__ __launch_bounds__(kTileWaves * kWave) void frontend_tiled_kernel(
     if (g0 >= G) return;  // the whole wave idles; the kernel has no barrier
     const int g = g0 + lane / 16;
     const bool live = g < G;
-    const int c0 = (live ? g : G - 1) * D + (lane % 16) * 8;  // this lane's 8 channels
+    const int c0 = (live ? g : G - 1) * D + Lane::first(lane % 16);  // this lane's first channel
     const int64_t t0 = (int64_t(blockIdx.x) - n_state) * kTileTokens;
 
     // the tile's rows, kAhead in flight (the last tile's missing ones repeat
     // row T-1, unused)
-    constexpr int kAhead = kTileTokens < 8 ? kTileTokens : 8;
+    constexpr int kAhead = kTileTokens < Lane::kAhead ? kTileTokens : Lane::kAhead;
     const auto row_at = [&](int i) {
         const int64_t t = t0 + i < T ? t0 + i : T - 1;
-        return *reinterpret_cast<const uint4*>(qkv + t * qs + c0);
+        return Lane::load(qkv + t * qs + c0);
     };
-    uint4 raw[kAhead];
+    typename Lane::Raw raw[kAhead];
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) raw[i] = row_at(i);
     int run = cu ? find_run(cu, N, t0) : int(t0 / L_uniform);
@@ -188,25 +284,25 @@ __global__ __launch_bounds__(kTileWaves * kWave) void frontend_tiled_kernel(
     for (int j = 0; j < S; ++j) {
         const int64_t row = t0 - S + j;
         if (row >= start) {
-            unpack8(*reinterpret_cast<const uint4*>(qkv + row * qs + c0), win[j]);
+            Lane::unpack(Lane::load(qkv + row * qs + c0), win[j]);
         } else {  // concat index row - start + S of the run's conv state
-            load_state8<kConvDt>(cs_in, (int64_t(run) * S + (row - start + S)) * C + c0, win[j]);
+            Lane::template state<kConvDt>(cs_in, (int64_t(run) * S + (row - start + S)) * C + c0, win[j]);
         }
     }
     float wr[8][K];
-    load_conv_w8(w, c0, wr);
+    Lane::taps(w, c0, wr);
 
     const float inv = 1.f / sqrtf(float(D));
-    const float sc = g < Hk ? round_bf16(inv * inv) : round_bf16(inv);
+    const float sc = g < Hk ? Act::round(inv * inv) : Act::round(inv);
     const bool is_v = g >= 2 * Hk;
     // whether the wave holds a q or k head (uniform: a wave may also hold v
     // heads when Hk is not a multiple of 4; their lanes keep o)
     const bool qk_wave = __builtin_amdgcn_readfirstlane(int(g0 < 2 * Hk)) != 0;
-    uint16_t* dst = g < Hk ? qo + int64_t(g) * D
+    typename Act::storage* dst = g < Hk ? qo + int64_t(g) * D
                   : !is_v ? ko + int64_t(g - Hk) * D
                           : vo + int64_t(g - 2 * Hk) * D;
     const int64_t dst_row = is_v ? int64_t(Hv) * D : int64_t(Hk) * D;
-    dst += (lane % 16) * 8;
+    dst += Lane::first(lane % 16);
 
 #pragma unroll
     for (int i = 0; i < kTileTokens; ++i) {
@@ -217,20 +313,20 @@ __global__ __launch_bounds__(kTileWaves * kWave) void frontend_tiled_kernel(
             next = cu ? cu[run + 1] : t + L_uniform;
 #pragma unroll
             for (int j = 0; j < S; ++j)
-                load_state8<kConvDt>(cs_in, (int64_t(run) * S + j) * C + c0, win[j]);
+                Lane::template state<kConvDt>(cs_in, (int64_t(run) * S + j) * C + c0, win[j]);
         }
         float x[8];
-        unpack8(raw[i % kAhead], x);
+        Lane::unpack(raw[i % kAhead], x);
         if (i + kAhead < kTileTokens) raw[i % kAhead] = row_at(i + kAhead);
         float o[8];
-        conv_silu8(wr, win, x, o);
+        Lane::conv_silu(wr, win, x, o);
         if (qk_wave) {  // q and k heads: scaled RMS norm (v lanes keep o)
             float n[8];
-            rms_norm8(o, n);
+            Lane::norm(o, sc, n);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = is_v ? o[e] : sc * n[e];
+            for (int e = 0; e < 8; ++e) o[e] = is_v ? o[e] : n[e];
         }
-        if (live && t < T) *reinterpret_cast<uint4*>(dst + t * dst_row) = pack8(o);
+        if (live && t < T) Lane::store(dst + t * dst_row, o);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             win[0][e] = win[1][e];
@@ -273,8 +369,8 @@ extern "C" int gdn_frontend(const void* qkv, int64_t qkv_stride, const void* con
                 "gdn_frontend: null pointer");
     const int64_t L_uniform = cu_seqlens ? 0 : T_total / N;
     const auto aligned = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-    if (act_dtype == GDN_BF16 && Dk == 128 && Dv == 128 && K == 4 && T_total > 0 && aligned(qkv) &&
-        qkv_stride % 8 == 0 &&
+    if (Dk == 128 && Dv == 128 && K == 4 && T_total > 0 && aligned(qkv) &&
+        qkv_stride * dtype_size(act_dtype) % 16 == 0 &&
         aligned(conv_state_in) && aligned(conv_weight) && aligned(q_out) && aligned(k_out) &&
         aligned(v_out)) {
         const int G = 2 * Hk + Hv;
@@ -289,22 +385,26 @@ extern "C" int gdn_frontend(const void* qkv, int64_t qkv_stride, const void* con
         const int64_t gx = n_state + n_tiles;
         GDN_REQUIRE(gx < (1LL << 31) / (kTileWaves * kWave) && gy < 65536,
                     "gdn_frontend: %lld tokens exceed the grid", (long long)T_total);
-        using Kernel = void (*)(const uint16_t*, int64_t, const void*, uint16_t*, const float*, const int32_t*,
-                                int, int64_t, int64_t, int, uint16_t*, uint16_t*, uint16_t*, int, int);
-        const auto pick = [&](auto tt) -> Kernel {
+        const auto launch = [&](auto act, auto tt) {
+            using Act = decltype(act);
+            using St = typename Act::storage;
             constexpr int TT = decltype(tt)::value;
-            return conv_dtype == GDN_F32    ? frontend_tiled_kernel<GDN_F32, TT>
-                   : conv_dtype == GDN_BF16 ? frontend_tiled_kernel<GDN_BF16, TT>
-                                            : frontend_tiled_kernel<GDN_F16, TT>;
+            const auto kern = conv_dtype == GDN_F32    ? frontend_tiled_kernel<Act, GDN_F32, TT>
+                              : conv_dtype == GDN_BF16 ? frontend_tiled_kernel<Act, GDN_BF16, TT>
+                                                       : frontend_tiled_kernel<Act, GDN_F16, TT>;
+            hipLaunchKernelGGL(kern, dim3(unsigned(gx), unsigned(gy)), dim3(kTileWaves * kWave), 0,
+                               as_stream(stream), static_cast<const St*>(qkv), qkv_stride, conv_state_in,
+                               static_cast<St*>(conv_state_out), conv_weight, cu_seqlens, N, T_total, L_uniform,
+                               int(n_state), static_cast<St*>(q_out), static_cast<St*>(k_out),
+                               static_cast<St*>(v_out), Hk, Hv);
         };
-        const Kernel kern = tile == 16 ? pick(std::integral_constant<int, 16>{})
-                            : tile == 8 ? pick(std::integral_constant<int, 8>{})
-                                        : pick(std::integral_constant<int, 4>{});
-        hipLaunchKernelGGL(kern, dim3(unsigned(gx), unsigned(gy)), dim3(kTileWaves * kWave), 0,
-                           as_stream(stream), static_cast<const uint16_t*>(qkv), qkv_stride, conv_state_in,
-                           static_cast<uint16_t*>(conv_state_out), conv_weight, cu_seqlens, N,
-                           T_total, L_uniform, int(n_state), static_cast<uint16_t*>(q_out),
-                           static_cast<uint16_t*>(k_out), static_cast<uint16_t*>(v_out), Hk, Hv);
+        const auto by_tile = [&](auto act) {
+            if (tile == 16) launch(act, std::integral_constant<int, 16>{});
+            else if (tile == 8) launch(act, std::integral_constant<int, 8>{});
+            else launch(act, std::integral_constant<int, 4>{});
+        };
+        if (act_dtype == GDN_F32) by_tile(ActF32{});
+        else by_tile(ActBF16{});
         return check_launch("gdn_frontend");
     }
     const int64_t blocks = T_total + (S > 0 ? N : 0);

@@ -314,7 +314,7 @@ def test_gated_rms_norm_row_shapes_match_oracle(gpu, D, rows, x_dtype, misaligne
 @pytest.mark.parametrize("zdt", [torch.bfloat16, torch.float32])
 def test_gated_rms_norm_reads_a_column_view_of_z(gpu, zdt):
     """z as the (T, H, D) column view of a stacked projection output, read
-    in place (bf16: the vectorised kernel; float32: the general one): bit
+    in place (bf16: the vectorised kernel; float32 with a bf16 result: the general one): bit
     for bit the packed z."""
 
     rng = np.random.default_rng(12)
@@ -343,3 +343,59 @@ def test_gated_rms_norm_matches_oracle(gpu, dtype):
         assert_bf16_out_close(out.float().cpu().numpy(), expected)
     else:
         np.testing.assert_allclose(out.cpu().numpy(), expected, atol=1e-5, rtol=1e-5)
+
+
+@pytest.mark.parametrize("conv_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("Hk,Hv", [(16, 32), (3, 6), (1, 1)])
+def test_frontend_float32_tiles_match_the_oracle_and_the_general_kernel(gpu, Hk, Hv, conv_dtype):
+    """float32 activations at 128-wide heads (tiled) over runs that are
+    empty, shorter than the conv window or cross the tiles, a column view of
+    qkv, against the oracle (float32 rounding of four products, SiLU's expf
+    and one divide: 1e-6 of values of order 1) and against the general
+    kernel, which a misaligned qkv takes: the same conv and SiLU bits (v,
+    conv state), q and k from a double sum in another order, so equal up to
+    one float ulp."""
+
+    dims = gdn.LinearAttentionDims(Hk, Hv, 128, 128, 4)
+    rng = np.random.default_rng(18 + Hk)
+    lens = [0, 1, 2, 3, 16, 0, 37, 5, 70, 1]  # 135 tokens
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    T, C = int(cu[-1]), dims.conv_dim
+    qkv = rng.standard_normal((T, C)).astype(np.float32)
+    conv = R.bf16_round(rng.standard_normal((len(lens), 3, C)))
+    w = (rng.standard_normal((C, 4)) * 0.2).astype(np.float32)
+    stacked = torch.zeros(T, C + 12, device=gpu)
+    stacked[:, :C] = _t(qkv, gpu)
+    args = (_t(conv, gpu, conv_dtype), _t(w, gpu), dims, torch.tensor(cu, device=gpu))
+    tiled = gdn.conv_frontend(stacked[:, :C], *args)
+    flat = torch.zeros(T * C + 1, device=gpu)
+    flat[1:] = _t(qkv, gpu).reshape(-1)
+    general = gdn.conv_frontend(flat[1:].view(T, C), *args)
+    assert torch.equal(tiled[2], general[2]) and torch.equal(tiled[3], general[3])
+    for x, y in zip(tiled[:2], general[:2]):
+        torch.testing.assert_close(x, y, rtol=1.3e-7, atol=0)
+    for i, (t0, t1) in enumerate(zip(cu, cu[1:])):
+        out, new = R.convolve(qkv[t0:t1], conv[i], w)
+        np.testing.assert_array_equal(tiled[3][i].cpu().numpy(), new.astype(np.float32))
+        if t1 == t0:
+            continue
+        q, k = R.qk_scale(out[:, :Hk * 128].reshape(-1, Hk, 128), out[:, Hk * 128:2 * Hk * 128].reshape(-1, Hk, 128))
+        for got, want in zip(tiled, (q, k, out[:, 2 * Hk * 128:].reshape(-1, Hv, 128))):
+            np.testing.assert_allclose(got[t0:t1].cpu().numpy(), want, rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("D,rows", [(64, 13), (128, 21), (256, 7), (128, 1)])
+def test_gated_rms_norm_float32_rows_match_the_oracle_and_the_general_kernel(gpu, D, rows):
+    """float32 x, gate and result: 16-byte rows take the vectorised kernel
+    (the last wave part empty), a misaligned x the general one; within a few
+    float ulps of the oracle and of each other (sums in other orders)."""
+
+    rng = np.random.default_rng(D + rows)
+    y, z = (rng.standard_normal((rows, D)).astype(np.float32) for _ in range(2))
+    w = rng.uniform(0.5, 1.5, D).astype(np.float32)
+    flat = torch.zeros(rows * D + 1, device=gpu)
+    flat[1:] = _t(y, gpu).reshape(-1)
+    vec = gdn.gated_rms_norm(_t(y, gpu), _t(z, gpu), _t(w, gpu), 1e-6)
+    general = gdn.gated_rms_norm(flat[1:].view(rows, D), _t(z, gpu), _t(w, gpu), 1e-6)
+    np.testing.assert_allclose(vec.cpu().numpy(), R.gated_rms_norm(y, z, w, 1e-6), rtol=2e-6, atol=1e-7)
+    torch.testing.assert_close(vec, general, rtol=1e-6, atol=1e-7)
