@@ -693,6 +693,17 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // Tb and P are lower triangular, so the waves of token rows 0-31
 // (kUpper = false) fetch and multiply only their first 32 columns.
 constexpr int kStateThreads = 512;
+// A state-pass workgroup holds its CU to itself (256 registers a thread, the
+// prefetch ring three chunks deep), which suits a grid of one a CU: the chain
+// of chunk steps is all there is to hide. With more workgroups than CUs a
+// second one on the CU hides more than the deep ring does: bf16 calls above
+// 256 workgroups take prefill_state_shared_kernel (128 registers, 76 KB of
+// LDS, the same bits). Whole calls, us, one a CU against two: 3 runs of 2048
+// tokens at 16 heads (384 workgroups) 120 -> 116, one run of 2048 at 64 heads
+// (512) 131 -> 126, 3 x 777 at 32 (768) 86 -> 79, 32 x 64 at 16 (4096) 87 ->
+// 52, 16 packed runs of 67 128 tokens in all at 32 heads 2232 -> 2054. Float32
+// tiles (111 KB) leave no room for a second workgroup.
+constexpr int kStateSharedAbove = 256;
 
 // Chunk operands of state wave w, fetched by output wave w. They pass
 // through registers on the way to LDS, so each load covers whole rows (full
@@ -742,8 +753,8 @@ struct StatePassCtx {
 // token, which contribute nothing: their beta and log-decay are zero, so
 // their columns of Tb and P and their rows of D vanish. Addresses are a
 // uniform per-chunk base plus a 32-bit lane offset.
-template <bool kUpper, bool kF32>
-GDN_DEV void fetch_staged(StagedOperands& op, const StatePassCtx& cx, int c, int w, int l) {
+template <bool kF32>
+GDN_DEV void fetch_k(StagedOperands& op, const StatePassCtx& cx, int c, int w, int l) {
     const int len = cx.len(c);
     const int64_t qk0 = cx.t0(c) * cx.qk_stride + cx.hk * kHD + 8 * (l & 15);
 #pragma unroll
@@ -759,24 +770,32 @@ GDN_DEV void fetch_staged(StagedOperands& op, const StatePassCtx& cx, int c, int
             op.ka[i] = load8(static_cast<const uint16_t*>(cx.k) + qk0 + o);
         }
     }
-    // Q: output wave w reads only its own 16 rows; they load straight into
-    // its A fragments (no LDS; float32 input: the raw floats, split into hi +
-    // lo by the projection).
-    {
-        const int qtok = 16 * w + (l & 15), qtok_c = qtok < len ? qtok : len - 1;
-        const int64_t q0 = cx.t0(c) * cx.qk_stride + cx.hk * kHD + 8 * (l >> 4) +
-                           uint32_t(qtok_c) * uint32_t(cx.qk_stride);
+}
+
+// Q: output wave w reads only its own 16 rows; they load straight into its A
+// fragments (no LDS; float32 input: the raw floats, split into hi + lo by the
+// projection).
+template <bool kF32>
+GDN_DEV void fetch_q(StagedOperands& op, const StatePassCtx& cx, int c, int w, int l) {
+    const int len = cx.len(c);
+    const int qtok = 16 * w + (l & 15), qtok_c = qtok < len ? qtok : len - 1;
+    const int64_t q0 = cx.t0(c) * cx.qk_stride + cx.hk * kHD + 8 * (l >> 4) +
+                       uint32_t(qtok_c) * uint32_t(cx.qk_stride);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if constexpr (kF32) {
-                const float* src = static_cast<const float*>(cx.q) + q0 + 32 * i;
-                op.qa[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const f32x4*>(src));
-                op.qal[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const f32x4*>(src + 4));
-            } else {
-                op.qa[i] = load8(static_cast<const uint16_t*>(cx.q) + q0 + 32 * i);
-            }
+    for (int i = 0; i < 4; ++i) {
+        if constexpr (kF32) {
+            const float* src = static_cast<const float*>(cx.q) + q0 + 32 * i;
+            op.qa[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const f32x4*>(src));
+            op.qal[i] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const f32x4*>(src + 4));
+        } else {
+            op.qa[i] = load8(static_cast<const uint16_t*>(cx.q) + q0 + 32 * i);
         }
     }
+}
+
+template <bool kF32>
+GDN_DEV void fetch_v(StagedOperands& op, const StatePassCtx& cx, int c, int w, int l) {
+    const int len = cx.len(c);
     const int tv = 16 * w + (l >> 2);
     const int tv_c = tv < len ? tv : len - 1;
     const int64_t vo = cx.t0(c) * cx.Hv * kHD + cx.h * kHD + cx.dv0 + 4 * (l & 3) +
@@ -788,6 +807,10 @@ GDN_DEV void fetch_staged(StagedOperands& op, const StatePassCtx& cx, int c, int
     } else {
         op.v = *reinterpret_cast<const u32x2*>(static_cast<const uint16_t*>(cx.v) + vo);
     }
+}
+
+template <bool kUpper>
+GDN_DEV void fetch_tb_e(StagedOperands& op, const StatePassCtx& cx, int c, int w, int l) {
     const char* rec = cx.rec(c);
     op.e = *reinterpret_cast<const f32x4*>(rec + kRecEl + 128 * w + 16 * (l & 7));
     const uint16_t* tb_hi = reinterpret_cast<const uint16_t*>(rec + kRecTbHi);
@@ -797,6 +820,14 @@ GDN_DEV void fetch_staged(StagedOperands& op, const StatePassCtx& cx, int c, int
         op.tbh[s] = load8(tb_hi + (64 * (2 * w + s) + l) * 8);
         op.tbl[s] = load8(tb_lo + (64 * (2 * w + s) + l) * 8);
     }
+}
+
+template <bool kUpper, bool kF32>
+GDN_DEV void fetch_staged(StagedOperands& op, const StatePassCtx& cx, int c, int w, int l) {
+    fetch_k<kF32>(op, cx, c, w, l);
+    fetch_q<kF32>(op, cx, c, w, l);
+    fetch_v<kF32>(op, cx, c, w, l);
+    fetch_tb_e<kUpper>(op, cx, c, w, l);
 }
 
 template <bool kUpper>
@@ -1201,11 +1232,56 @@ GDN_DEV void output_loop_3ahead(const StatePassCtx& cx, int nch, StatePassLds<kF
     if (c + 1 < nch) step(c + 1, g1, g2, p1, p0);
 }
 
-template <class Y, bool kF32>
-__global__ __launch_bounds__(kStateThreads) void prefill_state_kernel(
+// Two workgroups a CU: each operand register is refilled as soon as it has
+// been staged (Q and P: used), so one set of them (70 registers, not the 210
+// of the ring above) keeps the loads about a step ahead, and the other
+// workgroup's work covers what of their latency is left.
+template <class Y, bool kUpper>
+GDN_DEV void output_loop_1ahead(const StatePassCtx& cx, int nch, StatePassLds<false>& sm,
+                                typename Y::storage* __restrict__ y, int w, int l) {
+    const int last = nch - 1;
+    const auto at = [&](int c) { return c < last ? c : last; };
+    StagedOperands g;  // K, V, Tb and e of chunk c + 1, Q of chunk c
+    OutputOperands p;  // P of chunk c
+    auto step = [&](int c, int buf) {
+        __syncthreads();
+        const f32x4 yacc = output_project(g, sm, w, l);
+        __syncthreads();
+        stage_k(g, sm, buf ^ 1, w, l);
+        stage_v(g, sm, w, l);
+        fetch_k<false>(g, cx, at(c + 2), w, l);
+        fetch_v<false>(g, cx, at(c + 2), w, l);
+        fetch_q<false>(g, cx, at(c + 1), w, l);
+        __builtin_amdgcn_sched_barrier(0);  // the prefetches stay where they are issued
+        __syncthreads();
+        stage_tb_e<kUpper>(g, sm, w, l);
+        fetch_tb_e<kUpper>(g, cx, at(c + 2), w, l);
+        output_store<Y, kUpper>(p, yacc, sm, cx, c, y, w, l);
+        fetch_output<kUpper>(p, cx, at(c + 1), w, l);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    fetch_staged<kUpper, false>(g, cx, 0, w, l);
+    fetch_output<kUpper>(p, cx, 0, w, l);
+    stage_k(g, sm, 0, w, l);
+    stage_v(g, sm, w, l);
+    stage_tb_e<kUpper>(g, sm, w, l);
+    fetch_k<false>(g, cx, at(1), w, l);
+    fetch_v<false>(g, cx, at(1), w, l);
+    fetch_tb_e<kUpper>(g, cx, at(1), w, l);
+    int c = 0;
+    for (; c + 1 < nch; c += 2) {
+        step(c, 0);
+        step(c + 1, 1);
+    }
+    if (c < nch) step(c, 0);
+}
+
+// kShared: two workgroups of the kernel share a CU (bf16 input).
+template <class Y, bool kF32, bool kShared>
+GDN_DEV void prefill_state_body(
     const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     const float* __restrict__ state_in, float* __restrict__ state_out,
-    typename Y::storage* __restrict__ y, RunLayout rl, const char* __restrict__ records, int Hk,
+    typename Y::storage* __restrict__ y, const RunLayout& rl, const char* __restrict__ records, int Hk,
     int Hv) {
     __shared__ __attribute__((aligned(16))) StatePassLds<kF32> sm;
 
@@ -1266,7 +1342,10 @@ __global__ __launch_bounds__(kStateThreads) void prefill_state_kernel(
             *reinterpret_cast<float4*>(state_out + sbase + dk) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
         }
     } else if (nch > 0) {
-        if constexpr (kF32) {
+        if constexpr (kShared) {
+            if (w >= 2) output_loop_1ahead<Y, true>(cx, nch, sm, y, w, l);
+            else output_loop_1ahead<Y, false>(cx, nch, sm, y, w, l);
+        } else if constexpr (kF32) {
             if (w >= 2) output_loop_2ahead<Y, true>(cx, nch, sm, y, w, l);
             else output_loop_2ahead<Y, false>(cx, nch, sm, y, w, l);
         } else {
@@ -1274,6 +1353,37 @@ __global__ __launch_bounds__(kStateThreads) void prefill_state_kernel(
             else output_loop_3ahead<Y, false>(cx, nch, sm, y, w, l);
         }
     }
+}
+
+#define GDN_STATE_ARGS                                                                                \
+    const void *__restrict__ q, const void *__restrict__ k, const void *__restrict__ v,               \
+        const float *__restrict__ state_in, float *__restrict__ state_out,                            \
+        typename Y::storage *__restrict__ y, RunLayout rl, const char *__restrict__ records, int Hk, int Hv
+
+template <class Y, bool kF32>
+__global__ __launch_bounds__(kStateThreads) void prefill_state_kernel(GDN_STATE_ARGS) {
+    prefill_state_body<Y, kF32, false>(q, k, v, state_in, state_out, y, rl, records, Hk, Hv);
+}
+
+template <class Y>
+__global__ __launch_bounds__(kStateThreads) __attribute__((amdgpu_waves_per_eu(4))) void
+prefill_state_shared_kernel(GDN_STATE_ARGS) {
+    prefill_state_body<Y, false, true>(q, k, v, state_in, state_out, y, rl, records, Hk, Hv);
+}
+#undef GDN_STATE_ARGS
+
+// The state pass over every (run, value head, slice).
+template <class Y, bool kF32>
+int launch_state(const void* q, const void* k, const void* v, const float* state_in, float* state_out, void* y,
+                 const RunLayout& rl, const char* records, int Hk, int Hv, hipStream_t s, const char* what) {
+    const int64_t wgs = int64_t(rl.N) * Hv * kSlices;
+    auto kernel = prefill_state_kernel<Y, kF32>;
+    if constexpr (!kF32) {
+        if (wgs > kStateSharedAbove) kernel = prefill_state_shared_kernel<Y>;
+    }
+    hipLaunchKernelGGL(kernel, dim3(unsigned(wgs)), dim3(kStateThreads), 0, s, q, k, v, state_in, state_out,
+                       static_cast<typename Y::storage*>(y), rl, records, Hk, Hv);
+    return check_launch(what);
 }
 
 }  // namespace gdn
@@ -1350,21 +1460,17 @@ extern "C" int gdn_prefill_chunked(const void* q, const void* k, const void* v, 
                        cgrid, dim3(256), 0, s, q, k, ga, gb,
                        gb_dtype, gate_stride, A_log, dt_bias, gate_mode, rl, records, Hk, Hv);
     if (int rc = check_launch("gdn_prefill_chunked/chunk")) return rc;
-    const dim3 sgrid(unsigned(int64_t(N) * Hv * kSlices));
-#define GDN_STATE_LAUNCH(YT, F32)                                                                 \
-    hipLaunchKernelGGL((prefill_state_kernel<YT, F32>), sgrid, dim3(kStateThreads), 0, s, q, k, v, \
-                       state_in, state_out, static_cast<YT::storage*>(y), rl, records, Hk, Hv)
+    const auto launch = [&](auto kernel) {
+        return kernel(q, k, v, state_in, state_out, y, rl, records, Hk, Hv, s, "gdn_prefill_chunked/state");
+    };
     if (f32) {
-        if (y_dtype == GDN_F32) GDN_STATE_LAUNCH(ActF32, true);
-        else if (y_dtype == GDN_BF16) GDN_STATE_LAUNCH(ActBF16, true);
-        else GDN_STATE_LAUNCH(ActF16, true);
-    } else {
-        if (y_dtype == GDN_F32) GDN_STATE_LAUNCH(ActF32, false);
-        else if (y_dtype == GDN_BF16) GDN_STATE_LAUNCH(ActBF16, false);
-        else GDN_STATE_LAUNCH(ActF16, false);
+        if (y_dtype == GDN_F32) return launch(launch_state<ActF32, true>);
+        if (y_dtype == GDN_BF16) return launch(launch_state<ActBF16, true>);
+        return launch(launch_state<ActF16, true>);
     }
-#undef GDN_STATE_LAUNCH
-    return check_launch("gdn_prefill_chunked/state");
+    if (y_dtype == GDN_F32) return launch(launch_state<ActF32, false>);
+    if (y_dtype == GDN_BF16) return launch(launch_state<ActBF16, false>);
+    return launch(launch_state<ActF16, false>);
 }
 
 namespace {
@@ -1468,13 +1574,10 @@ extern "C" int gdn_prefill_fused(const void* qkv, int64_t qkv_stride, const void
                                cv, int(C));
         if (int rc = check_launch("gdn_prefill_fused/conv_state")) return rc;
     }
-    const dim3 sgrid(unsigned(int64_t(N) * Hv * kSlices));
-#define GDN_STATE_LAUNCH(YT)                                                                            \
-    hipLaunchKernelGGL((prefill_state_kernel<YT, false>), sgrid, dim3(kStateThreads), 0, s, cv.qo, cv.ko, \
-                       cv.vo, state_in, state_out, static_cast<YT::storage*>(y), rl, records, Hk, Hv)
-    if (y_dtype == GDN_F32) GDN_STATE_LAUNCH(ActF32);
-    else if (y_dtype == GDN_BF16) GDN_STATE_LAUNCH(ActBF16);
-    else GDN_STATE_LAUNCH(ActF16);
-#undef GDN_STATE_LAUNCH
-    return check_launch("gdn_prefill_fused/state");
+    const auto launch = [&](auto kernel) {
+        return kernel(cv.qo, cv.ko, cv.vo, state_in, state_out, y, rl, records, Hk, Hv, s, "gdn_prefill_fused/state");
+    };
+    if (y_dtype == GDN_F32) return launch(launch_state<ActF32, false>);
+    if (y_dtype == GDN_BF16) return launch(launch_state<ActBF16, false>);
+    return launch(launch_state<ActF16, false>);
 }

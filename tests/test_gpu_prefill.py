@@ -400,3 +400,29 @@ def test_prefill_float32_full_size_against_c_oracle(gpu):
                                     use_kernel=False)
     assert max_rel(s.cpu().numpy(), s2.cpu().numpy()) < 1e-4
     assert max_rel(y.cpu().numpy(), y2.cpu().numpy()) < 1e-4
+
+
+@pytest.mark.parametrize("lens", [[64, 1, 130, 63, 200, 65, 128, 320, 0], [192] * 9])
+def test_prefill_runs_sharing_a_cu_equal_each_run_alone(gpu, lens):
+    """Above 256 state-pass workgroups (here 9 runs of 4 heads, 8 slices
+    each) two of them share a CU, on a loop with shorter prefetches: the same
+    bits as each run by itself, on the other loop."""
+    rng = np.random.default_rng(31)
+    T, Hk, Hv = sum(lens), 2, 4
+    q, k, v = (torch.tensor(rng.standard_normal((T, h, 128)) / s, dtype=torch.bfloat16, device=gpu)
+               for h, s in ((Hk, 11.3), (Hk, 11.3), (Hv, 1.0)))
+    a, b = (torch.tensor(rng.standard_normal((T, Hv)), dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    A_log, dt = (torch.tensor(rng.uniform(-1, 1, Hv), dtype=torch.float32, device=gpu) for _ in range(2))
+    state = torch.tensor(rng.standard_normal((len(lens), Hv, 128, 128)) * 0.05, dtype=torch.float32, device=gpu)
+    cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
+    # a run under PREFILL_MIN_TOKENS takes this path in a batch only
+    for y_dtype in (torch.float32, torch.bfloat16, torch.float16):
+        y, s = gated_delta.gated_delta_update(q, k, v, a, b, A_log, dt, state, cu_seqlens=cu, y_dtype=y_dtype)
+        for r, n in enumerate(lens):
+            o = slice(cu[r], cu[r + 1])
+            if n >= gated_delta.PREFILL_MIN_TOKENS:
+                y1, s1 = gated_delta.gated_delta_update(q[o], k[o], v[o], a[o], b[o], A_log, dt, state[r:r + 1],
+                                               cu_seqlens=[0, n], y_dtype=y_dtype)
+                assert torch.equal(y[o], y1) and torch.equal(s[r], s1[0]), (r, n)
+            elif n == 0:
+                assert torch.equal(s[r], state[r])
