@@ -53,7 +53,8 @@ typedef enum {
  * 10 the gated norm's z layout, 11 gdn_quantized_matmul_noalloc, 12 the
  * prefill's float32 q/k/v, 13 gdn_prefill_fused, 14 gdn_dequantize's mode, 15
  * gdn_quantized_matmul_scheme and its workspace size, 16 conv_arrivals as
- * counters whose bit 16 is a parity of the half bit). */
+ * counters whose bit 16 is a parity of the half bit, 17
+ * gdn_quantized_matmul_f32 and its workspace size). */
 int gdn_abi_version(void);
 
 /* Message describing the calling thread's last non-zero return. */
@@ -348,6 +349,27 @@ int gdn_quantized_matmul_noalloc(const void *x, int x_dtype, const void *w, cons
  */
 int64_t gdn_quantized_matmul_workspace_size(int x_dtype, int sb_dtype, int M, int N, int K,
                                             int bits, int group_size);
+
+/*
+ * gdn_quantized_matmul_f32 - y = x W^T for float32 x of any row count, in
+ * float32 accuracy on the bf16 matrix cores.
+ *   x: (M, K) float32; w, scales, biases as gdn_quantized_matmul (bits 4 or
+ *   8; group_size 32, 64 or 128; K a multiple of 64 and of it)
+ *   y: (M, N) float32; residual: NULL or (M, N) float32 (may be y itself),
+ *   added to the product
+ * x enters as three bf16 pieces (all 24 significant bits), the codes exactly;
+ * scale and bias are applied per group to float32 partial sums (no weight is
+ * rounded). x, w and workspace 16-byte aligned; the workspace takes
+ * gdn_quantized_matmul_f32_workspace_size(...) bytes (0 for sizes the entry
+ * point does not take) and must not be shared by overlapping calls.
+ * Replaces mx.quantized_matmul(..., mode="affine") in quantized_linear
+ * (model/moe_block.py:44-55) for the float32 rows of a prompt.
+ */
+int gdn_quantized_matmul_f32(const float *x, const void *w, const void *scales, const void *biases,
+                             int sb_dtype, float *y, const float *residual, int M, int N, int K,
+                             int bits, int group_size, void *workspace, int64_t workspace_bytes,
+                             void *stream);
+int64_t gdn_quantized_matmul_f32_workspace_size(int M, int N, int K, int bits, int group_size);
 
 /* Quantization modes (the reference's QuantScheme.mode, config.py:17-33). */
 #define GDN_QUANT_AFFINE 0

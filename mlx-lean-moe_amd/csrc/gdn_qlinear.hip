@@ -20,6 +20,7 @@
 
 #include "gdn_common.h"
 #include "gdn_host.h"
+#include "gdn_qlinear.h"
 
 namespace gdn {
 namespace {
@@ -694,6 +695,8 @@ __global__ __launch_bounds__(256) void qlinear_split_sum_kernel(const float* __r
     }
 }
 
+}  // namespace
+
 // The split sum for S = 2, 4, 8 or 16 blocks (the split counts the split-K
 // kernels choose).
 int launch_split_sum(const float* partial, int splits, int64_t count, void* y, int y_dtype, const void* residual,
@@ -708,6 +711,8 @@ int launch_split_sum(const float* partial, int splits, int64_t count, void* y, i
     }
     return check_launch(who);
 }
+
+namespace {
 
 constexpr int kCUs = 256;  // compute units of an MI355X
 

@@ -1,0 +1,458 @@
+// Affine-quantized projections of float32 activations at prompt sizes
+// (gdn_quantized_matmul_f32): y = x W^T for float32 x (M, K) and MLX-packed
+// 4- or 8-bit codes, in float32 accuracy on the bf16 matrix cores.
+//
+// Both factors are taken exactly. A code less its centre, q - 2^(bits-1), is
+// a bf16 value; a float32 x is the sum of three bf16 values (its 24
+// significant bits cut into three 8-bit pieces). So with
+//   P[m][n] = sum over one quantization group's k of x[m][k] (q[n][k] - c)
+// (three MFMAs a fragment pair, float32 sums of exact products), X[m][g] the
+// group's sum of x and b' = b + c s,
+//   y[m][n] = sum over groups of s[n][g] P + b'[n][g] X[m][g]:
+// no weight is rounded and no product is, which leaves the float32 sums
+// (777 rows of 2048 normal values against 12352 columns of 4-bit codes in
+// groups of 64: 1.2e-7 from float64, where the float32 library product of
+// rounded weights is 8.1e-7 off and takes 345 us to this one's 134).
+//
+// Two launches (three where K is split): the preparation cuts x, sums its
+// groups and lays s and b' out group-major; the product kernel does the rest.
+#include "gdn_common.h"
+#include "gdn_host.h"
+#include "gdn_qlinear.h"
+
+namespace gdn {
+namespace {
+
+constexpr int kBK = 64;             // k per step
+constexpr int kParts = 3;           // bf16 pieces of a float32
+constexpr int kPK = kParts * kBK;   // a row's pieces of one step
+constexpr int kXS = kPK + 8;        // row stride of the LDS tile, bf16: 16 rows cover the banks
+constexpr int kTN = 4;              // 16-column tiles of a wave
+constexpr int kBN = 4 * 16 * kTN;   // columns of a workgroup (4 waves)
+constexpr int kMaxTM = 5;           // 16-row tiles of a workgroup, at most (6 spill)
+constexpr int kCUs = 256;
+
+GDN_DEV f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+}
+
+// ---------------------------------------------------------------------------
+// preparation
+// ---------------------------------------------------------------------------
+
+// Rows whose pieces would not be exact: a non-finite x, one so large that the
+// group sums could overflow where the products with the (small) weights do
+// not, or a row of magnitudes whose last piece leaves bf16's range. They are
+// multiplied apart (slow_row).
+constexpr float kRowMax = 0x1p100f, kRowMin = 0x1p-90f;
+
+// Blocks 0 .. M - 1: row m of x as bf16 pieces, pieces[m][step][part][64]
+// (part 0 the upper 8 significant bits; truncation, so no piece can round up
+// to infinity), its group sums (in double, rounded once) and its flag. The
+// blocks after them: s and b' = b + centre s in float32, group-major.
+__global__ __launch_bounds__(256) void prepare_f32_kernel(
+    const float* __restrict__ x, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
+    uint16_t* __restrict__ pieces, float* __restrict__ xsum, int* __restrict__ flags, float* __restrict__ s_t,
+    float* __restrict__ b_t, int M, int N, int K, int group_size, float centre) {
+    const int G = K / group_size;
+    if (int(blockIdx.x) >= M) {
+        const int64_t i = int64_t(int(blockIdx.x) - M) * 256 + threadIdx.x;  // (g, n), n fastest
+        if (i >= int64_t(N) * G) return;
+        const int64_t g = i / N, n = i % N;
+        const float s = load_any(scales, n * G + g, sb_dtype), b = load_any(biases, n * G + g, sb_dtype);
+        s_t[i] = s;
+        b_t[i] = __builtin_fmaf(centre, s, b);
+        return;
+    }
+    const int64_t m = blockIdx.x;
+    const int chunks = K / 8, lanes = group_size / 8;  // 8-element chunks; chunks of a group
+    bool odd = false;
+    float top = 0.f;
+    for (int c0 = 0; c0 < chunks; c0 += 256) {
+        const int c = c0 + int(threadIdx.x);
+        double sum = 0.0;
+        if (c < chunks) {
+            const float4 lo4 = *reinterpret_cast<const float4*>(x + m * K + 8 * c);
+            const float4 hi4 = *reinterpret_cast<const float4*>(x + m * K + 8 * c + 4);
+            const float v[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+            uint32_t part[kParts][4];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                odd |= !(fabsf(v[j]) < kRowMax);
+                top = fmaxf(top, fabsf(v[j]));
+                sum += double(v[j]);
+                const float h = __uint_as_float(__float_as_uint(v[j]) & 0xFFFF0000u);
+                const float r = v[j] - h;  // exact
+                const float mid = __uint_as_float(__float_as_uint(r) & 0xFFFF0000u);
+                const uint32_t bits[kParts] = {__float_as_uint(h), __float_as_uint(mid), __float_as_uint(r - mid)};
+#pragma unroll
+                for (int p = 0; p < kParts; ++p)
+                    part[p][j / 2] = j & 1 ? (part[p][j / 2] | (bits[p] & 0xFFFF0000u)) : bits[p] >> 16;
+            }
+            uint16_t* dst = pieces + (m * K + (c / 8) * kBK) * kParts + 8 * (c % 8);
+#pragma unroll
+            for (int p = 0; p < kParts; ++p)
+                *reinterpret_cast<uint4*>(dst + kBK * p) = make_uint4(part[p][0], part[p][1], part[p][2], part[p][3]);
+        }
+        // a group's 4, 8 or 16 chunks lie in consecutive lanes (K is a
+        // multiple of the group, so a group never ends inside `chunks`)
+        for (int d = 1; d < lanes; d *= 2) sum += __shfl_xor(sum, d);
+        if (c < chunks && c % lanes == 0) xsum[m * G + c / lanes] = float(sum);
+    }
+    odd |= __syncthreads_or(odd);
+    const bool small = top < kRowMin, zero = top == 0.f;
+    const bool all_small = !__syncthreads_or(!small), all_zero = !__syncthreads_or(!zero);
+    if (threadIdx.x == 0) flags[m] = odd || (all_small && !all_zero);
+}
+
+// ---------------------------------------------------------------------------
+// product
+// ---------------------------------------------------------------------------
+
+// 8 codes less their centre as bf16 (exact: the float's upper half).
+template <int kBits>
+GDN_DEV bf16x8 centred_fragment(const uint32_t* words) {
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int kPer = 32 / kBits;
+    u32x4 d;
+    float f[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        // flipping a field's top bit makes it the two's complement of q - centre
+        const int32_t v = int32_t(words[j / kPer] ^ (kBits == 4 ? 0x88888888u : 0x80808080u));
+        f[j] = float((v << (32 - kBits * (j % kPer + 1))) >> (32 - kBits));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        d[i] = __builtin_amdgcn_perm(__float_as_uint(f[2 * i + 1]), __float_as_uint(f[2 * i]), 0x07060302u);
+    return __builtin_bit_cast(bf16x8, d);
+}
+
+// One flagged row's columns of the workgroup, a thread a column, from the
+// float32 weights: what the pieces cannot carry (infinities, NaN, the ends
+// of the range).
+template <int kBits>
+GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__ w, const void* scales,
+                       const void* biases, int sb_dtype, int64_t n, int K, int group_size) {
+    constexpr int kPer = 32 / kBits;
+    const int64_t G = K / group_size;
+    float v = 0.f;
+    for (int k = 0; k < K; ++k) {
+        const uint32_t q = (w[n * (K / kPer) + k / kPer] >> (kBits * (k % kPer))) & ((1u << kBits) - 1u);
+        const int64_t gi = n * G + k / group_size;
+        v = __builtin_fmaf(x[k], __builtin_fmaf(load_any(scales, gi, sb_dtype), float(q), load_any(biases, gi, sb_dtype)), v);
+    }
+    return v;
+}
+
+// A workgroup holds 16 kTM rows by 256 columns, each of its 4 waves all the
+// rows by 64 columns, so a piece of x read from LDS serves four MFMAs and the
+// codes go from memory to the wave's own B fragments, converted once per
+// workgroup. A step is 64 k: x's pieces through LDS (one tile, the next step's
+// in registers), codes and scales a step ahead in registers. Two workgroups
+// share a CU (256 registers a thread). Per step and wave 24 kTM MFMAs stand
+// beside ~160 instructions of code conversion and 16 kTM of scaling.
+//
+// kG32: groups of 32 (an MFMA's k), each scaled by itself; else one group (64
+// or half of 128) a step. Lane quarter q = l / 16 holds k 8 q .. of each
+// 32-block, or 16 q .. of the step (one 8-byte load of 4-bit codes).
+//
+// Split K: blockIdx.y = j takes steps [j steps / S, (j + 1) steps / S) and
+// stores its float32 block at out + j M N, to be added in order afterwards.
+template <int kBits, int kTM, bool kG32>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void qlinear_f32_kernel(
+    const uint16_t* __restrict__ pieces, const float* __restrict__ xsum, const int* __restrict__ flags,
+    const float* __restrict__ s_t, const float* __restrict__ b_t, const float* __restrict__ x,
+    const uint32_t* __restrict__ w, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
+    float* out, const float* residual, int M, int N, int K, int group_size, int mt, int tiles) {
+    constexpr int kBM = 16 * kTM;
+    constexpr int kPiecesPerRow = kPK / 8;
+    constexpr int kXLoads = (kBM * kPiecesPerRow + 255) / 256;
+    constexpr int kWords = 2 * kBits / 4;  // packed words of a lane's 16 codes of a step
+    __shared__ __attribute__((aligned(16))) uint16_t xs[kBM * kXS];
+
+    // Tiles in row-major order within a column block, an eighth of them to
+    // each XCD (workgroups go round-robin over the XCDs): a column block's
+    // codes are read into one XCD's L2.
+    const int per_xcd = (tiles + 7) / 8;
+    const int t = int(blockIdx.x % 8) * per_xcd + int(blockIdx.x / 8);
+    if (t >= tiles || int(blockIdx.x / 8) >= per_xcd) return;
+    const int m0 = (t % mt) * kBM, n0 = (t / mt) * kBN;
+    const int tid = threadIdx.x, l = tid & 63, lr = l & 15, lq = l >> 4;
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int steps = K / kBK / int(gridDim.y), step0 = steps * int(blockIdx.y);
+    const int g0 = step0 * kBK / group_size, g1 = (step0 + steps) * kBK / group_size;
+
+    int col[kTN];
+#pragma unroll
+    for (int b = 0; b < kTN; ++b) {
+        const int n = n0 + 16 * kTN * wv + 16 * b + lr;
+        col[b] = n < N ? n : N - 1;  // clamped columns are not stored
+    }
+
+    // x: rows clamped to M - 1 (not stored); pieces past the tile repeat its last
+    const uint16_t* xtile = pieces + int64_t(m0) * K * kParts;
+    uint32_t xo[kXLoads];
+    int xl[kXLoads];
+#pragma unroll
+    for (int i = 0; i < kXLoads; ++i) {
+        int idx = tid + 256 * i;
+        idx = idx < kBM * kPiecesPerRow ? idx : kBM * kPiecesPerRow - 1;
+        const int row = idx / kPiecesPerRow, seg = idx % kPiecesPerRow;
+        const int r = m0 + row < M ? row : M - 1 - m0;
+        xo[i] = uint32_t(r) * uint32_t(K * kParts) + 8 * seg;
+        xl[i] = row * kXS + 8 * seg;
+    }
+    u16x8 xr[kXLoads];
+    auto fetch_x = [&](int s) {
+        const uint16_t* src = xtile + int64_t(s) * kPK;
+#pragma unroll
+        for (int i = 0; i < kXLoads; ++i) xr[i] = *reinterpret_cast<const u16x8*>(src + xo[i]);
+    };
+    auto stage_x = [&] {
+#pragma unroll
+        for (int i = 0; i < kXLoads; ++i) *reinterpret_cast<u16x8*>(xs + xl[i]) = xr[i];
+    };
+
+    const int64_t wpr = int64_t(K) * kBits / 32;
+    uint32_t wd[kTN][kWords];  // words of MFMA block kb at [b][kb kWords / 2 ..]
+    float sc[kTN][kG32 ? 2 : 1];
+    auto fetch_w = [&](int s) {
+        const int wk = s * kBK * kBits / 32;
+#pragma unroll
+        for (int b = 0; b < kTN; ++b) {
+            const uint32_t* src = w + col[b] * wpr + wk;
+            if constexpr (kG32) {
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+#pragma unroll
+                    for (int i = 0; i < kWords / 2; ++i)
+                        wd[b][kb * kWords / 2 + i] = src[kb * kBits + lq * kWords / 2 + i];
+            } else {
+#pragma unroll
+                for (int i = 0; i < kWords; ++i) wd[b][i] = src[lq * kWords + i];
+            }
+            const int g = s * kBK / group_size;
+#pragma unroll
+            for (int i = 0; i < (kG32 ? 2 : 1); ++i) sc[b][i] = s_t[int64_t(g + i) * N + col[b]];
+        }
+    };
+
+    fetch_x(step0);
+    fetch_w(step0);
+
+    // the bias terms first: X times b' over the range's groups, in float32
+    // MFMAs of four groups (lanes past the last group carry zeros)
+    f32x4 acc[kTM][kTN];
+#pragma unroll
+    for (int a = 0; a < kTM; ++a)
+#pragma unroll
+        for (int b = 0; b < kTN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int G = K / group_size;
+    for (int g = g0; g < g1; g += 4) {
+        const bool in = g + lq < g1;
+        const int gl = in ? g + lq : g1 - 1;
+        float xa[kTM], bb[kTN];
+#pragma unroll
+        for (int a = 0; a < kTM; ++a) {
+            const int m = m0 + 16 * a + lr;
+            xa[a] = xsum[int64_t(m < M ? m : M - 1) * G + gl];
+        }
+#pragma unroll
+        for (int b = 0; b < kTN; ++b) bb[b] = b_t[int64_t(gl) * N + col[b]];
+#pragma unroll
+        for (int a = 0; a < kTM; ++a)
+#pragma unroll
+            for (int b = 0; b < kTN; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xa[a] : 0.f, in ? bb[b] : 0.f, acc[a][b], 0, 0, 0);
+    }
+
+    stage_x();
+    for (int s = step0; s < step0 + steps; ++s) {
+        bf16x8 bf[kTN][2];
+        float scale[kTN][kG32 ? 2 : 1];
+#pragma unroll
+        for (int b = 0; b < kTN; ++b) {
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) bf[b][kb] = centred_fragment<kBits>(&wd[b][kb * kWords / 2]);
+#pragma unroll
+            for (int i = 0; i < (kG32 ? 2 : 1); ++i) scale[b][i] = sc[b][i];
+        }
+        const int next = s + 1 < step0 + steps ? s + 1 : s;  // the last step repeats itself
+        fetch_x(next);
+        fetch_w(next);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+#pragma unroll
+        for (int a = 0; a < kTM; ++a) {
+            const uint16_t* xrow = xs + (16 * a + lr) * kXS;
+            bf16x8 af[kParts][2];
+#pragma unroll
+            for (int p = 0; p < kParts; ++p)
+#pragma unroll
+                for (int kb = 0; kb < 2; ++kb)
+                    af[p][kb] = *reinterpret_cast<const bf16x8*>(xrow + kBK * p + (kG32 ? 32 * kb + 8 * lq : 16 * lq + 8 * kb));
+            f32x4 part[kTN];
+            auto scaled = [&](int i) {
+#pragma unroll
+                for (int b = 0; b < kTN; ++b)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[a][b][e] = __builtin_fmaf(scale[b][i], part[b][e], acc[a][b][e]);
+            };
+#pragma unroll
+            for (int kb = 0; kb < 2; ++kb) {
+                if (kG32 || kb == 0) {
+#pragma unroll
+                    for (int b = 0; b < kTN; ++b) part[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+#pragma unroll
+                for (int p = kParts - 1; p >= 0; --p)  // the small pieces first
+#pragma unroll
+                    for (int b = 0; b < kTN; ++b) part[b] = mfma_bf16(af[p][kb], bf[b][kb], part[b]);
+                if constexpr (kG32) scaled(kb);
+            }
+            if constexpr (!kG32) scaled(0);
+        }
+        __syncthreads();
+        stage_x();
+    }
+
+    int any = 0;
+    if (tid < kBM) any = flags[m0 + tid < M ? m0 + tid : M - 1];
+    any = __syncthreads_or(any);
+    float* dst = out + int64_t(blockIdx.y) * M * N;
+#pragma unroll
+    for (int a = 0; a < kTM; ++a)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + 16 * a + 4 * lq + i;
+            if (m >= M || (any && flags[m])) continue;
+#pragma unroll
+            for (int b = 0; b < kTN; ++b) {
+                const int n = n0 + 16 * kTN * wv + 16 * b + lr;
+                if (n >= N) continue;
+                const int64_t e = int64_t(m) * N + n;
+                dst[e] = acc[a][b][i] + (residual ? residual[e] : 0.f);
+            }
+        }
+    if (any && n0 + tid < N) {
+        for (int r = 0; r < kBM && m0 + r < M; ++r) {
+            if (!flags[m0 + r]) continue;
+            const int64_t m = m0 + r, n = n0 + tid, e = m * N + n;
+            const float v = blockIdx.y == 0 ? slow_row<kBits>(x + m * K, w, scales, biases, sb_dtype, n, K, group_size) : 0.f;
+            dst[e] = v + (residual ? residual[e] : 0.f);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// launch
+// ---------------------------------------------------------------------------
+
+struct F32Plan {
+    int tm, splits;
+    int64_t pieces, xsum, flags, s_t, b_t, partial, bytes;  // workspace offsets
+};
+
+// Rows of a workgroup and splits of K: the least time by the matrix cores'
+// share of the fullest CU, ceil(workgroups / 256) steps (fixed + per row tile)
+// (0.1 and 0.2 us as measured), and a split's partial blocks written and read.
+F32Plan plan_f32(int M, int N, int K, int group_size) {
+    F32Plan p{};
+    double best = 1e30;
+    const int64_t nt = (N + kBN - 1) / kBN;
+    for (int tm = 2; tm <= kMaxTM; ++tm)
+        for (int s = 1; s <= 16; s *= 2) {
+            if (K % (kBK * s) || K / s % group_size) break;
+            const int64_t wgs = (int64_t(M) + 16 * tm - 1) / (16 * tm) * nt * s;
+            const double us = double((wgs + kCUs - 1) / kCUs) * (K / kBK / s) * (0.1 + 0.2 * tm) +
+                              (s > 1 ? 3.0 + double(s) * M * N * 8 / 4e6 : 0.0);
+            if (us < best) {
+                best = us;
+                p.tm = tm;
+                p.splits = s;
+            }
+        }
+    const auto up = [](int64_t b) { return (b + 255) & ~int64_t(255); };
+    const int64_t G = K / group_size;
+    p.xsum = up(int64_t(M) * K * kParts * 2);
+    p.flags = p.xsum + up(M * G * 4);
+    p.s_t = p.flags + up(int64_t(M) * 4);
+    p.b_t = p.s_t + up(N * G * 4);
+    p.partial = p.b_t + up(N * G * 4);
+    p.bytes = p.partial + (p.splits > 1 ? int64_t(p.splits) * M * N * 4 : 0);
+    return p;
+}
+
+template <int kBits, bool kG32>
+auto kernel_of(int tm) {
+    switch (tm) {
+        case 2: return qlinear_f32_kernel<kBits, 2, kG32>;
+        case 3: return qlinear_f32_kernel<kBits, 3, kG32>;
+        case 4: return qlinear_f32_kernel<kBits, 4, kG32>;
+        default: return qlinear_f32_kernel<kBits, 5, kG32>;
+    }
+}
+
+bool f32_sizes_ok(int64_t M, int64_t N, int64_t K, int group_size) {
+    // 32-bit lane offsets and grid sizes
+    return M <= (1 << 24) && N <= (1 << 24) && K <= (1 << 20) && (group_size == 32 || group_size == 64 || group_size == 128) &&
+           K % kBK == 0 && K % group_size == 0;
+}
+
+}  // namespace
+}  // namespace gdn
+
+using namespace gdn;
+
+extern "C" int64_t gdn_quantized_matmul_f32_workspace_size(int M, int N, int K, int bits, int group_size) {
+    if (M < 1 || N < 1 || K < 1 || (bits != 4 && bits != 8) || !f32_sizes_ok(M, N, K, group_size)) return 0;
+    return plan_f32(M, N, K, group_size).bytes;
+}
+
+extern "C" int gdn_quantized_matmul_f32(const float* x, const void* w, const void* scales, const void* biases,
+                                        int sb_dtype, float* y, const float* residual, int M, int N, int K, int bits,
+                                        int group_size, void* workspace, int64_t workspace_bytes, void* stream) {
+    const char* fn = "gdn_quantized_matmul_f32";
+    GDN_REQUIRE(M >= 0 && N > 0 && K > 0, "%s: bad sizes M=%d N=%d K=%d", fn, M, N, K);
+    GDN_REQUIRE(w && scales && biases, "%s: null weight, scales or biases", fn);
+    GDN_REQUIRE(valid_dtype(sb_dtype), "%s: bad scales/biases dtype", fn);
+    if (bits != 4 && bits != 8) return fail(GDN_EUNSUPPORTED, "%s: %d-bit weights (4 and 8 are implemented)", fn, bits);
+    GDN_REQUIRE(f32_sizes_ok(M, N, K, group_size),
+                "%s: group_size must be 32, 64 or 128 and K=%d a multiple of 64 and of it", fn, K);
+    if (M == 0) return 0;
+    GDN_REQUIRE(x && y, "%s: null x or y", fn);
+    GDN_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |
+                 reinterpret_cast<uintptr_t>(workspace)) % 16 == 0,
+                "%s: x, weight and workspace must be 16-byte aligned", fn);
+    const int64_t xb = int64_t(M) * K * 4, yb = int64_t(M) * N * 4;
+    GDN_REQUIRE(!overlaps(x, xb, y, yb), "%s: y overlaps x", fn);
+    GDN_REQUIRE(!residual || residual == y || !overlaps(residual, yb, y, yb), "%s: residual partially overlaps y", fn);
+    const F32Plan p = plan_f32(M, N, K, group_size);
+    GDN_REQUIRE(workspace && workspace_bytes >= p.bytes, "%s: workspace of %lld bytes, need %lld", fn,
+                (long long)workspace_bytes, (long long)p.bytes);
+
+    hipStream_t s = as_stream(stream);
+    char* ws = static_cast<char*>(workspace);
+    auto* pieces = reinterpret_cast<uint16_t*>(ws);
+    auto* xsum = reinterpret_cast<float*>(ws + p.xsum);
+    auto* flags = reinterpret_cast<int*>(ws + p.flags);
+    auto* s_t = reinterpret_cast<float*>(ws + p.s_t);
+    auto* b_t = reinterpret_cast<float*>(ws + p.b_t);
+    auto* partial = reinterpret_cast<float*>(ws + p.partial);
+    const int64_t sb_blocks = (int64_t(N) * (K / group_size) + 255) / 256;
+    hipLaunchKernelGGL(prepare_f32_kernel, dim3(unsigned(M + sb_blocks)), dim3(256), 0, s, x, scales, biases, sb_dtype,
+                       pieces, xsum, flags, s_t, b_t, M, N, K, group_size, bits == 4 ? 8.f : 128.f);
+    if (int rc = check_launch("gdn_quantized_matmul_f32/prepare")) return rc;
+
+    const int mt = (M + 16 * p.tm - 1) / (16 * p.tm), tiles = mt * ((N + kBN - 1) / kBN);
+    const auto kernel = bits == 4 ? (group_size == 32 ? kernel_of<4, true>(p.tm) : kernel_of<4, false>(p.tm))
+                                  : (group_size == 32 ? kernel_of<8, true>(p.tm) : kernel_of<8, false>(p.tm));
+    hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8), unsigned(p.splits)), dim3(256), 0, s, pieces, xsum,
+                       flags, s_t, b_t, x, static_cast<const uint32_t*>(w), scales, biases, sb_dtype,
+                       p.splits > 1 ? partial : y, p.splits > 1 ? nullptr : residual, M, N, K, group_size, mt, tiles);
+    if (int rc = check_launch(fn)) return rc;
+    if (p.splits > 1)
+        return launch_split_sum(partial, p.splits, int64_t(M) * N, y, GDN_F32, residual, s, "gdn_quantized_matmul_f32/sum");
+    return 0;
+}

@@ -12,7 +12,8 @@ mxfp4 / mxfp8 / nvfp4: ``w`` = the e2m1 / e4m3 code's value times a uint8
 scale (e8m0, e4m3 for nvfp4), no biases. Affine 4- and 8-bit projections of
 bf16 activations run on ``gdn_quantized_matmul``; the other schemes and
 activation dtypes dequantize on the GPU (``gdn_dequantize``) and multiply on
-the vendor BLAS. Dense projections are ``x @ W.T``.
+the vendor BLAS, except that float32 rows times affine 4- and 8-bit codes run
+on ``gdn_quantized_matmul_f32``. Dense projections are ``x @ W.T``.
 """
 
 from __future__ import annotations
@@ -236,6 +237,8 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
         return with_residual(x @ wd.to(x.dtype).T)
     x_f32 = (x.dtype == torch.float32 and rows <= 32
              and decode_kernel_takes(rows, K, quant.bits, quant.group_size, scales.dtype))
+    if x.dtype == torch.float32 and not x_f32 and f32_workspace_bytes(rows, N, K, quant.bits, quant.group_size):
+        return _f32_matmul(x, w, scales, biases, quant, N, K, residual)
     if x.dtype != torch.bfloat16 and not x_f32:
         return with_residual(x @ dequantize(tensors, quant, x.dtype).T)
     x2 = _c(x.reshape(-1, K))
@@ -300,6 +303,29 @@ def _scheme_matmul(x, w, scales, biases, quant: QuantScheme, N: int, K: int, res
     return y.reshape(*lead, N)
 
 
+def _f32_matmul(x, w, scales, biases, quant: QuantScheme, N: int, K: int, residual):
+    """``x @ W.T`` (+ residual) for float32 rows beyond the decode kernel's
+    and affine 4- or 8-bit codes (gdn_quantized_matmul_f32): exact weights
+    and all of x's bits on the bf16 matrix cores."""
+
+    lead = x.shape[:-1]
+    x2 = _c(x.reshape(-1, K))
+    if x2.data_ptr() % 16:
+        x2 = x2.clone()
+    M = x2.shape[0]
+    y = torch.empty((M, N), dtype=x.dtype, device=x.device)
+    r = _residual_rows(residual, x, lead, M, N)
+    w, scales, biases = _c(w), _c(scales), _c(biases)
+    if w.data_ptr() % 16:
+        w = w.clone()
+    ws_bytes = f32_workspace_bytes(M, N, K, quant.bits, quant.group_size)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    _lib.call("gdn_quantized_matmul_f32", _lib.ptr(x2), _lib.ptr(w), _lib.ptr(scales), _lib.ptr(biases),
+              _lib.dtype_code(scales.dtype), _lib.ptr(y), _lib.ptr(r), M, N, K, quant.bits, quant.group_size,
+              _lib.ptr(ws), ws_bytes, _lib.stream_ptr(x.device))
+    return y.reshape(*lead, N)
+
+
 def quantized_linear_split(x: torch.Tensor, weights: LinearWeights, sizes) -> list[torch.Tensor]:
     """``x @ W.T`` for a quantized ``W`` stacked from projections that share
     ``x`` (:func:`concat_quantized`), returned as the column blocks ``sizes``
@@ -347,6 +373,13 @@ def scheme_workspace_bytes(M: int, N: int, K: int) -> int:
     """Workspace gdn_quantized_matmul_scheme splits K with (0: none)."""
 
     return int(_lib.load().gdn_quantized_matmul_scheme_workspace_size(M, N, K))
+
+
+@functools.lru_cache(maxsize=256)
+def f32_workspace_bytes(M: int, N: int, K: int, bits: int, group_size: int) -> int:
+    """Workspace of gdn_quantized_matmul_f32 (0: sizes it does not take)."""
+
+    return int(_lib.load().gdn_quantized_matmul_f32_workspace_size(M, N, K, bits, group_size))
 
 
 @functools.lru_cache(maxsize=256)

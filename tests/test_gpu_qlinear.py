@@ -537,3 +537,70 @@ def test_scheme_matmul_special_scale_codes(gpu, mode, gs, M):
     ok = ~nan_cols
     err = np.abs(got[:, ok] - ref[:, ok])
     assert (err <= 2.0 ** -20 * np.abs(ref[:, ok]) + 1e-5 * np.abs(ref[:, ok]).max()).all(), err.max()
+
+
+def _f32_bound(x, words, s, b, bits, gs):
+    """Worst-case rounding of gdn_quantized_matmul_f32: its products are
+    exact, and every value passes at most 3 gs + 2 float32 sums inside a group
+    and 2 G + 20 across the groups (the scaled sum, the bias term, split
+    blocks), each off by 2^-24 of the magnitudes it adds."""
+    K = x.shape[1]
+    centre = 2.0 ** (bits - 1)
+    bp = np.repeat(b + centre * s, gs, axis=1).astype(np.float64)
+    w = Q.dequantize(words, s, b, bits, gs, out="f32").astype(np.float64)
+    mass = np.abs(x).astype(np.float64) @ (np.abs(w - bp) + np.abs(bp)).T
+    return (3 * gs + 2 * K // gs + 22) * 2.0 ** -24 * mass
+
+
+@pytest.mark.parametrize("M,N,K,bits,gs,sb", [
+    (33, 300, 512, 4, 64, "bf16"),      # the first count past the decode kernel; ragged columns
+    (777, 520, 2048, 4, 64, "bf16"),
+    (81, 257, 384, 8, 128, "f32"),      # half a group a step, one row past five tiles
+    (200, 2048, 4096, 4, 64, "bf16"),   # K split
+    (130, 96, 1024, 4, 32, "f16"),      # an MFMA's k a group
+    (64, 40, 64, 8, 32, "f32"),         # a single step
+    (3, 512, 192, 4, 64, "bf16"),       # few rows of a K the decode kernel does not take
+    (1, 17, 64, 4, 64, "f16"),
+])
+def test_float32_rows_in_three_bf16_pieces(gpu, M, N, K, bits, gs, sb):
+    rng = np.random.default_rng(M * 5 + N)
+    words, s, b = _weights(rng, N, K, bits, gs, sb)
+    W = _dev_weights(gpu, words, s, b, sb)
+    x = (rng.standard_normal((M, K)) * np.exp(rng.uniform(-6, 6, (M, K))) + 0.5).astype(np.float32)
+    ref = Q.quantized_matmul(x, words, s, b, bits, gs, w_round="f32")
+    assert _lib.load().gdn_quantized_matmul_f32_workspace_size(M, N, K, bits, gs) > 0
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs))
+    assert y.dtype == torch.float32
+    assert (np.abs(y.cpu().numpy() - ref) <= _f32_bound(x, words, s, b, bits, gs) + 1e-30).all()
+    r = torch.tensor(rng.standard_normal((M, N)), dtype=torch.float32, device=gpu)
+    got = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs), residual=r)
+    assert torch.equal(got, y + r)
+
+
+@pytest.mark.parametrize("N,K", [(300, 512), (256, 4096)])  # K unsplit and split
+def test_float32_rows_outside_the_pieces_range(gpu, N, K):
+    """Rows with infinities, NaN, values near the ends of float32's range:
+    the float32 weights' sums, element for element as float64 gives them
+    (finite where it is finite, the same infinities and NaN)."""
+    rng = np.random.default_rng(N)
+    words, s, b = _weights(rng, N, K, 4, 64, "bf16")
+    W = _dev_weights(gpu, words, s, b, "bf16")
+    x = rng.standard_normal((70, K)).astype(np.float32)
+    x[3, 5] = np.inf
+    x[10, 7], x[10, 9] = np.inf, -np.inf
+    x[20, 1] = np.nan
+    x[33] = 0
+    x[33, 4] = 3.3e38
+    x[40] *= np.float32(1e-37)
+    x[50] = 0
+    x[69] *= np.float32(2.0 ** 99)
+    w = Q.dequantize(words, s, b, 4, 64, out="f32").astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref = x.astype(np.float64) @ w.T
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
+    finite = np.isfinite(x).all(axis=1)
+    mass = np.abs(x[finite]).astype(np.float64) @ np.abs(w).T
+    assert (np.abs(y[finite] - ref[finite]) <= 2 * K * 2.0 ** -24 * mass + 1e-38 * K).all()
+    np.testing.assert_array_equal(np.isnan(y[~finite]), np.isnan(ref[~finite]))
+    inf = np.isinf(ref)
+    np.testing.assert_array_equal(y[inf], ref[inf].astype(np.float32))
