@@ -54,7 +54,8 @@ typedef enum {
  * prefill's float32 q/k/v, 13 gdn_prefill_fused, 14 gdn_dequantize's mode, 15
  * gdn_quantized_matmul_scheme and its workspace size, 16 conv_arrivals as
  * counters whose bit 16 is a parity of the half bit, 17
- * gdn_quantized_matmul_f32 and its workspace size). */
+ * gdn_quantized_matmul_f32, its workspace size and
+ * gdn_quantized_matmul_rows_workspace_size). */
 int gdn_abi_version(void);
 
 /* Message describing the calling thread's last non-zero return. */
@@ -303,7 +304,10 @@ int gdn_gated_rmsnorm(const void *x, int x_dtype, const void *z, int z_dtype, in
  *      it splits less or not at all. 17-64 rows of bf16 x against 4-bit
  *      codes in 64-k slices with few column tiles (out_proj's shape) run
  *      instead as 16-row blocks in one launch and take no workspace (its
- *      size is 0 there). Calls sharing a workspace must not overlap.
+ *      size is 0 there). Above 64 rows gdn_quantized_matmul_rows_workspace_size
+ *      gives the bytes of the full split instead (the size function below
+ *      is of the decode kernel's calls). Calls sharing a workspace must not
+ *      overlap.
  * Replaces mx.quantized_matmul(..., mode="affine") in quantized_linear
  * (model/moe_block.py:44-55), used for the layer's projections
  * (model/qwen3_5/linear_attention.py:96-101,125).
@@ -370,6 +374,14 @@ int gdn_quantized_matmul_f32(const float *x, const void *w, const void *scales, 
                              int bits, int group_size, void *workspace, int64_t workspace_bytes,
                              void *stream);
 int64_t gdn_quantized_matmul_f32_workspace_size(int M, int N, int K, int bits, int group_size);
+
+/*
+ * gdn_quantized_matmul_rows_workspace_size - workspace bytes
+ * gdn_quantized_matmul splits K with for M > 64 bf16 rows (0: it does not; a
+ * call without a workspace keeps K whole).
+ */
+int64_t gdn_quantized_matmul_rows_workspace_size(int sb_dtype, int M, int N, int K, int bits,
+                                                 int group_size);
 
 /* Quantization modes (the reference's QuantScheme.mode, config.py:17-33). */
 #define GDN_QUANT_AFFINE 0

@@ -75,6 +75,7 @@ _SIGNATURES = {
                                           _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p,
                                           _c_i64, _c_void_p]),
     "gdn_quantized_matmul_f32_workspace_size": (_c_i64, [_c_int, _c_int, _c_int, _c_int, _c_int]),
+    "gdn_quantized_matmul_rows_workspace_size": (_c_i64, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),
     "gdn_dequantize": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int,
                                 _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p]),
     "gdn_quantized_matmul_scheme": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int,

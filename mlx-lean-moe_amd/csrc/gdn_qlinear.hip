@@ -1214,6 +1214,14 @@ extern "C" int64_t gdn_quantized_matmul_workspace_size(int x_dtype, int sb_dtype
     return decode_workspace_bytes(x_f32, sb_dtype, M, N, K, bits, group_size);
 }
 
+extern "C" int64_t gdn_quantized_matmul_rows_workspace_size(int sb_dtype, int M, int N, int K, int bits,
+                                                            int group_size) {
+    if (M <= 64 || N < 1 || K < 1 || (bits != 4 && bits != 8) || !valid_dtype(sb_dtype) ||
+        (group_size != 32 && group_size != 64 && group_size != 128))
+        return 0;
+    return mid_workspace_bytes(M, N, K, group_size, sb_dtype);
+}
+
 namespace gdn {
 namespace {
 
@@ -1253,6 +1261,9 @@ int quantized_matmul(const void* x, int x_dtype, const void* w, const void* scal
     }
     if (x_f32)
         return fail(GDN_EUNSUPPORTED, "gdn_quantized_matmul: float32 x needs a shape the decode kernel takes");
+    if (mid_kernel_takes(M, N, K, group_size, sb_dtype, workspace ? workspace_bytes : 0))
+        return launch_mid(x, wp, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, bits, group_size, workspace,
+                          workspace_bytes, s);
     if (bits == 4) return dispatch_sb<4>(x, wp, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, group_size, s);
     return dispatch_sb<8>(x, wp, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, group_size, s);
 }

@@ -12,7 +12,7 @@
 // no weight is rounded and no product is, which leaves the float32 sums
 // (777 rows of 2048 normal values against 12352 columns of 4-bit codes in
 // groups of 64: 1.2e-7 from float64, where the float32 library product of
-// rounded weights is 8.1e-7 off and takes 345 us to this one's 134).
+// rounded weights is 8.1e-7 off and takes 345 us to this one's 131).
 //
 // Two launches (three where K is split): the preparation cuts x, sums its
 // groups and lays s and b' out group-major; the product kernel does the rest.
@@ -148,10 +148,15 @@ GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__
 // A workgroup holds 16 kTM rows by 256 columns, each of its 4 waves all the
 // rows by 64 columns, so a piece of x read from LDS serves four MFMAs and the
 // codes go from memory to the wave's own B fragments, converted once per
-// workgroup. A step is 64 k: x's pieces through LDS (one tile, the next step's
-// in registers), codes and scales a step ahead in registers. Two workgroups
-// share a CU (256 registers a thread). Per step and wave 24 kTM MFMAs stand
-// beside ~160 instructions of code conversion and 16 kTM of scaling.
+// workgroup. A step is 64 k: x's pieces through two LDS tiles (one barrier a
+// step), the next step's pieces, codes and scales in registers meanwhile. Two
+// workgroups share a CU (256 registers a thread). At 777 rows, 2048 -> 12352,
+// the matrix cores are busy half the time (118 TFLOP of bf16 products against
+// 2.1 PFLOP/s: 58 us of 131): with two waves on a SIMD a wave's LDS reads,
+// conversions and scaling are not all covered. Fetching the codes two steps
+// ahead, or the next row tile's fragments, spilled or gained nothing, and
+// codes converted by the fp8 instruction (uncentred, a third of the
+// instructions) gained 1 % at 2.5 times the error.
 //
 // kG32: groups of 32 (an MFMA's k), each scaled by itself; else one group (64
 // or half of 128) a step. Lane quarter q = l / 16 holds k 8 q .. of each
@@ -169,7 +174,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     constexpr int kPiecesPerRow = kPK / 8;
     constexpr int kXLoads = (kBM * kPiecesPerRow + 255) / 256;
     constexpr int kWords = 2 * kBits / 4;  // packed words of a lane's 16 codes of a step
-    __shared__ __attribute__((aligned(16))) uint16_t xs[kBM * kXS];
+    __shared__ __attribute__((aligned(16))) uint16_t xs[2][kBM * kXS];
 
     // Tiles in row-major order within a column block, an eighth of them to
     // each XCD (workgroups go round-robin over the XCDs): a column block's
@@ -192,7 +197,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 
     // x: rows clamped to M - 1 (not stored); pieces past the tile repeat its last
     const uint16_t* xtile = pieces + int64_t(m0) * K * kParts;
-    uint32_t xo[kXLoads];
+    uint32_t xo[kXLoads];  // byte offsets from a uniform base, as below: no address arithmetic in the loop
     int xl[kXLoads];
 #pragma unroll
     for (int i = 0; i < kXLoads; ++i) {
@@ -200,44 +205,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         idx = idx < kBM * kPiecesPerRow ? idx : kBM * kPiecesPerRow - 1;
         const int row = idx / kPiecesPerRow, seg = idx % kPiecesPerRow;
         const int r = m0 + row < M ? row : M - 1 - m0;
-        xo[i] = uint32_t(r) * uint32_t(K * kParts) + 8 * seg;
+        xo[i] = (uint32_t(r) * uint32_t(K * kParts) + 8 * seg) * 2;
         xl[i] = row * kXS + 8 * seg;
     }
     u16x8 xr[kXLoads];
     auto fetch_x = [&](int s) {
-        const uint16_t* src = xtile + int64_t(s) * kPK;
+        const char* src = reinterpret_cast<const char*>(xtile + int64_t(s) * kPK);
 #pragma unroll
         for (int i = 0; i < kXLoads; ++i) xr[i] = *reinterpret_cast<const u16x8*>(src + xo[i]);
     };
-    auto stage_x = [&] {
+    auto stage_x = [&](int buf) {
 #pragma unroll
-        for (int i = 0; i < kXLoads; ++i) *reinterpret_cast<u16x8*>(xs + xl[i]) = xr[i];
+        for (int i = 0; i < kXLoads; ++i) *reinterpret_cast<u16x8*>(xs[buf] + xl[i]) = xr[i];
     };
 
     const int64_t wpr = int64_t(K) * kBits / 32;
-    uint32_t wd[kTN][kWords];  // words of MFMA block kb at [b][kb kWords / 2 ..]
-    float sc[kTN][kG32 ? 2 : 1];
+    uint32_t wo[kTN], so[kTN];
+#pragma unroll
+    for (int b = 0; b < kTN; ++b) {
+        wo[b] = (uint32_t(col[b] - n0) * uint32_t(wpr) + lq * (kG32 ? kWords / 2 : kWords)) * 4;
+        so[b] = uint32_t(col[b] - n0) * 4;
+    }
+    // a step's codes (words of MFMA block kb at [b][kb kWords / 2 ..]) and scales
+    struct Codes {
+        uint32_t wd[kTN][kWords];
+        float sc[kTN][kG32 ? 2 : 1];
+    };
+    Codes c;
     auto fetch_w = [&](int s) {
-        const int wk = s * kBK * kBits / 32;
+        const char* wtile = reinterpret_cast<const char*>(w + n0 * wpr + s * kBK * kBits / 32);
+        const int g = s * kBK / group_size;
 #pragma unroll
         for (int b = 0; b < kTN; ++b) {
-            const uint32_t* src = w + col[b] * wpr + wk;
-            if constexpr (kG32) {
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(wtile + wo[b]);
 #pragma unroll
-                for (int kb = 0; kb < 2; ++kb)
+            for (int i = 0; i < kWords; ++i) c.wd[b][i] = src[kG32 ? i / (kWords / 2) * kBits + i % (kWords / 2) : i];
 #pragma unroll
-                    for (int i = 0; i < kWords / 2; ++i)
-                        wd[b][kb * kWords / 2 + i] = src[kb * kBits + lq * kWords / 2 + i];
-            } else {
-#pragma unroll
-                for (int i = 0; i < kWords; ++i) wd[b][i] = src[lq * kWords + i];
-            }
-            const int g = s * kBK / group_size;
-#pragma unroll
-            for (int i = 0; i < (kG32 ? 2 : 1); ++i) sc[b][i] = s_t[int64_t(g + i) * N + col[b]];
+            for (int i = 0; i < (kG32 ? 2 : 1); ++i)
+                c.sc[b][i] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(s_t + int64_t(g + i) * N + n0) + so[b]);
         }
     };
 
+    const int last = step0 + steps - 1;
     fetch_x(step0);
     fetch_w(step0);
 
@@ -267,25 +276,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
                 acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? xa[a] : 0.f, in ? bb[b] : 0.f, acc[a][b], 0, 0, 0);
     }
 
-    stage_x();
-    for (int s = step0; s < step0 + steps; ++s) {
+    stage_x(0);
+    for (int s = step0; s <= last; ++s) {
         bf16x8 bf[kTN][2];
         float scale[kTN][kG32 ? 2 : 1];
 #pragma unroll
         for (int b = 0; b < kTN; ++b) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) bf[b][kb] = centred_fragment<kBits>(&wd[b][kb * kWords / 2]);
+            for (int kb = 0; kb < 2; ++kb) bf[b][kb] = centred_fragment<kBits>(&c.wd[b][kb * kWords / 2]);
 #pragma unroll
-            for (int i = 0; i < (kG32 ? 2 : 1); ++i) scale[b][i] = sc[b][i];
+            for (int i = 0; i < (kG32 ? 2 : 1); ++i) scale[b][i] = c.sc[b][i];
         }
-        const int next = s + 1 < step0 + steps ? s + 1 : s;  // the last step repeats itself
+        const int next = s < last ? s + 1 : last;  // the last step again, unused
         fetch_x(next);
         fetch_w(next);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
 #pragma unroll
         for (int a = 0; a < kTM; ++a) {
-            const uint16_t* xrow = xs + (16 * a + lr) * kXS;
+            const uint16_t* xrow = xs[(s - step0) & 1] + (16 * a + lr) * kXS;
             bf16x8 af[kParts][2];
 #pragma unroll
             for (int p = 0; p < kParts; ++p)
@@ -313,8 +322,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
             }
             if constexpr (!kG32) scaled(0);
         }
-        __syncthreads();
-        stage_x();
+        stage_x((s - step0 + 1) & 1);
     }
 
     int any = 0;

@@ -38,9 +38,8 @@ _MODES = {"affine": 0, "mxfp4": 1, "mxfp8": 2, "nvfp4": 3}
 # dequantize, then multiply on the vendor BLAS)
 _KERNEL_BITS = {4, 8}
 # From this many rows on, quantized_linear dequantizes the weights to bf16
-# once and multiplies on the vendor BLAS (measured at hidden 2048 -> 12352:
-# 73 vs 103 us at 1024 rows, 242 vs 336 us at 4096; even at 512 rows);
-# below it gdn_quantized_matmul's kernels run directly, see _dense_rows.
+# once and multiplies on the vendor BLAS; below it gdn_quantized_matmul's
+# kernels run directly where _mid_rows or _dense_rows says so.
 _BLAS_ROWS = 512
 # quantized_linear_split multiplies per block from this many rows on (one
 # product of the stacked 2048 -> 12352 weight: 32.7 us at 512 rows against
@@ -49,18 +48,41 @@ _BLAS_ROWS = 512
 _SPLIT_ROWS = 2048
 
 
+def _mid_rows(rows: int, N: int, K: int, group_size: int, sb_dtype: torch.dtype) -> bool:
+    """Whether more than 64 bf16 rows run on gdn_quantized_matmul's kernel for
+    them (gdn_qlinear_mid.hip), which takes K in steps of 256 with a k range's
+    scales and biases of 128 columns in 32 KB of LDS, rather than on
+    dequantized weights and the vendor BLAS (which read the codes once more as
+    bf16, but keep the larger tiles busy). Device time from graphs, kernel
+    against dense, us: 2048 -> 12352 at 66 rows 21 and 35, 200 rows 28 and 43,
+    256 rows 40 and 43, 384 rows 47 and 46, 512 rows 55 and 52; 4096 -> 12352
+    at 200 rows 47 and 60; 1024 -> 12352 at 500 rows 36 and 41; 4096 -> 2048 at
+    128 rows 17 and 24, 384 rows 26 and 29, 600 rows 36 and 27; 2048 -> 2048 at
+    350 rows 22 and 19. Up to 224 rows the largest of these is one workgroup a
+    CU."""
+
+    if rows <= 64 or K % 256 or K // group_size * 256 * sb_dtype.itemsize > 32768:
+        return False
+    if N * K > 26_000_000 or (N < 4096 and K < 4096):
+        return rows <= 224
+    return rows <= (384 if K >= 2048 else _BLAS_ROWS - 1)
+
+
 def _dense_rows(rows: int, N: int, K: int) -> bool:
-    """Whether ``rows`` bf16 rows times a quantized ``(N, K)`` weight run on
-    dequantized weights and the vendor BLAS rather than the quantized
-    kernels. Above 64 rows the quantized tiled kernel takes 128 x 128 tiles
-    with no K split, so a narrow or deep weight leaves the GPU idle: for
-    4096 -> 2048 (out_proj) it takes 73-76 us from 65 to 1024 rows against
-    23-34 us dense; for 2048 -> 12352 it wins up to ~400 rows (41-44 us
-    against 45-57 us, device time from graphs)."""
+    """Whether ``rows`` bf16 rows times a quantized ``(N, K)`` weight that
+    _mid_rows leaves run on dequantized weights and the vendor BLAS rather
+    than the tiled kernel. That one takes 128 x 128 tiles with no K split, so
+    a narrow or deep weight leaves the GPU idle: for 4096 -> 2048 (out_proj)
+    it takes 73-76 us from 65 to 1024 rows against 23-34 us dense; for 2048 ->
+    12352 it is even around 300 rows."""
 
     if rows >= _BLAS_ROWS:
         return True
     return rows > 64 and (N < 4096 or K >= 4096)
+
+
+def _runs_dense(rows: int, N: int, K: int, group_size: int, sb_dtype: torch.dtype) -> bool:
+    return _dense_rows(rows, N, K) and not _mid_rows(rows, N, K, group_size, sb_dtype)
 
 
 @dataclass(frozen=True)
@@ -242,7 +264,7 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
     if x.dtype != torch.bfloat16 and not x_f32:
         return with_residual(x @ dequantize(tensors, quant, x.dtype).T)
     x2 = _c(x.reshape(-1, K))
-    if _dense_rows(x2.shape[0], N, K):
+    if _runs_dense(x2.shape[0], N, K, quant.group_size, scales.dtype):
         # the same bf16-rounded weights as the tiled kernel (gdn_dequantize),
         # one transient copy, and the vendor BLAS for the GEMM itself
         wd = dense if dense is not None else dequantize(tensors, quant, torch.bfloat16)
@@ -332,7 +354,7 @@ def quantized_linear_split(x: torch.Tensor, weights: LinearWeights, sizes) -> li
     (which sum to ``W``'s rows): what :func:`quantized_linear` of each
     projection would give, in one launch where that pays.
 
-    Where the dense path runs (bf16 ``x``, :func:`_dense_rows`: prefill
+    Where the dense path runs (bf16 ``x``, :func:`_runs_dense`: prefill
     sizes) ``W`` is dequantized once (or its kept copy used); from
     ``_SPLIT_ROWS`` rows on each block is its own GEMM on the vendor BLAS
     with a packed output: for hidden 2048 -> 8192|4096|64 at 4096 rows the
@@ -349,7 +371,7 @@ def quantized_linear_split(x: torch.Tensor, weights: LinearWeights, sizes) -> li
     K = x.shape[-1]
     rows = x.reshape(-1, K).shape[0]
     if (x.dtype == torch.bfloat16 and x.device.type == "cuda"
-            and (_dense_rows(rows, tensors["weight"].shape[0], K)
+            and (_runs_dense(rows, tensors["weight"].shape[0], K, quant.group_size, tensors["scales"].dtype)
                  or not (_on_kernels(quant) or _scheme_kernel_takes(x, rows, K, quant)))):
         _check_quantized(tensors, quant, K)
         lead = x.shape[:-1]
@@ -387,6 +409,9 @@ def workspace_bytes(x_dtype: torch.dtype, sb_dtype: torch.dtype, M: int, N: int,
                     group_size: int) -> int:
     """Workspace gdn_quantized_matmul splits K with for these sizes (0: none)."""
 
+    if M > 64:
+        return int(_lib.load().gdn_quantized_matmul_rows_workspace_size(
+            _lib.dtype_code(sb_dtype), M, N, K, bits, group_size))
     return int(_lib.load().gdn_quantized_matmul_workspace_size(
         _lib.dtype_code(x_dtype), _lib.dtype_code(sb_dtype), M, N, K, bits, group_size))
 

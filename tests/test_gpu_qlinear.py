@@ -604,3 +604,41 @@ def test_float32_rows_outside_the_pieces_range(gpu, N, K):
     np.testing.assert_array_equal(np.isnan(y[~finite]), np.isnan(ref[~finite]))
     inf = np.isinf(ref)
     np.testing.assert_array_equal(y[inf], ref[inf].astype(np.float32))
+
+
+@pytest.mark.parametrize("M,N,K,bits,gs,sb", [
+    (65, 300, 256, 4, 64, "bf16"),      # one step; ragged columns; the fewest rows
+    (112, 128, 512, 4, 32, "f16"),      # a whole 112-row tile, two groups a lane quarter pair
+    (113, 130, 768, 4, 128, "bf16"),    # an odd step count, half a group a wave
+    (200, 2048, 4096, 4, 64, "bf16"),   # K split over the grid
+    (130, 257, 1024, 8, 64, "f32"),
+    (220, 100, 2048, 8, 32, "bf16"),    # the most groups the LDS holds
+    (100, 64, 1024, 4, 32, "f32"),      # the same in float32
+])
+def test_rows_above_the_decode_sizes(gpu, M, N, K, bits, gs, sb):
+    """65 to 511 bf16 rows: x times the weights rounded to bf16, with and
+    without a workspace to split K in, within float32 sums of the float64
+    product: at most K + 20 roundings of 2^-24 of the magnitudes added."""
+    from mlx_lean_moe_amd.quant import _mid_rows, workspace_bytes
+
+    assert _mid_rows(M, N, K, gs, _TORCH[sb])
+    rng = np.random.default_rng(M * 3 + N)
+    words, s, b = _weights(rng, N, K, bits, gs, sb)
+    W = _dev_weights(gpu, words, s, b, sb)
+    x = R.bf16_round(rng.standard_normal((M, K)))
+    w = Q.dequantize(words, s, b, bits, gs, out="bf16").astype(np.float64)
+    ref = x.astype(np.float64) @ w.T
+    bound = (K + 20) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    xt = torch.tensor(x, dtype=torch.float32, device=gpu).to(torch.bfloat16)
+    nbytes = workspace_bytes(torch.bfloat16, _TORCH[sb], M, N, K, bits, gs)
+    assert nbytes > 0 or N != 2048
+    for ws in (None, torch.empty(nbytes, dtype=torch.uint8, device=gpu) if nbytes else None):
+        y = torch.empty(M, N, device=gpu)
+        _lib.call("gdn_quantized_matmul", _lib.ptr(xt), _lib.GDN_BF16, _lib.ptr(W["weight"]), _lib.ptr(W["scales"]),
+                  _lib.ptr(W["biases"]), _lib.dtype_code(W["scales"].dtype), _lib.ptr(y), _lib.GDN_F32, None, M, N, K,
+                  bits, gs, _lib.ptr(ws), nbytes if ws is not None else 0, _lib.stream_ptr(xt.device))
+        assert (np.abs(y.cpu().numpy() - ref) <= bound).all()
+    r = torch.tensor(rng.standard_normal((M, N)), dtype=torch.float32, device=gpu).to(torch.bfloat16)
+    y = gdn.quantized_linear(xt, W, gdn.QuantScheme(bits, gs))
+    assert (np.abs(y.float().cpu().numpy() - ref) <= bound + 2.0 ** -8 * np.abs(ref)).all()
+    assert torch.equal(gdn.quantized_linear(xt, W, gdn.QuantScheme(bits, gs), residual=r), y + r)
