@@ -1397,44 +1397,78 @@ GDN_DEV float e4m3_value(uint32_t c) {
 
 GDN_DEV float e8m0_value(uint32_t c) { return c == 255 ? __builtin_nanf("") : ldexpf(1.f, int(c) - 127); }
 
-// Dense weights of any scheme QuantScheme accepts, one thread per 32
-// elements of a row (the last may hold 16): element k of a row is the
-// bits-wide field at bit bits * k of the row's little-endian bit stream
-// (MLX packs 3-, 5- and 6-bit codes into byte groups, which reads the same),
-// so a thread's 32 codes are its `bits` consecutive words. affine:
-// s * q + b in float32, rounded once to out's dtype; mxfp4 / mxfp8 / nvfp4:
-// the code's value times the group's scale (e8m0, or e4m3 for nvfp4), exact
-// in float32 and in bf16 (at most 6 significant bits).
+// Dense weights of any scheme QuantScheme accepts: element k of a row is the
+// kBits-wide field at bit kBits k of the row's little-endian bit stream (MLX
+// packs 3-, 5- and 6-bit codes into byte groups, which reads the same).
+// affine: s q + b in float32, rounded once to out's dtype; mxfp4 / mxfp8 /
+// nvfp4: the code's value (gfx950's conversions) times the group's scale
+// (e8m0, or e4m3 for nvfp4), exact in float32 and in bf16 (at most 6
+// significant bits).
+// A thread takes 8 consecutive codes: kBits whole bytes inside two words, one
+// group's scale, one 16-byte store (two in float32), so a wave writes whole
+// lines. wide: out is 16-byte aligned (K is a multiple of 16). With 32 codes a
+// thread, each stored by itself (a wave's stores 64 bytes apart), a 512-row
+// product with 12352 x 2048 mxfp4, mxfp8, nvfp4, 3- or 6-bit weights took
+// 280-286 us, nearly all of it here; 51-53 now, as with the 4-bit codes.
+template <int kMode, int kBits>
 __global__ __launch_bounds__(256) void dequantize_scheme_kernel(
     const uint32_t* __restrict__ w, const void* __restrict__ scales, const void* __restrict__ biases,
-    int sb_dtype, void* __restrict__ out, int out_dtype, int N, int K, int bits, int group_size, int mode) {
-    const int chunks = (K + 31) / 32;
-    const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+    int sb_dtype, void* __restrict__ out, int out_dtype, int N, int K, int group_size, bool wide) {
+    const int chunks = K / 8;
+    const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
     if (t >= int64_t(N) * chunks) return;
-    const int n = int(t / chunks), k0 = int(t % chunks) * 32;
-    const int64_t row_words = int64_t(K) * bits / 32;
-    const uint32_t* rw = w + int64_t(n) * row_words + int64_t(k0) * bits / 32;
-    const int words = int((int64_t(K - k0 < 32 ? K - k0 : 32) * bits + 31) / 32);
-    uint32_t wd[9];
+    const int64_t n = t / chunks, row_words = int64_t(K) * kBits / 32;
+    const int k0 = int(t % chunks) * 8;
+    const int64_t bit = int64_t(k0) * kBits;
+    const int first = int(bit / 32), shift = int(bit % 32);
+    const uint32_t* rw = w + n * row_words;
+    // the second word is clamped into the row: past it no code needs it
+    const uint64_t pair = uint64_t(rw[first]) | uint64_t(rw[first + 1 < row_words ? first + 1 : first]) << 32;
+    const uint64_t run = pair >> shift;
+    const int64_t g = n * (K / group_size) + k0 / group_size;
+    float v[8];
+    if constexpr (kMode == GDN_QUANT_AFFINE) {
+        const float sc = load_any(scales, g, sb_dtype), b = load_any(biases, g, sb_dtype);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) wd[i] = i < words ? rw[i] : 0u;
-    const uint32_t mask = (1u << bits) - 1u;
-    const int gpr = K / group_size;
-    const int64_t sb_row = int64_t(n) * gpr;
-    for (int e = 0; e < 32 && k0 + e < K; ++e) {
-        const int off = bits * e, wi = off >> 5, sh = off & 31;
-        const uint64_t pair = uint64_t(wd[wi]) | (uint64_t(wd[wi + 1]) << 32);
-        const uint32_t q = uint32_t(pair >> sh) & mask;
-        const int64_t g = sb_row + (k0 + e) / group_size;
-        float v;
-        if (mode == GDN_QUANT_AFFINE) {
-            v = __builtin_fmaf(load_any(scales, g, sb_dtype), float(q), load_any(biases, g, sb_dtype));
+        for (int j = 0; j < 8; ++j)
+            v[j] = __builtin_fmaf(sc, float(uint32_t(run >> (kBits * j)) & ((1u << kBits) - 1u)), b);
+    } else {
+        const uint32_t code = static_cast<const uint8_t*>(scales)[g];
+        const float sc = kMode == GDN_QUANT_NVFP4 ? e4m3_value(code) : e8m0_value(code);
+        const uint32_t lo = uint32_t(run), hi = uint32_t(run >> 32);
+        if constexpr (kMode == GDN_QUANT_MXFP8) {
+            const auto f0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 1.0f, false);
+            const auto f1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 1.0f, true);
+            const auto f2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 1.0f, false);
+            const auto f3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 1.0f, true);
+            const float f[8] = {f0[0], f0[1], f1[0], f1[1], f2[0], f2[1], f3[0], f3[1]};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = f[j] * sc;
         } else {
-            const uint32_t sc = static_cast<const uint8_t*>(scales)[g];
-            const float code = mode == GDN_QUANT_MXFP8 ? e4m3_value(q) : e2m1_value(q);
-            v = code * (mode == GDN_QUANT_NVFP4 ? e4m3_value(sc) : e8m0_value(sc));
+            const auto f0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(lo, 1.0f, 0);
+            const auto f1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(lo, 1.0f, 1);
+            const auto f2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(lo, 1.0f, 2);
+            const auto f3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(lo, 1.0f, 3);
+            const float f[8] = {f0[0], f0[1], f1[0], f1[1], f2[0], f2[1], f3[0], f3[1]};
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = f[j] * sc;
         }
-        store_any(out, int64_t(n) * K + k0 + e, out_dtype, v);
+    }
+    const int64_t at = n * K + k0;
+    if (!wide) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) store_any(out, at + j, out_dtype, v[j]);
+    } else if (out_dtype == GDN_F32) {
+        float4* dst = reinterpret_cast<float4*>(static_cast<float*>(out) + at);
+        dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+        dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+    } else if (out_dtype == GDN_BF16) {
+        *reinterpret_cast<uint4*>(static_cast<uint16_t*>(out) + at) = pack8(v);
+    } else {
+        u16x8 h;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) h[j] = f32_to_f16_bits(v[j]);
+        *reinterpret_cast<u16x8*>(static_cast<uint16_t*>(out) + at) = h;
     }
 }
 
@@ -1891,9 +1925,19 @@ extern "C" int gdn_dequantize(const void* w, const void* scales, const void* bia
     const int64_t threads = int64_t(N) * ((K + 31) / 32);
     GDN_REQUIRE(threads < (int64_t(1) << 31), "gdn_dequantize: %lld elements exceed the grid",
                 (long long)N * K);
-    hipLaunchKernelGGL(dequantize_scheme_kernel, dim3(unsigned((threads + 255) / 256)), dim3(256), 0, s,
-                       static_cast<const uint32_t*>(w), scales, biases, sb_dtype, out, out_dtype, N, K, bits,
-                       group_size, mode);
+    auto kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 2>;
+    switch (mode) {
+        case GDN_QUANT_MXFP4: kernel = dequantize_scheme_kernel<GDN_QUANT_MXFP4, 4>; break;
+        case GDN_QUANT_MXFP8: kernel = dequantize_scheme_kernel<GDN_QUANT_MXFP8, 8>; break;
+        case GDN_QUANT_NVFP4: kernel = dequantize_scheme_kernel<GDN_QUANT_NVFP4, 4>; break;
+        default:
+            if (bits == 3) kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 3>;
+            if (bits == 5) kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 5>;
+            if (bits == 6) kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 6>;
+    }
+    hipLaunchKernelGGL(kernel, dim3(unsigned((int64_t(N) * (K / 8) + 255) / 256)), dim3(256), 0, s,
+                       static_cast<const uint32_t*>(w), scales, biases, sb_dtype, out, out_dtype, N, K, group_size,
+                       reinterpret_cast<uintptr_t>(out) % 16 == 0);
     return check_launch("gdn_dequantize");
 }
 

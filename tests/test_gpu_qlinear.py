@@ -642,3 +642,35 @@ def test_rows_above_the_decode_sizes(gpu, M, N, K, bits, gs, sb):
     y = gdn.quantized_linear(xt, W, gdn.QuantScheme(bits, gs))
     assert (np.abs(y.float().cpu().numpy() - ref) <= bound + 2.0 ** -8 * np.abs(ref)).all()
     assert torch.equal(gdn.quantized_linear(xt, W, gdn.QuantScheme(bits, gs), residual=r), y + r)
+
+
+@pytest.mark.parametrize("mode,bits,gs", [("mxfp4", 4, 32), ("mxfp8", 8, 32), ("nvfp4", 4, 16), ("affine", 3, 32),
+                                          ("affine", 5, 64), ("affine", 6, 32), ("affine", 2, 128)])
+@pytest.mark.parametrize("out", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_dequantize_into_any_alignment(gpu, mode, bits, gs, out, shift):
+    """Every code under every scale code (NaN and the smallest among them),
+    rows that end inside a word pair, outputs on and off 16 bytes, and nothing
+    written beyond the output."""
+    rng = np.random.default_rng(bits + gs + shift)
+    K, N = 3 * max(gs, 32), 256
+    q = rng.integers(0, 2 ** bits, (N, K))
+    q[:, :2 ** min(bits, 4)] = np.arange(2 ** min(bits, 4))
+    if mode == "affine":
+        s = R.bf16_round(rng.standard_normal((N, K // gs)))
+        b = R.bf16_round(rng.standard_normal((N, K // gs)))
+        ref = Q.dequantize(Q.pack(q, bits), s, b, bits, gs, out=out)
+        scales, biases = (torch.tensor(v, dtype=torch.float32, device=gpu) for v in (s, b))
+    else:
+        s = np.repeat(np.arange(256)[:, None], K // gs, 1)
+        with np.errstate(all="ignore"):
+            ref = torch.tensor(Q.dequantize_fp(Q.pack(q, bits), s, mode, gs)).float().to(_TORCH[out]).float().numpy()
+        scales, biases = torch.tensor(s.astype(np.uint8), device=gpu), None
+    w = torch.tensor(Q.pack(q, bits).view(np.int32), device=gpu)
+    buf = torch.full((N * K + 16,), 7.0, dtype=_TORCH[out], device=gpu)
+    _lib.call("gdn_dequantize", _lib.ptr(w), _lib.ptr(scales), _lib.ptr(biases), _lib.GDN_F32, _lib.ptr(buf[shift:]),
+              _lib.dtype_code(buf.dtype), N, K, bits, gs, {"affine": 0, "mxfp4": 1, "mxfp8": 2, "nvfp4": 3}[mode],
+              _lib.stream_ptr(buf.device))
+    got = buf.float().cpu().numpy()
+    np.testing.assert_array_equal(got[shift:shift + N * K].reshape(N, K), ref)
+    assert (got[:shift] == 7).all() and (got[shift + N * K:] == 7).all()
