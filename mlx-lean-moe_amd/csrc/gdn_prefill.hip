@@ -696,13 +696,14 @@ constexpr int kStateThreads = 512;
 // A state-pass workgroup holds its CU to itself (256 registers a thread, the
 // prefetch ring three chunks deep), which suits a grid of one a CU: the chain
 // of chunk steps is all there is to hide. With more workgroups than CUs a
-// second one on the CU hides more than the deep ring does: bf16 calls above
-// 256 workgroups take prefill_state_shared_kernel (128 registers, 76 KB of
-// LDS, the same bits). Whole calls, us, one a CU against two: 3 runs of 2048
-// tokens at 16 heads (384 workgroups) 120 -> 116, one run of 2048 at 64 heads
-// (512) 131 -> 126, 3 x 777 at 32 (768) 86 -> 79, 32 x 64 at 16 (4096) 87 ->
-// 52, 16 packed runs of 67 128 tokens in all at 32 heads 2232 -> 2054. Float32
-// tiles (111 KB) leave no room for a second workgroup.
+// second one on the CU hides more than the deep ring does: calls above 256
+// workgroups take prefill_state_shared_kernel (128 registers and 76-78 KB of
+// LDS, the same bits). Whole calls, us, one a CU against two, bf16: 3 runs of
+// 2048 tokens at 16 heads (384 workgroups) 120 -> 116, one run of 2048 at 64
+// heads (512) 131 -> 126, 3 x 777 at 32 (768) 86 -> 79, 32 x 64 at 16 (4096)
+// 87 -> 52, 16 packed runs of 67 128 tokens in all at 32 heads 2232 -> 2054;
+// float32 in the same order 193 -> 171, 192 -> 172, 145 -> 131, 99 -> 84, and
+// 8 packed runs of 300 to 1000 tokens at 32 heads 315 -> 287.
 constexpr int kStateSharedAbove = 256;
 
 // Chunk operands of state wave w, fetched by output wave w. They pass
@@ -844,17 +845,19 @@ GDN_DEV void fetch_output(OutputOperands& op, const StatePassCtx& cx, int c, int
 
 // kF32 (float32 q, k, v): K and V also keep their bf16 residuals (Q stays
 // in the output waves' registers for either input).
-template <bool kF32>
+// kKBufs: K tiles held (with float32 input one leaves room for a second
+// workgroup on the CU).
+template <bool kF32, int kKBufs>
 struct StatePassLds {
     uint16_t Ss_hi[kSliceRows * kSS], Ss_lo[kSliceRows * kSS];  // S[dv][dk]
-    uint16_t Kr[2][kChunk * kHD];                                 // K[token][dk] (swizzled), two buffers
+    uint16_t Kr[kKBufs][kChunk * kHD];                            // K[token][dk] (swizzled)
     uint16_t Tb_hi[kChunk * kTS], Tb_lo[kChunk * kTS];            // Tb[token][token]
     uint16_t Vs[kChunk * kSliceRows];                             // V[token][dv]
     uint16_t Rs_hi[kSliceRows * kTS], Rs_lo[kSliceRows * kTS];    // R[dv][token]
     uint16_t Ds_hi[kSliceRows * kTS], Ds_lo[kSliceRows * kTS];    // D[dv][token]
     uint16_t D2_hi[kSliceRows * kTS], D2_lo[kSliceRows * kTS];    // D''[dv][token]
     float ex[2 * kChunk];                                         // exp(l), exp(l_C - l)
-    uint16_t Kr_lo[kF32 ? 2 : 1][kF32 ? kChunk * kHD : 8];        // residuals (float32 input)
+    uint16_t Kr_lo[kF32 ? kKBufs : 1][kF32 ? kChunk * kHD : 8];   // residuals (float32 input)
     uint16_t Vs_lo[kF32 ? kChunk * kSliceRows : 8];
 };
 
@@ -887,8 +890,8 @@ GDN_DEV void split8_bits(const bf16x8& a, const bf16x8& b, bf16x8& hi, bf16x8& l
     lo = __builtin_bit_cast(bf16x8, r);
 }
 
-template <bool kF32>
-GDN_DEV void stage_k(const StagedOperands& op, StatePassLds<kF32>& sm, int buf, int w, int l) {
+template <bool kF32, int kKBufs>
+GDN_DEV void stage_k(const StagedOperands& op, StatePassLds<kF32, kKBufs>& sm, int buf, int w, int l) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int o = kr_off(16 * w + 4 * i + (l >> 4), l & 15);
@@ -903,8 +906,8 @@ GDN_DEV void stage_k(const StagedOperands& op, StatePassLds<kF32>& sm, int buf, 
     }
 }
 
-template <bool kF32>
-GDN_DEV void stage_v(const StagedOperands& op, StatePassLds<kF32>& sm, int w, int l) {
+template <bool kF32, int kKBufs>
+GDN_DEV void stage_v(const StagedOperands& op, StatePassLds<kF32, kKBufs>& sm, int w, int l) {
     const int o = (16 * w + (l >> 2)) * kSliceRows + 4 * (l & 3);
     if constexpr (kF32) {
         uint32_t h0, r0, h1, r1;
@@ -919,8 +922,8 @@ GDN_DEV void stage_v(const StagedOperands& op, StatePassLds<kF32>& sm, int w, in
 
 // Lanes 8-63 repeat lanes 0-7 for the decay words (same words, same values):
 // an unconditional store keeps the operand registers out of any branch.
-template <bool kUpper, bool kF32>
-GDN_DEV void stage_tb_e(const StagedOperands& op, StatePassLds<kF32>& sm, int w, int l) {
+template <bool kUpper, bool kF32, int kKBufs>
+GDN_DEV void stage_tb_e(const StagedOperands& op, StatePassLds<kF32, kKBufs>& sm, int w, int l) {
     const int row = (16 * w + (l & 15)) * kTS + 8 * (l >> 4);
 #pragma unroll
     for (int s = 0; s < (kUpper ? 2 : 1); ++s) {
@@ -931,8 +934,8 @@ GDN_DEV void stage_tb_e(const StagedOperands& op, StatePassLds<kF32>& sm, int w,
 }
 
 // State waves, chunk part 1: the S operand (hi + lo) into LDS.
-template <bool kF32>
-GDN_DEV void state_stage(const f32x4 (&acc)[2], StatePassLds<kF32>& sm, int w, int l) {
+template <bool kF32, int kKBufs>
+GDN_DEV void state_stage(const f32x4 (&acc)[2], StatePassLds<kF32, kKBufs>& sm, int w, int l) {
     const int lr = l & 15, lq = l >> 4;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -947,8 +950,8 @@ GDN_DEV void state_stage(const f32x4 (&acc)[2], StatePassLds<kF32>& sm, int w, i
 
 // State waves, part 2 (between the staging and R barriers):
 // R^T = V^T - S K^T diag(exp l), lane (dv = 4(l/16) + i, token = 16w + l%16).
-template <bool kF32>
-GDN_DEV void state_residual(const StatePassLds<kF32>& sm, StatePassLds<kF32>& smw, int buf, int w, int l) {
+template <bool kF32, int kKBufs>
+GDN_DEV void state_residual(const StatePassLds<kF32, kKBufs>& sm, StatePassLds<kF32, kKBufs>& smw, int buf, int w, int l) {
     const int lr = l & 15, lq = l >> 4, lg8 = 8 * lq;
     const int tok = 16 * w + lr;
     f32x4 xk = {0.f, 0.f, 0.f, 0.f}, xk2 = xk;
@@ -986,8 +989,8 @@ GDN_DEV void state_residual(const StatePassLds<kF32>& sm, StatePassLds<kF32>& sm
 
 // State waves, part 3 (between the R and D barriers): D = Tb R, stored as
 // D (hi + lo, for Y) and D'' = exp(l_C - l) D (hi + lo, for the update).
-template <bool kUpper, bool kF32>
-GDN_DEV void state_delta(StatePassLds<kF32>& sm, int w, int l) {
+template <bool kUpper, bool kF32, int kKBufs>
+GDN_DEV void state_delta(StatePassLds<kF32, kKBufs>& sm, int w, int l) {
     const int lr = l & 15, lq = l >> 4, lg8 = 8 * lq;
     const int row = (16 * w + lr) * kTS + lg8;
     f32x4 d = {0.f, 0.f, 0.f, 0.f}, d2 = d;
@@ -1021,8 +1024,8 @@ GDN_DEV void state_delta(StatePassLds<kF32>& sm, int w, int l) {
 // within each 16-lane group, lane i of a ds_read_b64_tr_b16 receives element
 // i%4 of source lane i/4 + 4k (k = 0..3); source lane s of group g points at
 // K[8g + 4h + s/4][dk0 + 4(s%4)] for the tokens 8g + 4h .. +3.
-template <bool kF32>
-GDN_DEV void state_update(f32x4 (&acc)[2], const StatePassLds<kF32>& sm, int buf, float eC, int w,
+template <bool kF32, int kKBufs>
+GDN_DEV void state_update(f32x4 (&acc)[2], const StatePassLds<kF32, kKBufs>& sm, int buf, float eC, int w,
                           int l) {
     const int g = l >> 4, sl = l & 15, lr = sl, lg8 = 8 * g;
     const uint16_t* kr = sm.Kr[buf];
@@ -1057,8 +1060,8 @@ GDN_DEV void state_update(f32x4 (&acc)[2], const StatePassLds<kF32>& sm, int buf
 
 // Output waves, part 1 (between the staging and R barriers): exp(l) Q S^T,
 // Q from the wave's registers (the chunk's operands).
-template <bool kF32>
-GDN_DEV f32x4 output_project(const StagedOperands& op, const StatePassLds<kF32>& sm, int w, int l) {
+template <bool kF32, int kKBufs>
+GDN_DEV f32x4 output_project(const StagedOperands& op, const StatePassLds<kF32, kKBufs>& sm, int w, int l) {
     const int lr = l & 15, lq = l >> 4, lg8 = 8 * lq;
     f32x4 xq = {0.f, 0.f, 0.f, 0.f}, xq2 = xq;
 #pragma unroll
@@ -1080,8 +1083,8 @@ GDN_DEV f32x4 output_project(const StagedOperands& op, const StatePassLds<kF32>&
 }
 
 // Output waves, part 2 (after the D barrier): y = exp(l) Q S^T + P D.
-template <class Y, bool kUpper, bool kF32>
-GDN_DEV void output_store(const OutputOperands& op, f32x4 yacc, const StatePassLds<kF32>& sm,
+template <class Y, bool kUpper, bool kF32, int kKBufs>
+GDN_DEV void output_store(const OutputOperands& op, f32x4 yacc, const StatePassLds<kF32, kKBufs>& sm,
                           const StatePassCtx& cx, int c, typename Y::storage* __restrict__ y, int w,
                           int l) {
     const int lr = l & 15, lq = l >> 4, lg8 = 8 * lq;
@@ -1125,8 +1128,8 @@ GDN_DEV void output_store(const OutputOperands& op, f32x4 yacc, const StatePassL
 // lets the compiler sink the first step's prefetch (invariant loads) to just
 // before its use. Chunk indices past the run repeat its last chunk, so every
 // fetch is unconditional.
-template <bool kUpper, bool kF32>
-GDN_DEV void state_loop(int nch, StatePassLds<kF32>& sm, f32x4 (&acc)[2], int w, int l) {
+template <bool kUpper, bool kF32, int kKBufs>
+GDN_DEV void state_loop(int nch, StatePassLds<kF32, kKBufs>& sm, f32x4 (&acc)[2], int w, int l) {
     auto step = [&](int buf) {
         state_stage(acc, sm, w, l);
         __syncthreads();
@@ -1136,11 +1139,12 @@ GDN_DEV void state_loop(int nch, StatePassLds<kF32>& sm, f32x4 (&acc)[2], int w,
         state_delta<kUpper>(sm, w, l);
         __syncthreads();
         state_update(acc, sm, buf, eC, w, l);
+        if constexpr (kKBufs == 1) __syncthreads();  // the next chunk's K takes this one's place
     };
     int c = 0;
     for (; c + 1 < nch; c += 2) {
         step(0);
-        step(1);
+        step(kKBufs - 1);
     }
     if (c < nch) step(0);
 }
@@ -1148,7 +1152,7 @@ GDN_DEV void state_loop(int nch, StatePassLds<kF32>& sm, f32x4 (&acc)[2], int w,
 // Float32 input (operands with their residuals): chunk c + 2's operands
 // fetched at step c, its P fragments one chunk ahead.
 template <class Y, bool kUpper, bool kF32>
-GDN_DEV void output_loop_2ahead(const StatePassCtx& cx, int nch, StatePassLds<kF32>& sm,
+GDN_DEV void output_loop_2ahead(const StatePassCtx& cx, int nch, StatePassLds<kF32, 2>& sm,
                          typename Y::storage* __restrict__ y, int w, int l) {
     const int last = nch - 1;
     StagedOperands ga, gb;
@@ -1191,7 +1195,7 @@ GDN_DEV void output_loop_2ahead(const StatePassCtx& cx, int nch, StatePassLds<kF
 // the second and third barrier is the step's longest). Chunk c's operands
 // live in slot c % 3 of the ring, its P fragments in slot c % 3 of theirs.
 template <class Y, bool kUpper, bool kF32>
-GDN_DEV void output_loop_3ahead(const StatePassCtx& cx, int nch, StatePassLds<kF32>& sm,
+GDN_DEV void output_loop_3ahead(const StatePassCtx& cx, int nch, StatePassLds<kF32, 2>& sm,
                                 typename Y::storage* __restrict__ y, int w, int l) {
     const int last = nch - 1;
     const auto at = [&](int c) { return c < last ? c : last; };
@@ -1237,7 +1241,7 @@ GDN_DEV void output_loop_3ahead(const StatePassCtx& cx, int nch, StatePassLds<kF
 // of the ring above) keeps the loads about a step ahead, and the other
 // workgroup's work covers what of their latency is left.
 template <class Y, bool kUpper>
-GDN_DEV void output_loop_1ahead(const StatePassCtx& cx, int nch, StatePassLds<false>& sm,
+GDN_DEV void output_loop_1ahead(const StatePassCtx& cx, int nch, StatePassLds<false, 2>& sm,
                                 typename Y::storage* __restrict__ y, int w, int l) {
     const int last = nch - 1;
     const auto at = [&](int c) { return c < last ? c : last; };
@@ -1276,14 +1280,51 @@ GDN_DEV void output_loop_1ahead(const StatePassCtx& cx, int nch, StatePassLds<fa
     if (c < nch) step(c, 0);
 }
 
-// kShared: two workgroups of the kernel share a CU (bf16 input).
+// The same for float32 input, whose operands are twice as many: a fourth
+// barrier lets one K tile (hi + lo) do, and K, V and Tb are fetched in the
+// step before they are staged (phases apart, not a step), so that they and
+// the Q and P fragments fit 128 registers.
+template <class Y, bool kUpper>
+GDN_DEV void output_loop_one_k(const StatePassCtx& cx, int nch, StatePassLds<true, 1>& sm,
+                               typename Y::storage* __restrict__ y, int w, int l) {
+    const int last = nch - 1;
+    StagedOperands g;
+    OutputOperands p;
+    fetch_staged<kUpper, true>(g, cx, 0, w, l);
+    stage_k(g, sm, 0, w, l);
+    stage_v(g, sm, w, l);
+    stage_tb_e<kUpper>(g, sm, w, l);
+    for (int c = 0; c < nch; ++c) {
+        const int next = c < last ? c + 1 : last;
+        __syncthreads();
+        const f32x4 yacc = output_project(g, sm, w, l);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_output<kUpper>(p, cx, c, w, l);
+        fetch_tb_e<kUpper>(g, cx, next, w, l);
+        fetch_k<true>(g, cx, next, w, l);
+        fetch_v<true>(g, cx, next, w, l);
+        __builtin_amdgcn_sched_barrier(0);  // the prefetches stay where they are issued
+        __syncthreads();
+        __syncthreads();
+        stage_tb_e<kUpper>(g, sm, w, l);
+        output_store<Y, kUpper>(p, yacc, sm, cx, c, y, w, l);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_q<true>(g, cx, next, w, l);
+        __builtin_amdgcn_sched_barrier(0);
+        __syncthreads();
+        stage_k(g, sm, 0, w, l);
+        stage_v(g, sm, w, l);
+    }
+}
+
+// kShared: two workgroups of the kernel share a CU.
 template <class Y, bool kF32, bool kShared>
 GDN_DEV void prefill_state_body(
     const void* __restrict__ q, const void* __restrict__ k, const void* __restrict__ v,
     const float* __restrict__ state_in, float* __restrict__ state_out,
     typename Y::storage* __restrict__ y, const RunLayout& rl, const char* __restrict__ records, int Hk,
     int Hv) {
-    __shared__ __attribute__((aligned(16))) StatePassLds<kF32> sm;
+    __shared__ __attribute__((aligned(16))) StatePassLds<kF32, kF32 && kShared ? 1 : 2> sm;
 
     // Work mapping: the 8 slices of one (run, head) share its K/Q and chunk
     // records, so they are placed on one XCD (workgroups go round-robin over
@@ -1342,7 +1383,10 @@ GDN_DEV void prefill_state_body(
             *reinterpret_cast<float4*>(state_out + sbase + dk) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
         }
     } else if (nch > 0) {
-        if constexpr (kShared) {
+        if constexpr (kShared && kF32) {
+            if (w >= 2) output_loop_one_k<Y, true>(cx, nch, sm, y, w, l);
+            else output_loop_one_k<Y, false>(cx, nch, sm, y, w, l);
+        } else if constexpr (kShared) {
             if (w >= 2) output_loop_1ahead<Y, true>(cx, nch, sm, y, w, l);
             else output_loop_1ahead<Y, false>(cx, nch, sm, y, w, l);
         } else if constexpr (kF32) {
@@ -1365,10 +1409,10 @@ __global__ __launch_bounds__(kStateThreads) void prefill_state_kernel(GDN_STATE_
     prefill_state_body<Y, kF32, false>(q, k, v, state_in, state_out, y, rl, records, Hk, Hv);
 }
 
-template <class Y>
+template <class Y, bool kF32>
 __global__ __launch_bounds__(kStateThreads) __attribute__((amdgpu_waves_per_eu(4))) void
 prefill_state_shared_kernel(GDN_STATE_ARGS) {
-    prefill_state_body<Y, false, true>(q, k, v, state_in, state_out, y, rl, records, Hk, Hv);
+    prefill_state_body<Y, kF32, true>(q, k, v, state_in, state_out, y, rl, records, Hk, Hv);
 }
 #undef GDN_STATE_ARGS
 
@@ -1377,10 +1421,7 @@ template <class Y, bool kF32>
 int launch_state(const void* q, const void* k, const void* v, const float* state_in, float* state_out, void* y,
                  const RunLayout& rl, const char* records, int Hk, int Hv, hipStream_t s, const char* what) {
     const int64_t wgs = int64_t(rl.N) * Hv * kSlices;
-    auto kernel = prefill_state_kernel<Y, kF32>;
-    if constexpr (!kF32) {
-        if (wgs > kStateSharedAbove) kernel = prefill_state_shared_kernel<Y>;
-    }
+    const auto kernel = wgs > kStateSharedAbove ? prefill_state_shared_kernel<Y, kF32> : prefill_state_kernel<Y, kF32>;
     hipLaunchKernelGGL(kernel, dim3(unsigned(wgs)), dim3(kStateThreads), 0, s, q, k, v, state_in, state_out,
                        static_cast<typename Y::storage*>(y), rl, records, Hk, Hv);
     return check_launch(what);

@@ -402,16 +402,17 @@ def test_prefill_float32_full_size_against_c_oracle(gpu):
     assert max_rel(y.cpu().numpy(), y2.cpu().numpy()) < 1e-4
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("lens", [[64, 1, 130, 63, 200, 65, 128, 320, 0], [192] * 9])
-def test_prefill_runs_sharing_a_cu_equal_each_run_alone(gpu, lens):
+def test_prefill_runs_sharing_a_cu_equal_each_run_alone(gpu, lens, dtype):
     """Above 256 state-pass workgroups (here 9 runs of 4 heads, 8 slices
     each) two of them share a CU, on a loop with shorter prefetches: the same
     bits as each run by itself, on the other loop."""
     rng = np.random.default_rng(31)
     T, Hk, Hv = sum(lens), 2, 4
-    q, k, v = (torch.tensor(rng.standard_normal((T, h, 128)) / s, dtype=torch.bfloat16, device=gpu)
+    q, k, v = (torch.tensor(rng.standard_normal((T, h, 128)) / s, dtype=dtype, device=gpu)
                for h, s in ((Hk, 11.3), (Hk, 11.3), (Hv, 1.0)))
-    a, b = (torch.tensor(rng.standard_normal((T, Hv)), dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    a, b = (torch.tensor(rng.standard_normal((T, Hv)), dtype=dtype, device=gpu) for _ in range(2))
     A_log, dt = (torch.tensor(rng.uniform(-1, 1, Hv), dtype=torch.float32, device=gpu) for _ in range(2))
     state = torch.tensor(rng.standard_normal((len(lens), Hv, 128, 128)) * 0.05, dtype=torch.float32, device=gpu)
     cu = np.concatenate([[0], np.cumsum(lens)]).tolist()
