@@ -12,7 +12,7 @@
 // no weight is rounded and no product is, which leaves the float32 sums
 // (777 rows of 2048 normal values against 12352 columns of 4-bit codes in
 // groups of 64: 1.2e-7 from float64, where the float32 library product of
-// rounded weights is 8.1e-7 off and takes 345 us to this one's 131).
+// rounded weights is 8.1e-7 off and takes 345 us to this one's 125).
 //
 // Two launches (three where K is split): the preparation cuts x, sums its
 // groups and lays s and b' out group-major; the product kernel does the rest.
@@ -152,8 +152,9 @@ GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__
 // step), the next step's pieces, codes and scales in registers meanwhile. Two
 // workgroups share a CU (256 registers a thread). At 777 rows, 2048 -> 12352,
 // the matrix cores are busy half the time (118 TFLOP of bf16 products against
-// 2.1 PFLOP/s: 58 us of 131): with two waves on a SIMD a wave's LDS reads,
-// conversions and scaling are not all covered. Fetching the codes two steps
+// 2.1 PFLOP/s: 58 us of 125): with two waves on a SIMD a wave's LDS reads,
+// conversions and scaling are not all covered. A wave in its MFMAs goes before
+// one that loads or converts (131 us without). Fetching the codes two steps
 // ahead, or the next row tile's fragments, spilled or gained nothing, and
 // codes converted by the fp8 instruction (uncentred, a third of the
 // instructions) gained 1 % at 2.5 times the error.
@@ -292,6 +293,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         fetch_w(next);
         __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
+        __builtin_amdgcn_s_setprio(1);
 #pragma unroll
         for (int a = 0; a < kTM; ++a) {
             const uint16_t* xrow = xs[(s - step0) & 1] + (16 * a + lr) * kXS;
@@ -322,6 +324,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
             }
             if constexpr (!kG32) scaled(0);
         }
+        __builtin_amdgcn_s_setprio(0);
         stage_x((s - step0 + 1) & 1);
     }
 
