@@ -160,7 +160,7 @@ def stream_ptr(device: torch.device):
 def call(name: str, *args) -> None:
     """Call an entry point and raise ``KernelError`` on a non-zero status."""
 
-    lib = load()
+    lib = _lib or load()  # bound once and never replaced
     rc = getattr(lib, name)(*args)
     if rc != 0:
         msg = lib.gdn_last_error().decode(errors="replace")

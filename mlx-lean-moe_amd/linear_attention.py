@@ -29,7 +29,7 @@ import torch
 
 from . import _lib
 from .config import LinearAttentionDims
-from .gated_delta import (PREFILL_MIN_TOKENS, _c, _check_cu_seqlens, _check_out, _require_device,
+from .gated_delta import (PREFILL_MIN_TOKENS, _as, _c, _check_cu_seqlens, _check_out, _require_device,
                           _stream, gated_delta_update)
 from .quant import (LinearWeights, QuantScheme, concat_quantized, quantized_linear,
                     quantized_linear_split)
@@ -252,6 +252,8 @@ def _rows(t: torch.Tensor) -> tuple[torch.Tensor, int]:
     width, e.g. a column slice of a stacked projection output; anything else
     is copied. Returns the tensor and its row stride in elements."""
 
+    if t.shape[0] and t.is_contiguous():
+        return t, t.numel() // t.shape[0]
     width, packed = 1, True
     for n, st in zip(reversed(t.shape[1:]), reversed(t.stride()[1:])):
         packed &= n == 1 or st == width
@@ -311,9 +313,12 @@ def fused_decode_step(qkv, z, a, b, conv_state, ssm_state, conv_weight, A_log, d
     slices of one stacked projection output); they are read in place.
     Returns ``(out (B, Hv, Dv), conv_out, state_out)``."""
 
+    # a decode step is host-bound at a few sequences, hence no conversions or
+    # tuples that change nothing below
     device = _require_device(qkv, z, a, b, conv_state, ssm_state)
     B = qkv.shape[0]
     act = qkv.dtype
+    C, Hv, Dv, K = dims.conv_dim, dims.num_value_heads, dims.value_head_dim, dims.conv_kernel_dim
     if not _fused_decode_ok(dims, act):
         raise ValueError("the fused decode kernel needs Dk = Dv = 128, K = 4 and float32 or "
                          "bfloat16 activations")
@@ -338,7 +343,6 @@ def fused_decode_step(qkv, z, a, b, conv_state, ssm_state, conv_weight, A_log, d
         conv_rows = 2 * P
         conv_out = conv_state
     if conv_arrivals is not None:
-        Hv = dims.num_value_heads
         if Hv & (Hv - 1):
             raise ValueError(f"conv_arrivals needs a power-of-two number of value heads (got {Hv})")
         if half_t is None or half_t is not conv_half:
@@ -347,12 +351,10 @@ def fused_decode_step(qkv, z, a, b, conv_state, ssm_state, conv_weight, A_log, d
                 or conv_arrivals.dtype != torch.int32 or conv_arrivals.shape != (P,)
                 or not conv_arrivals.is_contiguous()):
             raise ValueError(f"conv_arrivals must be a contiguous int32 device tensor of {P} counters")
-    if (tuple(qkv.shape) != (B, dims.conv_dim) or tuple(a.shape) != (B, dims.num_value_heads)
-            or b.shape != a.shape
-            or tuple(conv_state.shape) != (conv_rows, dims.conv_kernel_dim - 1, dims.conv_dim)
-            or tuple(ssm_state.shape) != (P, dims.num_value_heads, dims.value_head_dim,
-                                           dims.key_head_dim)
-            or (z is not None and tuple(z.shape) != (B, dims.num_value_heads, dims.value_head_dim))):
+    if (qkv.shape != (B, C) or a.shape != (B, Hv) or b.shape != a.shape
+            or conv_state.shape != (conv_rows, K - 1, C)
+            or ssm_state.shape != (P, Hv, Dv, dims.key_head_dim)
+            or (z is not None and z.shape != (B, Hv, Dv))):
         raise ValueError("fused_decode_step: inconsistent shapes")
     if conv_state.dtype != act or a.dtype != act or b.dtype != act or (z is not None and z.dtype != act):
         raise ValueError("qkv, z, a, b and conv_state must share the activation dtype")
@@ -362,27 +364,26 @@ def fused_decode_step(qkv, z, a, b, conv_state, ssm_state, conv_weight, A_log, d
     z, s_z = _rows(z) if z is not None else (None, dims.value_dim)
     conv_state = _c(conv_state)
     strides = (s_qkv, s_z, s_a, s_b)
-    dense = (dims.conv_dim, dims.value_dim, dims.num_value_heads, dims.num_value_heads)
-    row_strides = None if strides == dense else (ctypes.c_int64 * 4)(*strides)
-    conv_weight = _c(conv_weight.float().reshape(dims.conv_dim, dims.conv_kernel_dim))
-    A_log, dt_bias = _c(A_log.float()), _c(dt_bias.float())
-    norm_weight = _c(norm_weight.float()) if z is not None else None
+    row_strides = None if strides == (C, dims.value_dim, Hv, Hv) else (ctypes.c_int64 * 4)(*strides)
+    conv_weight = _as(conv_weight, torch.float32)
+    conv_weight = _c(conv_weight if conv_weight.shape == (C, K) else conv_weight.reshape(C, K))
+    A_log, dt_bias = _c(_as(A_log, torch.float32)), _c(_as(dt_bias, torch.float32))
+    norm_weight = _c(_as(norm_weight, torch.float32)) if z is not None else None
     if conv_out is None:
-        conv_out = torch.empty((B,) + tuple(conv_state.shape[1:]), dtype=act, device=device)
-    elif half_t is None and (tuple(conv_out.shape) != (B, dims.conv_kernel_dim - 1, dims.conv_dim)
-                             or conv_out.dtype != act or not conv_out.is_contiguous()):
+        conv_out = torch.empty((B, K - 1, C), dtype=act, device=device)
+    elif half_t is None and (conv_out.shape != (B, K - 1, C) or conv_out.dtype != act
+                             or not conv_out.is_contiguous()):
         raise ValueError("conv_out must be contiguous (B, K-1, C) in the activation dtype")
     if state_out is None:
         state_out = torch.empty_like(ssm_state)
     out_dtype = act if z is not None else (y_dtype or torch.float32)
-    out = torch.empty((B, dims.num_value_heads, dims.value_head_dim), dtype=out_dtype,
-                      device=device)
+    out = torch.empty((B, Hv, Dv), dtype=out_dtype, device=device)
     _lib.call("gdn_decode_step", _lib.ptr(qkv), _lib.ptr(conv_state), _lib.ptr(conv_out),
               _lib.ptr(conv_weight), _lib.ptr(a), _lib.ptr(b), _lib.ptr(A_log),
               _lib.ptr(dt_bias), _lib.ptr(ssm_state), _lib.ptr(state_out), _lib.ptr(z),
               _lib.ptr(norm_weight), float(eps), _lib.ptr(out), _lib.dtype_code(out_dtype), B,
-              dims.num_key_heads, dims.num_value_heads, dims.key_head_dim, dims.value_head_dim,
-              dims.conv_kernel_dim, _lib.dtype_code(act), _lib.ptr(slot_t), P, _lib.ptr(half_t),
+              dims.num_key_heads, Hv, dims.key_head_dim, Dv,
+              K, _lib.dtype_code(act), _lib.ptr(slot_t), P, _lib.ptr(half_t),
               row_strides, _lib.ptr(conv_arrivals), _stream(device))
     return out, conv_out, state_out
 
