@@ -41,6 +41,9 @@ _KERNEL_BITS = {4, 8}
 # once and multiplies on the vendor BLAS; below it gdn_quantized_matmul's
 # kernels run directly where _mid_rows or _dense_rows says so.
 _BLAS_ROWS = 512
+# Rows gdn_quantized_matmul_f32 takes in one call (its workspace: 1.6 GB at
+# 4096 columns of x)
+_F32_ROWS = 65536
 # quantized_linear_split multiplies per block from this many rows on (one
 # product of the stacked 2048 -> 12352 weight: 32.7 us at 512 rows against
 # 45.9 us per block, 53.9 against 62.1 at 1024, even at 2048, 246 against
@@ -81,8 +84,20 @@ def _dense_rows(rows: int, N: int, K: int) -> bool:
     return rows > 64 and (N < 4096 or K >= 4096)
 
 
-def _runs_dense(rows: int, N: int, K: int, group_size: int, sb_dtype: torch.dtype) -> bool:
-    return _dense_rows(rows, N, K) and not _mid_rows(rows, N, K, group_size, sb_dtype)
+def _runs_dense(rows: int, N: int, K: int, group_size: int, sb_dtype: torch.dtype, *operands) -> bool:
+    return _dense_rows(rows, N, K) and (not _mid_rows(rows, N, K, group_size, sb_dtype)
+                                        or _transformed(*operands))
+
+
+def _transformed(*operands: torch.Tensor | None) -> bool:
+    """Whether autograd or a function transform (vmap, forward mode) follows
+    these operands: torch's own products take part in those, the kernels'
+    calls do not, so such calls stay on the dense products."""
+
+    if torch.autograd.forward_ad._current_level >= 0:
+        return True
+    return any(t is not None and (t.requires_grad and torch.is_grad_enabled()
+                                  or torch._C._functorch.is_functorch_wrapped_tensor(t)) for t in operands)
 
 
 @dataclass(frozen=True)
@@ -259,12 +274,13 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
         return with_residual(x @ wd.to(x.dtype).T)
     x_f32 = (x.dtype == torch.float32 and rows <= 32
              and decode_kernel_takes(rows, K, quant.bits, quant.group_size, scales.dtype))
-    if x.dtype == torch.float32 and not x_f32 and f32_workspace_bytes(rows, N, K, quant.bits, quant.group_size):
+    if (x.dtype == torch.float32 and not x_f32 and not _transformed(x, residual)
+            and f32_workspace_bytes(min(rows, _F32_ROWS), N, K, quant.bits, quant.group_size)):
         return _f32_matmul(x, w, scales, biases, quant, N, K, residual)
     if x.dtype != torch.bfloat16 and not x_f32:
         return with_residual(x @ dequantize(tensors, quant, x.dtype).T)
     x2 = _c(x.reshape(-1, K))
-    if _runs_dense(x2.shape[0], N, K, quant.group_size, scales.dtype):
+    if _runs_dense(x2.shape[0], N, K, quant.group_size, scales.dtype, x, residual):
         # the same bf16-rounded weights as the tiled kernel (gdn_dequantize),
         # one transient copy, and the vendor BLAS for the GEMM itself
         wd = dense if dense is not None else dequantize(tensors, quant, torch.bfloat16)
@@ -340,11 +356,14 @@ def _f32_matmul(x, w, scales, biases, quant: QuantScheme, N: int, K: int, residu
     w, scales, biases = _c(w), _c(scales), _c(biases)
     if w.data_ptr() % 16:
         w = w.clone()
-    ws_bytes = f32_workspace_bytes(M, N, K, quant.bits, quant.group_size)
-    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
-    _lib.call("gdn_quantized_matmul_f32", _lib.ptr(x2), _lib.ptr(w), _lib.ptr(scales), _lib.ptr(biases),
-              _lib.dtype_code(scales.dtype), _lib.ptr(y), _lib.ptr(r), M, N, K, quant.bits, quant.group_size,
-              _lib.ptr(ws), ws_bytes, _lib.stream_ptr(x.device))
+    for i in range(0, M, _F32_ROWS):  # x's pieces take 6 K bytes a row of workspace
+        m = min(_F32_ROWS, M - i)
+        ws_bytes = f32_workspace_bytes(m, N, K, quant.bits, quant.group_size)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+        _lib.call("gdn_quantized_matmul_f32", _lib.ptr(x2[i:i + m]), _lib.ptr(w), _lib.ptr(scales),
+                  _lib.ptr(biases), _lib.dtype_code(scales.dtype), _lib.ptr(y[i:i + m]),
+                  _lib.ptr(None if r is None else r[i:i + m]), m, N, K, quant.bits,
+                  quant.group_size, _lib.ptr(ws), ws_bytes, _lib.stream_ptr(x.device))
     return y.reshape(*lead, N)
 
 
@@ -371,7 +390,7 @@ def quantized_linear_split(x: torch.Tensor, weights: LinearWeights, sizes) -> li
     K = x.shape[-1]
     rows = x.reshape(-1, K).shape[0]
     if (x.dtype == torch.bfloat16 and x.device.type == "cuda"
-            and (_runs_dense(rows, tensors["weight"].shape[0], K, quant.group_size, tensors["scales"].dtype)
+            and (_runs_dense(rows, tensors["weight"].shape[0], K, quant.group_size, tensors["scales"].dtype, x)
                  or not (_on_kernels(quant) or _scheme_kernel_takes(x, rows, K, quant)))):
         _check_quantized(tensors, quant, K)
         lead = x.shape[:-1]

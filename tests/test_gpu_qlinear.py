@@ -674,3 +674,29 @@ def test_dequantize_into_any_alignment(gpu, mode, bits, gs, out, shift):
     got = buf.float().cpu().numpy()
     np.testing.assert_array_equal(got[shift:shift + N * K].reshape(N, K), ref)
     assert (got[:shift] == 7).all() and (got[shift + N * K:] == 7).all()
+
+
+def test_products_under_transforms_stay_on_torch(gpu):
+    """float32 rows and narrow bf16 products that are differentiated, run
+    under vmap or carry a tangent give what torch's product of the
+    dequantized weights gives there, as calls the kernels do not see."""
+    rng = np.random.default_rng(9)
+    words, s, b = _weights(rng, 48, 256, 4, 64, "bf16")
+    W = _dev_weights(gpu, words, s, b, "bf16")
+    scheme = gdn.QuantScheme(4, 64)
+    for dtype in (torch.float32, torch.bfloat16):
+        dense = gdn.dequantize(W, scheme, dtype)
+        x = torch.tensor(rng.standard_normal((100, 256)), dtype=dtype, device=gpu)
+        xg = x.clone().requires_grad_()
+        gdn.quantized_linear(xg, W, scheme).float().sum().backward()
+        want = dense.float().sum(0).expand(100, 256)
+        assert (xg.grad.float() - want).abs().max() <= (2 ** -7 if dtype is torch.bfloat16 else 1e-5) * want.abs().max()
+        with torch.no_grad():
+            assert gdn.quantized_linear(xg, W, scheme).grad_fn is None
+        with torch.autograd.forward_ad.dual_level():
+            y = gdn.quantized_linear(torch.autograd.forward_ad.make_dual(x, x), W, scheme)
+            assert torch.equal(torch.autograd.forward_ad.unpack_dual(y).tangent, x @ dense.T)
+    x = torch.tensor(rng.standard_normal((3, 40, 256)), dtype=torch.float32, device=gpu)
+    got = torch.vmap(lambda r: gdn.quantized_linear(r, W, scheme))(x)
+    ref = x @ gdn.dequantize(W, scheme, torch.float32).T
+    assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
