@@ -304,8 +304,8 @@ int gdn_gated_rmsnorm(const void *x, int x_dtype, const void *z, int z_dtype, in
  *      it splits less or not at all. 17-64 rows of bf16 x against 4-bit
  *      codes in 64-k slices with few column tiles (out_proj's shape) run
  *      instead as 16-row blocks in one launch and take no workspace (its
- *      size is 0 there). Above 64 rows gdn_quantized_matmul_rows_workspace_size
- *      gives the bytes of the full split instead (the size function below
+ *      size is 0 there). From 65 to 511 rows
+ *      gdn_quantized_matmul_rows_workspace_size gives the bytes of the full split instead (the size function below
  *      is of the decode kernel's calls). Calls sharing a workspace must not
  *      overlap.
  * Replaces mx.quantized_matmul(..., mode="affine") in quantized_linear
@@ -377,8 +377,8 @@ int64_t gdn_quantized_matmul_f32_workspace_size(int M, int N, int K, int bits, i
 
 /*
  * gdn_quantized_matmul_rows_workspace_size - workspace bytes
- * gdn_quantized_matmul splits K with for M > 64 bf16 rows (0: it does not; a
- * call without a workspace keeps K whole).
+ * gdn_quantized_matmul splits K with for 65 to 511 bf16 rows (0: it does not;
+ * a call without a workspace keeps K whole).
  */
 int64_t gdn_quantized_matmul_rows_workspace_size(int sb_dtype, int M, int N, int K, int bits,
                                                  int group_size);

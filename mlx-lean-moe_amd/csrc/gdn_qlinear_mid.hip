@@ -19,6 +19,7 @@ constexpr int kSlice = 64;           // a wave's k of a step
 constexpr int kStep = kSlice * kKW;  // k of a step
 constexpr int kXS = kStep + 8;       // row stride of the x tile: 16 rows cover the banks
 constexpr int kMaxTM = 7;
+constexpr int kMaxRows = 511;
 // Bytes of scales and biases the LDS holds (of a workgroup's columns over its k range)
 constexpr int kSBBytes = 32 * 1024;
 constexpr int kCUs = 256;
@@ -315,10 +316,13 @@ int launch_mid_sb(const MidArgs& a, int sb_dtype, int y_dtype, MidPlan p) {
 
 }  // namespace
 
-// 32-bit byte offsets inside a tile bound K; the scales of a k range have to
-// fit the LDS (ws_bytes: the workspace a split may use).
+// Up to kMaxRows rows: with more of them than workgroups want, the 128 x 128
+// tiles read x less often (2048 -> 12352 at 4096 rows 352 us there, 397 here,
+// even at 2048; 1024 -> 12352 at 600 rows 36 and 46). 32-bit byte offsets
+// inside a tile bound K; the scales of a k range have to fit the LDS
+// (ws_bytes: the workspace a split may use).
 bool mid_kernel_takes(int M, int N, int K, int group_size, int sb_dtype, int64_t ws_bytes) {
-    return M > 64 && N > 0 && K > 0 && K % kStep == 0 && K % group_size == 0 && K <= (1 << 20) &&
+    return M > 64 && M <= kMaxRows && N > 0 && K > 0 && K % kStep == 0 && K % group_size == 0 && K <= (1 << 20) &&
            mid_plan(M, N, K, group_size, sb_dtype, ws_bytes).tm > 0;
 }
 
