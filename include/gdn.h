@@ -322,8 +322,9 @@ int gdn_quantized_matmul(const void *x, int x_dtype, const void *w, const void *
  * and takes no workspace: a call that splits K keeps its float32 partial
  * products in the library's own device scratch (a static 4 MiB array per
  * GPU, held until the process ends; every call the decode kernel takes
- * needs at most that), so it splits exactly as gdn_quantized_matmul does
- * with a full workspace and gives the same bits. A call needing more
+ * needs at most that), so up to 64 rows it splits exactly as
+ * gdn_quantized_matmul does with a full workspace and gives the same bits
+ * (above, as without a workspace). A call needing more
  * returns GDN_EINVAL. The first call on a GPU looks up that GPU's copy of
  * the array (hipGetSymbolAddress, which may load the library's code object
  * there): make that first call eagerly, before capturing calls into a HIP

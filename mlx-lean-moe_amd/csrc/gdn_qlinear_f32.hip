@@ -12,7 +12,7 @@
 // no weight is rounded and no product is, which leaves the float32 sums
 // (777 rows of 2048 normal values against 12352 columns of 4-bit codes in
 // groups of 64: 1.2e-7 from float64, where the float32 library product of
-// rounded weights is 8.1e-7 off and takes 345 us to this one's 125).
+// rounded weights is 8.1e-7 off and takes 345 us to this one's 125-129).
 //
 // Two launches (three where K is split): the preparation cuts x, sums its
 // groups and lays s and b' out group-major; the product kernel does the rest.
@@ -45,23 +45,32 @@ GDN_DEV f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 // not, or a row of magnitudes whose last piece leaves bf16's range. They are
 // multiplied apart (slow_row).
 constexpr float kRowMax = 0x1p100f, kRowMin = 0x1p-90f;
+// Columns whose scales or biases are not finite or so large that a group's
+// scaled sum could overflow are multiplied apart too (flags of 64 columns).
+constexpr float kScaleMax = 0x1p16f, kBiasMax = 0x1p24f;
+constexpr int kFlagCols = 64;
 
 // Blocks 0 .. M - 1: row m of x as bf16 pieces, pieces[m][step][part][64]
 // (part 0 the upper 8 significant bits; truncation, so no piece can round up
 // to infinity), its group sums (in double, rounded once) and its flag. The
-// blocks after them: s and b' = b + centre s in float32, group-major.
+// blocks after them, 64 columns each: s and b' = b + centre s in float32,
+// group-major, and the columns' flag (at flags[M + block]).
 __global__ __launch_bounds__(256) void prepare_f32_kernel(
     const float* __restrict__ x, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
     uint16_t* __restrict__ pieces, float* __restrict__ xsum, int* __restrict__ flags, float* __restrict__ s_t,
     float* __restrict__ b_t, int M, int N, int K, int group_size, float centre) {
     const int G = K / group_size;
     if (int(blockIdx.x) >= M) {
-        const int64_t i = int64_t(int(blockIdx.x) - M) * 256 + threadIdx.x;  // (g, n), n fastest
-        if (i >= int64_t(N) * G) return;
-        const int64_t g = i / N, n = i % N;
-        const float s = load_any(scales, n * G + g, sb_dtype), b = load_any(biases, n * G + g, sb_dtype);
-        s_t[i] = s;
-        b_t[i] = __builtin_fmaf(centre, s, b);
+        const int64_t n = int64_t(int(blockIdx.x) - M) * kFlagCols + (threadIdx.x & 63);
+        bool far = false;
+        for (int g = threadIdx.x >> 6; g < G && n < N; g += 4) {
+            const float s = load_any(scales, n * G + g, sb_dtype), b = load_any(biases, n * G + g, sb_dtype);
+            far |= !(fabsf(s) < kScaleMax && fabsf(b) < kBiasMax);
+            s_t[int64_t(g) * N + n] = s;
+            b_t[int64_t(g) * N + n] = __builtin_fmaf(centre, s, b);
+        }
+        far = __syncthreads_or(far);
+        if (threadIdx.x == 0) flags[blockIdx.x] = far;
         return;
     }
     const int64_t m = blockIdx.x;
@@ -328,16 +337,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
         stage_x((s - step0 + 1) & 1);
     }
 
+    // flagged rows, and the wave's own 64 columns when flagged, are left to
+    // the loop below
+    static_assert(kFlagCols == 16 * kTN, "a wave's columns share a flag");
+    const int cols = (N + kFlagCols - 1) / kFlagCols, col0 = n0 / kFlagCols;
     int any = 0;
     if (tid < kBM) any = flags[m0 + tid < M ? m0 + tid : M - 1];
+    if (tid < kBN / kFlagCols && col0 + tid < cols) any |= flags[M + col0 + tid];
     any = __syncthreads_or(any);
+    const int far = any && col0 + wv < cols ? flags[M + col0 + wv] : 0;
     float* dst = out + int64_t(blockIdx.y) * M * N;
 #pragma unroll
     for (int a = 0; a < kTM; ++a)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int m = m0 + 16 * a + 4 * lq + i;
-            if (m >= M || (any && flags[m])) continue;
+            if (m >= M || far || (any && flags[m])) continue;
 #pragma unroll
             for (int b = 0; b < kTN; ++b) {
                 const int n = n0 + 16 * kTN * wv + 16 * b + lr;
@@ -346,9 +361,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
                 dst[e] = acc[a][b][i] + (residual ? residual[e] : 0.f);
             }
         }
-    if (any && n0 + tid < N) {
+    if (any && n0 + tid < N) {  // thread tid's column lies in its own wave's 64
         for (int r = 0; r < kBM && m0 + r < M; ++r) {
-            if (!flags[m0 + r]) continue;
+            if (!far && !flags[m0 + r]) continue;
             const int64_t m = m0 + r, n = n0 + tid, e = m * N + n;
             const float v = blockIdx.y == 0 ? slow_row<kBits>(x + m * K, w, scales, biases, sb_dtype, n, K, group_size) : 0.f;
             dst[e] = v + (residual ? residual[e] : 0.f);
@@ -388,7 +403,7 @@ F32Plan plan_f32(int M, int N, int K, int group_size) {
     const int64_t G = K / group_size;
     p.xsum = up(int64_t(M) * K * kParts * 2);
     p.flags = p.xsum + up(M * G * 4);
-    p.s_t = p.flags + up(int64_t(M) * 4);
+    p.s_t = p.flags + up((int64_t(M) + (N + kFlagCols - 1) / kFlagCols) * 4);
     p.b_t = p.s_t + up(N * G * 4);
     p.partial = p.b_t + up(N * G * 4);
     p.bytes = p.partial + (p.splits > 1 ? int64_t(p.splits) * M * N * 4 : 0);
@@ -451,7 +466,7 @@ extern "C" int gdn_quantized_matmul_f32(const float* x, const void* w, const voi
     auto* s_t = reinterpret_cast<float*>(ws + p.s_t);
     auto* b_t = reinterpret_cast<float*>(ws + p.b_t);
     auto* partial = reinterpret_cast<float*>(ws + p.partial);
-    const int64_t sb_blocks = (int64_t(N) * (K / group_size) + 255) / 256;
+    const int64_t sb_blocks = (int64_t(N) + kFlagCols - 1) / kFlagCols;
     hipLaunchKernelGGL(prepare_f32_kernel, dim3(unsigned(M + sb_blocks)), dim3(256), 0, s, x, scales, biases, sb_dtype,
                        pieces, xsum, flags, s_t, b_t, M, N, K, group_size, bits == 4 ? 8.f : 128.f);
     if (int rc = check_launch("gdn_quantized_matmul_f32/prepare")) return rc;

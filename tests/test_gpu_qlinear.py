@@ -700,3 +700,27 @@ def test_products_under_transforms_stay_on_torch(gpu):
     got = torch.vmap(lambda r: gdn.quantized_linear(r, W, scheme))(x)
     ref = x @ gdn.dequantize(W, scheme, torch.float32).T
     assert (got - ref).abs().max() <= 1e-5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("N,K", [(300, 512), (256, 4096)])
+def test_float32_rows_times_scales_out_of_range(gpu, N, K):
+    """Infinite, NaN and huge float32 scales and biases reach exactly the
+    columns they belong to, with the infinities and NaN of the float32
+    weights."""
+    rng = np.random.default_rng(N + 1)
+    words, s, b = _weights(rng, N, K, 4, 64, "f32")
+    s, b = np.array(s, np.float32), np.array(b, np.float32)
+    s[3, 1], s[70, 0], b[100, 2], s[N - 1, 0], b[N - 1, 0] = np.inf, np.nan, -np.inf, 1e30, 1e30
+    W = _dev_weights(gpu, words, s, b, "f32")
+    x = rng.standard_normal((70, K)).astype(np.float32)
+    q = Q.unpack(words, 4).astype(np.float64)
+    with np.errstate(all="ignore"):
+        w = (np.repeat(s, 64, 1).astype(np.float64) * q + np.repeat(b, 64, 1)).astype(np.float32).astype(np.float64)
+        ref = x.astype(np.float64) @ w.T
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
+    np.testing.assert_array_equal(np.isposinf(y), np.isposinf(ref))
+    np.testing.assert_array_equal(np.isneginf(y), np.isneginf(ref))
+    ok = np.isfinite(w).all(axis=1)
+    mass = np.abs(x).astype(np.float64) @ np.abs(w[ok]).T
+    assert (np.abs(y[:, ok] - ref[:, ok]) <= 2 * K * 2.0 ** -24 * mass).all()
