@@ -318,12 +318,23 @@ int launch_mid_sb(const MidArgs& a, int sb_dtype, int y_dtype, MidPlan p) {
 
 // Up to kMaxRows rows: with more of them than workgroups want, the 128 x 128
 // tiles read x less often (2048 -> 12352 at 4096 rows 352 us there, 397 here,
-// even at 2048; 1024 -> 12352 at 600 rows 36 and 46). 32-bit byte offsets
-// inside a tile bound K; the scales of a k range have to fit the LDS
-// (ws_bytes: the workspace a split may use).
+// even at 2048; 1024 -> 12352 at 600 rows 36 and 46). The same where this
+// kernel's workgroups, one a CU, need a second round and the 128 x 128 tiles,
+// two a CU, one: at 256 rows of 12352 columns (291 and 194 of them) K = 256
+// takes 16 us here and 12 there, 1024 27 and 25 (groups of 32: 29 and 26),
+// 2048 45 and 44 (53 and 45), 4096 79 and 81. And where both need two but the
+// work of a round is short: K = 512, 384 rows 22.0 and 21.3, 511 rows 26.1 and
+// 22.0; K = 1024, 384 rows 29.6 and 33.8, 511 rows, five row tiles to four,
+// 34.7 and 34.5 (8-bit 38.1 and 33.6). 32-bit byte offsets inside a tile bound
+// K; the scales of a k range have to fit the LDS (ws_bytes: the workspace a
+// split may use).
 bool mid_kernel_takes(int M, int N, int K, int group_size, int sb_dtype, int64_t ws_bytes) {
-    return M > 64 && M <= kMaxRows && N > 0 && K > 0 && K % kStep == 0 && K % group_size == 0 && K <= (1 << 20) &&
-           mid_plan(M, N, K, group_size, sb_dtype, ws_bytes).tm > 0;
+    if (M <= 64 || M > kMaxRows || N < 1 || K < 1 || K % kStep || K % group_size || K > (1 << 20)) return false;
+    const MidPlan p = mid_plan(M, N, K, group_size, sb_dtype, ws_bytes);
+    if (p.tm == 0) return false;
+    const int64_t wgs = (int64_t(M) + 16 * p.tm - 1) / (16 * p.tm) * ((int64_t(N) + kBN - 1) / kBN);
+    const int64_t tiled = (int64_t(M) + 127) / 128 * ((int64_t(N) + 127) / 128);
+    return p.splits > 1 || wgs <= kCUs || (tiled > kCUs && K >= 1024 && (K > 1024 || M <= 448));
 }
 
 int64_t mid_workspace_bytes(int M, int N, int K, int group_size, int sb_dtype) {
