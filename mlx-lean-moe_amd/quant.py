@@ -38,9 +38,11 @@ _MODES = {"affine": 0, "mxfp4": 1, "mxfp8": 2, "nvfp4": 3}
 # dequantize, then multiply on the vendor BLAS)
 _KERNEL_BITS = {4, 8}
 # From this many rows on, quantized_linear dequantizes the weights to bf16
-# once and multiplies on the vendor BLAS; below it gdn_quantized_matmul's
-# kernels run directly where _mid_rows or _dense_rows says so.
+# once and multiplies on the vendor BLAS; below it see _runs_dense.
 _BLAS_ROWS = 512
+# Largest tile of gdn_quantized_matmul's kernel for 65-511 rows (gdn_qlinear_mid.hip)
+_MID_TILE_ROWS, _MID_TILE_COLUMNS = 112, 128
+_CUS = 256
 # Rows gdn_quantized_matmul_f32 takes in one call (its workspace: 1.6 GB at
 # 4096 columns of x)
 _F32_ROWS = 65536
@@ -52,41 +54,59 @@ _SPLIT_ROWS = 2048
 
 
 def _mid_rows(rows: int, N: int, K: int, group_size: int, sb_dtype: torch.dtype) -> bool:
-    """Whether more than 64 bf16 rows run on gdn_quantized_matmul's kernel for
-    them (gdn_qlinear_mid.hip), which takes K in steps of 256 with a k range's
-    scales and biases of 128 columns in 32 KB of LDS, rather than on
-    dequantized weights and the vendor BLAS (which read the codes once more as
-    bf16, but keep the larger tiles busy). Device time from graphs, kernel
-    against dense, us: 2048 -> 12352 at 66 rows 21 and 35, 200 rows 28 and 43,
-    256 rows 40 and 43, 384 rows 47 and 46, 512 rows 55 and 52; 4096 -> 12352
-    at 200 rows 47 and 60; 1024 -> 12352 at 500 rows 36 and 41; 4096 -> 2048 at
-    128 rows 17 and 24, 384 rows 26 and 29, 600 rows 36 and 27; 2048 -> 2048 at
-    350 rows 22 and 19. Up to 224 rows the largest of these is one workgroup a
-    CU."""
+    """Whether gdn_quantized_matmul's kernel for 65 to 511 bf16 rows
+    (gdn_qlinear_mid.hip) takes the shape with K whole: K in steps of 256, the
+    scales and biases of 128 columns in 32 KB of LDS."""
 
-    if rows <= 64 or K % 256 or K // group_size * 256 * sb_dtype.itemsize > 32768:
-        return False
-    if N * K > 26_000_000 or (N < 4096 and K < 4096):
-        return rows <= 224
-    return rows <= (384 if K >= 2048 else _BLAS_ROWS - 1)
+    return (64 < rows < _BLAS_ROWS and K % 256 == 0
+            and K // group_size * 256 * sb_dtype.itemsize <= 32768)
 
 
 def _dense_rows(rows: int, N: int, K: int) -> bool:
     """Whether ``rows`` bf16 rows times a quantized ``(N, K)`` weight that
-    _mid_rows leaves run on dequantized weights and the vendor BLAS rather
-    than the tiled kernel. That one takes 128 x 128 tiles with no K split, so
-    a narrow or deep weight leaves the GPU idle: for 4096 -> 2048 (out_proj)
-    it takes 73-76 us from 65 to 1024 rows against 23-34 us dense; for 2048 ->
-    12352 it is even around 300 rows."""
+    _mid_rows does not take run on dequantized weights and the vendor BLAS
+    rather than the tiled kernel. That one takes 128 x 128 tiles with no K
+    split, so a narrow or deep weight leaves the GPU idle: for 4096 -> 2048
+    (out_proj) it takes 73-76 us from 65 to 1024 rows against 23-36 us dense;
+    for 2048 -> 12352 it is even at 256 rows (44 and 43)."""
 
     if rows >= _BLAS_ROWS:
         return True
     return rows > 64 and (N < 4096 or K >= 4096)
 
 
-def _runs_dense(rows: int, N: int, K: int, group_size: int, sb_dtype: torch.dtype, *operands) -> bool:
-    return _dense_rows(rows, N, K) and (not _mid_rows(rows, N, K, group_size, sb_dtype)
-                                        or _transformed(*operands))
+def _runs_dense(rows: int, N: int, K: int, quant: QuantScheme, sb_dtype: torch.dtype, *operands) -> bool:
+    """Whether ``rows`` bf16 rows times 4- or 8-bit affine ``(N, K)`` weights
+    run on dequantized weights and the vendor BLAS rather than on
+    gdn_quantized_matmul. Where the kernel for 65-511 rows takes the shape,
+    device time from graphs decides (us, 4-bit groups of 64, weights not in a
+    cache, kernel against dense):
+
+    - small weights, to 2^20: even (10 to 14 us both ways), dense.
+    - K split over the grid: kernel (4096 -> 2048 at 66 rows 15 and 23, 448
+      rows 26 and 31; 4096 -> 4096 at 224 rows 28 and 34).
+    - unsplit, N < 4096: a few workgroups walk all of K; dense (2048 -> 2048
+      at 200 rows 21 and 17, 4096 -> 2048 at 511 rows 35 and 30; even for 1024
+      -> 2048, and at N = 4096: 4096 -> 4096 at 256 rows 35 and 35).
+    - K < 2048: kernel (1024 -> 12352 at 200 rows 19 and 32, 511 rows 35 and
+      39).
+    - else kernel while its workgroups fit the CUs in one round (2048 -> 12352
+      at 224 rows 31 and 41, 256 rows 45 and 43, 384 rows 49 and 45, 511 rows
+      57 and 51; 3072 -> 12352 at 224 rows 40 and 53, 256 rows 59 and 55, 511
+      rows 74 and 65; 4096 -> 12352 at 224 rows 51 and 67, 256 rows 79 and 68;
+      2048 -> 8192 at 448 rows 29 and 38, 511 rows 43 and 38)."""
+
+    dense = _dense_rows(rows, N, K)
+    if not _mid_rows(rows, N, K, quant.group_size, sb_dtype) or (dense and _transformed(*operands)):
+        return dense
+    if N * K <= 1 << 20:
+        return dense
+    if workspace_bytes(torch.bfloat16, sb_dtype, rows, N, K, quant.bits, quant.group_size):
+        return False
+    if N < 4096:
+        return True
+    tiles = -(-rows // _MID_TILE_ROWS) * -(-N // _MID_TILE_COLUMNS)
+    return K >= 2048 and tiles > _CUS
 
 
 def _transformed(*operands: torch.Tensor | None) -> bool:
@@ -280,7 +300,7 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
     if x.dtype != torch.bfloat16 and not x_f32:
         return with_residual(x @ dequantize(tensors, quant, x.dtype).T)
     x2 = _c(x.reshape(-1, K))
-    if _runs_dense(x2.shape[0], N, K, quant.group_size, scales.dtype, x, residual):
+    if _runs_dense(x2.shape[0], N, K, quant, scales.dtype, x, residual):
         # the same bf16-rounded weights as the tiled kernel (gdn_dequantize),
         # one transient copy, and the vendor BLAS for the GEMM itself
         wd = dense if dense is not None else dequantize(tensors, quant, torch.bfloat16)
@@ -390,7 +410,7 @@ def quantized_linear_split(x: torch.Tensor, weights: LinearWeights, sizes) -> li
     K = x.shape[-1]
     rows = x.reshape(-1, K).shape[0]
     if (x.dtype == torch.bfloat16 and x.device.type == "cuda"
-            and (_runs_dense(rows, tensors["weight"].shape[0], K, quant.group_size, tensors["scales"].dtype, x)
+            and (_on_kernels(quant) and _runs_dense(rows, tensors["weight"].shape[0], K, quant, tensors["scales"].dtype, x)
                  or not (_on_kernels(quant) or _scheme_kernel_takes(x, rows, K, quant)))):
         _check_quantized(tensors, quant, K)
         lead = x.shape[:-1]

@@ -166,6 +166,29 @@ def test_dense_path_choice_follows_the_measured_crossovers():
     assert _dense_rows(100, 300, 512)            # narrow weights
 
 
+@pytest.mark.parametrize("N,K,kernel,dense", [
+    (12352, 2048, (64, 65, 224), (225, 384, 511, 512)),   # stacked input projection: one round of workgroups
+    (12352, 3072, (65, 224), (225, 300, 511)),
+    (12352, 4096, (65, 224), (225, 511)),
+    (12352, 1024, (65, 256, 511), (512,)),
+    (8192, 2048, (448,), (449,)),
+    (2048, 4096, (65, 200, 448), (511,)),                 # out_proj: while K is split
+    (2048, 2048, (65, 112), (160, 200, 224, 511)),
+    (2048, 1024, (64,), (65, 224, 511)),
+    (256, 4096, (64,), (65, 511)),                        # small weights
+    (12352, 2880, (65, 511), (512,)),                     # K not in steps of 256: the tiled kernel
+    (2048, 2880, (64,), (65, 511)),
+])
+def test_bf16_projections_run_where_they_measured_faster(N, K, kernel, dense):
+    """The route of every row count is _runs_dense's alone: nothing behind it
+    takes a call back."""
+    from mlx_lean_moe_amd.quant import QuantScheme, _runs_dense
+
+    q = QuantScheme(4, 64)
+    for rows in (*kernel, *dense):
+        assert _runs_dense(rows, N, K, q, torch.bfloat16) == (rows in dense), rows
+
+
 def test_pool_host_bookkeeping_flips_bits_and_sizes():
     """The pool's host copies of the half bits and sizes (NumPy views of its
     torch tensors): a decode of some slots flips exactly their bits and adds
