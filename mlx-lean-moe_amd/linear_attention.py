@@ -447,7 +447,10 @@ class Qwen3_5LinearAttention:
         stacked input one and out_proj) next to them: prompt-sized calls then
         skip converting the weights each time (23 us of a 512-token chunk at
         hidden 2048), for 2 bytes per weight of memory. Results are
-        unchanged; decode-sized calls do not use the copies."""
+        unchanged, bit for bit where the call without copies converts the
+        weights too, and up to the order of the float32 sums where it runs on
+        a quantized kernel (out_proj at 65 to 448 rows); decode-sized calls do
+        not use the copies."""
 
         if self._in_stacked is not None and self._in_stacked.dense is None:
             self._in_stacked = self._in_stacked.with_dense()

@@ -75,7 +75,8 @@ def _dense_rows(rows: int, N: int, K: int) -> bool:
     return rows > 64 and (N < 4096 or K >= 4096)
 
 
-def _runs_dense(rows: int, N: int, K: int, quant: QuantScheme, sb_dtype: torch.dtype, *operands) -> bool:
+def _runs_dense(rows: int, N: int, K: int, quant: QuantScheme, sb_dtype: torch.dtype, *operands,
+                kept: bool = False) -> bool:
     """Whether ``rows`` bf16 rows times 4- or 8-bit affine ``(N, K)`` weights
     run on dequantized weights and the vendor BLAS rather than on
     gdn_quantized_matmul. Where the kernel for 65-511 rows takes the shape,
@@ -94,10 +95,15 @@ def _runs_dense(rows: int, N: int, K: int, quant: QuantScheme, sb_dtype: torch.d
       at 224 rows 31 and 41, 256 rows 45 and 43, 384 rows 49 and 45, 511 rows
       57 and 51; 3072 -> 12352 at 224 rows 40 and 53, 256 rows 59 and 55, 511
       rows 74 and 65; 4096 -> 12352 at 224 rows 51 and 67, 256 rows 79 and 68;
-      2048 -> 8192 at 448 rows 29 and 38, 511 rows 43 and 38)."""
+      2048 -> 8192 at 448 rows 29 and 38, 511 rows 43 and 38).
+
+    ``kept``: a bf16 copy of the weights is at hand. The library's product
+    alone is then faster than the kernel wherever _dense_rows holds (copy
+    against kernel, us: 4096 -> 2048 at 66 rows 10 and 15, 200 rows 14 and 20,
+    384 rows 18 and 26; 4096 -> 12352 at 200 rows 42 and 51)."""
 
     dense = _dense_rows(rows, N, K)
-    if not _mid_rows(rows, N, K, quant.group_size, sb_dtype) or (dense and _transformed(*operands)):
+    if not _mid_rows(rows, N, K, quant.group_size, sb_dtype) or (dense and (kept or _transformed(*operands))):
         return dense
     if N * K <= 1 << 20:
         return dense
@@ -149,7 +155,10 @@ class LinearWeights:
     dequantization (``dequantize(tensors, quant, bfloat16)``, see
     :meth:`with_dense`): the prefill-sized products, which multiply on
     exactly those values, then skip converting the weights on every call, at
-    the cost of keeping the copy (2 bytes per weight)."""
+    the cost of keeping the copy (2 bytes per weight). Where without a copy
+    65 to 511 rows of a narrow or deep weight run on a quantized kernel, they
+    run on the copy too: the same bf16 weights and float32 sums, in the
+    library's order."""
 
     tensors: object
     quant: QuantScheme | None
@@ -300,7 +309,7 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
     if x.dtype != torch.bfloat16 and not x_f32:
         return with_residual(x @ dequantize(tensors, quant, x.dtype).T)
     x2 = _c(x.reshape(-1, K))
-    if _runs_dense(x2.shape[0], N, K, quant, scales.dtype, x, residual):
+    if _runs_dense(x2.shape[0], N, K, quant, scales.dtype, x, residual, kept=dense is not None):
         # the same bf16-rounded weights as the tiled kernel (gdn_dequantize),
         # one transient copy, and the vendor BLAS for the GEMM itself
         wd = dense if dense is not None else dequantize(tensors, quant, torch.bfloat16)
@@ -410,7 +419,8 @@ def quantized_linear_split(x: torch.Tensor, weights: LinearWeights, sizes) -> li
     K = x.shape[-1]
     rows = x.reshape(-1, K).shape[0]
     if (x.dtype == torch.bfloat16 and x.device.type == "cuda"
-            and (_on_kernels(quant) and _runs_dense(rows, tensors["weight"].shape[0], K, quant, tensors["scales"].dtype, x)
+            and (_on_kernels(quant) and _runs_dense(rows, tensors["weight"].shape[0], K, quant, tensors["scales"].dtype, x,
+                                                    kept=weights.dense is not None)
                  or not (_on_kernels(quant) or _scheme_kernel_takes(x, rows, K, quant)))):
         _check_quantized(tensors, quant, K)
         lead = x.shape[:-1]

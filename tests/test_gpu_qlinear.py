@@ -724,3 +724,27 @@ def test_float32_rows_times_scales_out_of_range(gpu, N, K):
     ok = np.isfinite(w).all(axis=1)
     mass = np.abs(x).astype(np.float64) @ np.abs(w[ok]).T
     assert (np.abs(y[:, ok] - ref[:, ok]) <= 2 * K * 2.0 ** -24 * mass).all()
+
+
+@pytest.mark.parametrize("rows", [65, 128, 224, 384, 448])
+@pytest.mark.parametrize("N,K", [(2048, 4096), (4096, 4096), (12352, 4096)])
+def test_kept_copies_are_multiplied_above_the_decode_sizes(gpu, rows, N, K, monkeypatch):
+    """Narrow or deep weights whose bf16 copy is kept: no call reads the codes
+    above 64 rows, and the result is the library's product of the copy."""
+    rng = np.random.default_rng(rows)
+    scheme = gdn.QuantScheme(4, 64)
+    W = {"weight": torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), dtype=torch.int32, device=gpu),
+         "scales": torch.full((N, K // 64), 0.01, dtype=torch.bfloat16, device=gpu),
+         "biases": torch.full((N, K // 64), -0.08, dtype=torch.bfloat16, device=gpu)}
+    kept = gdn.LinearWeights(W, scheme).with_dense()
+    x = torch.tensor(rng.standard_normal((rows, K)), dtype=torch.float32, device=gpu).to(torch.bfloat16)
+    with monkeypatch.context() as m:
+        m.setattr(_lib, "call", lambda name, *a: pytest.fail(f"{name} called"))
+        y = gdn.quantized_linear(x, kept)
+        blocks = quantized_linear_split(x, kept, [N - 64, 64])
+    assert torch.equal(y, x @ kept.dense.T)
+    assert torch.equal(torch.cat(blocks, dim=-1), y)
+    # the codes' result: the same weights in float32 sums of another order
+    plain = gdn.quantized_linear(x, W, scheme).double()
+    mass = x.double().abs() @ kept.dense.double().abs().T
+    assert ((y.double() - plain).abs() <= 2.0 ** -8 * plain.abs() + 2 * (K + 20) * 2.0 ** -24 * mass).all()
