@@ -55,7 +55,8 @@ typedef enum {
  * gdn_quantized_matmul_scheme and its workspace size, 16 conv_arrivals as
  * counters whose bit 16 is a parity of the half bit, 17
  * gdn_quantized_matmul_f32, its workspace size and
- * gdn_quantized_matmul_rows_workspace_size). */
+ * gdn_quantized_matmul_rows_workspace_size, 18 gdn_quantized_matmul_rows, which
+ * alone uses that workspace). */
 int gdn_abi_version(void);
 
 /* Message describing the calling thread's last non-zero return. */
@@ -304,10 +305,9 @@ int gdn_gated_rmsnorm(const void *x, int x_dtype, const void *z, int z_dtype, in
  *      it splits less or not at all. 17-64 rows of bf16 x against 4-bit
  *      codes in 64-k slices with few column tiles (out_proj's shape) run
  *      instead as 16-row blocks in one launch and take no workspace (its
- *      size is 0 there). From 65 to 511 rows
- *      gdn_quantized_matmul_rows_workspace_size gives the bytes of the full split instead (the size function below
- *      is of the decode kernel's calls). Calls sharing a workspace must not
- *      overlap.
+ *      size is 0 there). Above 64 rows K is not split, whatever the
+ *      workspace (gdn_quantized_matmul_rows does). Calls sharing a workspace
+ *      must not overlap.
  * Replaces mx.quantized_matmul(..., mode="affine") in quantized_linear
  * (model/moe_block.py:44-55), used for the layer's projections
  * (model/qwen3_5/linear_attention.py:96-101,125).
@@ -322,9 +322,8 @@ int gdn_quantized_matmul(const void *x, int x_dtype, const void *w, const void *
  * and takes no workspace: a call that splits K keeps its float32 partial
  * products in the library's own device scratch (a static 4 MiB array per
  * GPU, held until the process ends; every call the decode kernel takes
- * needs at most that), so up to 64 rows it splits exactly as
- * gdn_quantized_matmul does with a full workspace and gives the same bits
- * (above, as without a workspace). A call needing more
+ * needs at most that), so it splits exactly as gdn_quantized_matmul does
+ * with a full workspace and gives the same bits. A call needing more
  * returns GDN_EINVAL. The first call on a GPU looks up that GPU's copy of
  * the array (hipGetSymbolAddress, which may load the library's code object
  * there): make that first call eagerly, before capturing calls into a HIP
@@ -377,10 +376,18 @@ int gdn_quantized_matmul_f32(const float *x, const void *w, const void *scales, 
 int64_t gdn_quantized_matmul_f32_workspace_size(int M, int N, int K, int bits, int group_size);
 
 /*
- * gdn_quantized_matmul_rows_workspace_size - workspace bytes
- * gdn_quantized_matmul splits K with for 65 to 511 bf16 rows (0: it does not;
- * a call without a workspace keeps K whole).
+ * gdn_quantized_matmul_rows - gdn_quantized_matmul that also splits K for 65
+ * to 511 bf16 rows, as far as the workspace goes: with few column tiles
+ * (out_proj's shape) several workgroups share K, store float32 partial
+ * products in the workspace and a second kernel adds them in a fixed order.
+ * 4096 -> 2048 at 200 rows: 20 us, 34 unsplit. Up to 64 rows and above 511 it
+ * is gdn_quantized_matmul. gdn_quantized_matmul_rows_workspace_size: the bytes
+ * of the full split (0: K is not split).
  */
+int gdn_quantized_matmul_rows(const void *x, int x_dtype, const void *w, const void *scales,
+                              const void *biases, int sb_dtype, void *y, int y_dtype,
+                              const void *residual, int M, int N, int K, int bits, int group_size,
+                              void *workspace, int64_t workspace_bytes, void *stream);
 int64_t gdn_quantized_matmul_rows_workspace_size(int sb_dtype, int M, int N, int K, int bits,
                                                  int group_size);
 

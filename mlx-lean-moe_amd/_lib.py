@@ -16,7 +16,7 @@ import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libgdn.so")
-ABI_VERSION = 17
+ABI_VERSION = 18
 
 GDN_F32, GDN_BF16, GDN_F16 = 0, 1, 2
 GDN_EINVAL, GDN_EUNSUPPORTED = -1, -2
@@ -66,6 +66,9 @@ _SIGNATURES = {
     "gdn_quantized_matmul": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
                                       _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                                       _c_int, _c_void_p, _c_i64, _c_void_p]),
+    "gdn_quantized_matmul_rows": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,
+                                           _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
+                                           _c_int, _c_void_p, _c_i64, _c_void_p]),
     "gdn_quantized_matmul_noalloc": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p,
                                               _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int,
                                               _c_int, _c_int, _c_int, _c_void_p]),

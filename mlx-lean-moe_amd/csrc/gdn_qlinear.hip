@@ -1225,9 +1225,10 @@ extern "C" int64_t gdn_quantized_matmul_rows_workspace_size(int sb_dtype, int M,
 namespace gdn {
 namespace {
 
+// rows_bytes: what of the workspace a call of 65 to 511 rows may split K in.
 int quantized_matmul(const void* x, int x_dtype, const void* w, const void* scales, const void* biases,
                      int sb_dtype, void* y, int y_dtype, const void* residual, int M, int N, int K, int bits,
-                     int group_size, void* workspace, int64_t workspace_bytes, void* stream) {
+                     int group_size, void* workspace, int64_t workspace_bytes, int64_t rows_bytes, void* stream) {
     if (int rc = check_quant_args("gdn_quantized_matmul", w, scales, biases, sb_dtype, N, K, bits,
                                   group_size))
         return rc;
@@ -1261,9 +1262,10 @@ int quantized_matmul(const void* x, int x_dtype, const void* w, const void* scal
     }
     if (x_f32)
         return fail(GDN_EUNSUPPORTED, "gdn_quantized_matmul: float32 x needs a shape the decode kernel takes");
-    if (mid_kernel_takes(M, N, K, group_size, sb_dtype, workspace ? workspace_bytes : 0))
+    if (!workspace) rows_bytes = 0;
+    if (mid_kernel_takes(M, N, K, group_size, sb_dtype, rows_bytes))
         return launch_mid(x, wp, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, bits, group_size, workspace,
-                          workspace_bytes, s);
+                          rows_bytes, s);
     if (bits == 4) return dispatch_sb<4>(x, wp, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, group_size, s);
     return dispatch_sb<8>(x, wp, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, group_size, s);
 }
@@ -1326,7 +1328,15 @@ extern "C" int gdn_quantized_matmul(const void* x, int x_dtype, const void* w, c
                                     const void* residual, int M, int N, int K, int bits, int group_size,
                                     void* workspace, int64_t workspace_bytes, void* stream) {
     return quantized_matmul(x, x_dtype, w, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, bits,
-                            group_size, workspace, workspace_bytes, stream);
+                            group_size, workspace, workspace_bytes, 0, stream);
+}
+
+extern "C" int gdn_quantized_matmul_rows(const void* x, int x_dtype, const void* w, const void* scales,
+                                         const void* biases, int sb_dtype, void* y, int y_dtype,
+                                         const void* residual, int M, int N, int K, int bits, int group_size,
+                                         void* workspace, int64_t workspace_bytes, void* stream) {
+    return quantized_matmul(x, x_dtype, w, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, bits,
+                            group_size, workspace, workspace_bytes, workspace_bytes, stream);
 }
 
 extern "C" int gdn_quantized_matmul_noalloc(const void* x, int x_dtype, const void* w, const void* scales,
@@ -1341,7 +1351,7 @@ extern "C" int gdn_quantized_matmul_noalloc(const void* x, int x_dtype, const vo
                     static_cast<long long>(need), static_cast<long long>(kScratchBytes));
     if (need == 0)  // no split: the scratch is not touched
         return quantized_matmul(x, x_dtype, w, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K, bits,
-                                group_size, nullptr, 0, stream);
+                                group_size, nullptr, 0, 0, stream);
     const hipStream_t s = as_stream(stream);
     int dev = -1;
     hipError_t err = hipStreamGetDevice(s, &dev);
@@ -1365,7 +1375,7 @@ extern "C" int gdn_quantized_matmul_noalloc(const void* x, int x_dtype, const vo
             return fail(int(err), "gdn_quantized_matmul_noalloc: hipStreamWaitEvent: %s", hipGetErrorString(err));
     }
     const int rc = quantized_matmul(x, x_dtype, w, scales, biases, sb_dtype, y, y_dtype, residual, M, N, K,
-                                    bits, group_size, st.ptr, need, stream);
+                                    bits, group_size, st.ptr, need, 0, stream);
     if (rc != 0 || !eager) return rc;
     err = hipEventRecord(st.done, s);
     if (err != hipSuccess)

@@ -324,7 +324,8 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
     # a transient from the caching allocator (graph-capture safe); the split
     # kernels overwrite what they read
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device) if ws_bytes else None
-    _lib.call("gdn_quantized_matmul", _lib.ptr(x2), _lib.dtype_code(x2.dtype), _lib.ptr(w), _lib.ptr(scales),
+    # (above 64 rows only the second entry point splits K)
+    _lib.call("gdn_quantized_matmul" if M <= 64 else "gdn_quantized_matmul_rows", _lib.ptr(x2), _lib.dtype_code(x2.dtype), _lib.ptr(w), _lib.ptr(scales),
               _lib.ptr(biases), _lib.dtype_code(scales.dtype), _lib.ptr(y),
               _lib.dtype_code(y.dtype), _lib.ptr(r), M, N, K, quant.bits, quant.group_size, _lib.ptr(ws),
               ws_bytes, _lib.stream_ptr(x.device))
@@ -456,7 +457,8 @@ def f32_workspace_bytes(M: int, N: int, K: int, bits: int, group_size: int) -> i
 @functools.lru_cache(maxsize=256)
 def workspace_bytes(x_dtype: torch.dtype, sb_dtype: torch.dtype, M: int, N: int, K: int, bits: int,
                     group_size: int) -> int:
-    """Workspace gdn_quantized_matmul splits K with for these sizes (0: none)."""
+    """Workspace gdn_quantized_matmul (gdn_quantized_matmul_rows above 64 rows)
+    splits K with for these sizes (0: none)."""
 
     if M > 64:
         return int(_lib.load().gdn_quantized_matmul_rows_workspace_size(

@@ -748,3 +748,40 @@ def test_kept_copies_are_multiplied_above_the_decode_sizes(gpu, rows, N, K, monk
     plain = gdn.quantized_linear(x, W, scheme).double()
     mass = x.double().abs() @ kept.dense.double().abs().T
     assert ((y.double() - plain).abs() <= 2.0 ** -8 * plain.abs() + 2 * (K + 20) * 2.0 ** -24 * mass).all()
+
+
+@pytest.mark.parametrize("M,N,K,bits,gs", [(66, 2048, 4096, 4, 64), (200, 2048, 4096, 8, 64), (130, 1000, 2048, 4, 32),
+                                           (448, 2048, 4096, 4, 64)])
+def test_rows_above_the_decode_sizes_split_k_only_where_asked(gpu, M, N, K, bits, gs):
+    """gdn_quantized_matmul_rows splits K in a workspace (every partial block
+    is written, the sum is the same each time, half a workspace splits less);
+    gdn_quantized_matmul and gdn_quantized_matmul_noalloc do not, and agree bit
+    for bit whatever workspace the first one is given."""
+    rng = np.random.default_rng(M + K)
+    words, s, b = _weights(rng, N, K, bits, gs, "bf16")
+    W = _dev_weights(gpu, words, s, b, "bf16")
+    x = R.bf16_round(rng.standard_normal((M, K)))
+    w = Q.dequantize(words, s, b, bits, gs, out="bf16").astype(np.float64)
+    ref = x.astype(np.float64) @ w.T
+    bound = (K + 20) * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)
+    xt = torch.tensor(x, dtype=torch.float32, device=gpu).to(torch.bfloat16)
+    nbytes = _lib.load().gdn_quantized_matmul_rows_workspace_size(_lib.GDN_BF16, M, N, K, bits, gs)
+    assert nbytes >= 2 * M * N * 4
+
+    def run(name, ws_bytes):
+        y = torch.empty(M, N, device=gpu)
+        ws = torch.full((max(ws_bytes, 4) // 4,), float("nan"), device=gpu)
+        tail = () if name.endswith("noalloc") else (_lib.ptr(ws) if ws_bytes else None, ws_bytes)
+        _lib.call(name, _lib.ptr(xt), _lib.GDN_BF16, _lib.ptr(W["weight"]), _lib.ptr(W["scales"]),
+                  _lib.ptr(W["biases"]), _lib.GDN_BF16, _lib.ptr(y), _lib.GDN_F32, None, M, N, K, bits, gs, *tail,
+                  _lib.stream_ptr(xt.device))
+        assert (np.abs(y.cpu().numpy() - ref) <= bound).all()
+        return y
+
+    whole = run("gdn_quantized_matmul_noalloc", 0)
+    for ws_bytes in (0, nbytes, 4 * nbytes):
+        assert torch.equal(run("gdn_quantized_matmul", ws_bytes), whole)
+    assert torch.equal(run("gdn_quantized_matmul_rows", 0), whole)
+    split = run("gdn_quantized_matmul_rows", nbytes)
+    assert torch.equal(run("gdn_quantized_matmul_rows", nbytes), split) and not torch.equal(split, whole)
+    run("gdn_quantized_matmul_rows", nbytes // 2)
