@@ -23,6 +23,7 @@ import functools
 from dataclasses import dataclass
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -116,14 +117,22 @@ def _runs_dense(rows: int, N: int, K: int, quant: QuantScheme, sb_dtype: torch.d
 
 
 def _transformed(*operands: torch.Tensor | None) -> bool:
-    """Whether autograd or a function transform (vmap, forward mode) follows
-    these operands: torch's own products take part in those, the kernels'
-    calls do not, so such calls stay on the dense products."""
+    """Whether autograd, forward mode or a function transform (torch.vmap,
+    torch.func) follows these operands: torch's own products take part in
+    those, the kernels' calls do not, so such calls stay on the dense
+    products. An operand wrapped by a transform has no memory of its own,
+    which is what data_ptr raises for."""
 
-    if torch.autograd.forward_ad._current_level >= 0:
-        return True
-    return any(t is not None and (t.requires_grad and torch.is_grad_enabled()
-                                  or torch._C._functorch.is_functorch_wrapped_tensor(t)) for t in operands)
+    for t in operands:
+        if t is None:
+            continue
+        if t.requires_grad and torch.is_grad_enabled() or forward_ad.unpack_dual(t).tangent is not None:
+            return True
+        try:
+            t.data_ptr()
+        except RuntimeError:
+            return True
+    return False
 
 
 @dataclass(frozen=True)

@@ -85,3 +85,32 @@ def test_concat_quantized_stacks_along_rows():
     a, b = _qweights(N=3), _qweights(N=5)
     c = quant.concat_quantized([a, b])
     assert tuple(c["weight"].shape) == (8, 16) and tuple(c["scales"].shape) == (8, 2)
+
+
+def test_transforms_are_seen_through_public_interfaces(monkeypatch):
+    """Which operands keep a product on torch: one that autograd or forward
+    mode follows, or that a function transform wraps; asked without torch's
+    private modules, whose names change between versions."""
+    from torch.autograd import forward_ad
+
+    from mlx_lean_moe_amd.quant import _transformed
+
+    monkeypatch.delattr(torch._C._functorch, "is_functorch_wrapped_tensor")
+    x = torch.randn(3, 4)
+    seen = []
+
+    def probe(t):
+        seen.append((_transformed(t), _transformed(x, None, t), _transformed(x, None)))
+        return t * 2
+
+    torch.vmap(probe)(x)
+    torch.func.jvp(probe, (x,), (x,))
+    torch.func.grad(lambda t: probe(t).sum())(x)
+    torch.vmap(lambda t: torch.func.jvp(probe, (t,), (t,))[1])(x)
+    with forward_ad.dual_level():
+        probe(forward_ad.make_dual(x, x))
+        assert not _transformed(x)
+    probe(x.clone().requires_grad_())
+    assert seen == [(True, True, False)] * 6
+    with torch.no_grad():
+        assert not _transformed(x.clone().requires_grad_())
