@@ -40,13 +40,14 @@ GDN_DEV f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 // preparation
 // ---------------------------------------------------------------------------
 
-// Rows whose pieces would not be exact: a non-finite x, one so large that the
-// group sums could overflow where the products with the (small) weights do
-// not, or a row of magnitudes whose last piece leaves bf16's range. They are
-// multiplied apart (slow_row).
-constexpr float kRowMax = 0x1p100f, kRowMin = 0x1p-90f;
-// Columns whose scales or biases are not finite or so large that a group's
-// scaled sum could overflow are multiplied apart too (flags of 64 columns).
+// Rows whose pieces would not be exact (a non-finite x, a row of magnitudes
+// whose last piece leaves bf16's range), and rows and columns whose partial
+// sums could overflow where the products with the weights do not, are
+// multiplied apart (slow_row; flags of rows and of 64 columns). Inside the
+// limits no partial sum over K <= 2^20 of a scaled P (|q - c| <= 2^8: 2^20 2^16
+// 2^8 2^80) or of b' X (|b'| <= 2^24 + 2^8 2^16 = 2^25: 2^20 2^25 2^80), nor
+// their sum, reaches 2^127.
+constexpr float kRowMax = 0x1p80f, kRowMin = 0x1p-90f;
 constexpr float kScaleMax = 0x1p16f, kBiasMax = 0x1p24f;
 constexpr int kFlagCols = 64;
 

@@ -785,3 +785,32 @@ def test_rows_above_the_decode_sizes_split_k_only_where_asked(gpu, M, N, K, bits
     split = run("gdn_quantized_matmul_rows", nbytes)
     assert torch.equal(run("gdn_quantized_matmul_rows", nbytes), split) and not torch.equal(split, whole)
     run("gdn_quantized_matmul_rows", nbytes // 2)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("edge", [79, 80, 99, 126])
+def test_float32_rows_at_the_ends_of_their_range_do_not_overflow(gpu, bits, edge):
+    """Rows of +-2^edge against scales and biases just inside their limits and
+    codes whose weights s q + b cancel to zero, or to one scale: the partial
+    sums s (q - c) x and b' x must not overflow where the product does not."""
+    N, K, gs = 70, 4096, 128
+    s = 2.0 ** 15
+    top = 2 ** bits - 1
+    rng = np.random.default_rng(edge)
+    q0 = np.array([0, top, 8])[np.arange(N) % 3]
+    q = np.repeat(q0[:, None], K, 1)
+    q[:, 5] += np.where(q0 == top, -1, 1)  # one weight of a row is a scale, the others zero
+    W = {"weight": torch.tensor(Q.pack(q, bits).view(np.int32), device=gpu),
+         "scales": torch.full((N, K // gs), s, device=gpu),
+         "biases": torch.tensor(np.repeat(-q0[:, None] * s, K // gs, 1), dtype=torch.float32, device=gpu)}
+    x = np.ldexp(np.where(rng.random((40, K)) < 0.3, -1.0, 1.0), edge).astype(np.float32)
+    x[::2] = np.abs(x[::2])
+    x[:, 5] = np.ldexp(1.0, edge - 20)
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
+    want = np.ldexp(np.where(q0 == top, -1.0, 1.0), edge - 5)
+    # float32 sums of the cancelling terms |q0| s |x| of each of K elements
+    assert np.isfinite(y).all()
+    if edge >= 80:
+        np.testing.assert_array_equal(y, np.repeat(want[None], 40, 0).astype(np.float32))
+    else:
+        assert (np.abs(y - want) <= K * 2.0 ** -24 * K * s * 2 * 2 ** bits * 2.0 ** edge).all()
