@@ -363,7 +363,7 @@ int64_t gdn_quantized_matmul_workspace_size(int x_dtype, int sb_dtype, int M, in
  *   added to the product
  * x enters as three bf16 pieces (all 24 significant bits), the codes exactly;
  * scale and bias are applied per group to float32 partial sums (no weight is
- * rounded). x, w and workspace 16-byte aligned; the workspace takes
+ * rounded; the error is that of float32 sums over |x| |w|). x, w and workspace 16-byte aligned; the workspace takes
  * gdn_quantized_matmul_f32_workspace_size(...) bytes (0 for sizes the entry
  * point does not take) and must not be shared by overlapping calls.
  * Replaces mx.quantized_matmul(..., mode="affine") in quantized_linear

@@ -2,8 +2,8 @@
 // (gdn_quantized_matmul_f32): y = x W^T for float32 x (M, K) and MLX-packed
 // 4- or 8-bit codes, in float32 accuracy on the bf16 matrix cores.
 //
-// Both factors are taken exactly. A code less its centre, q - 2^(bits-1), is
-// a bf16 value; a float32 x is the sum of three bf16 values (its 24
+// Both factors are taken exactly. A code less an integer c of [0, 255] is a
+// bf16 value; a float32 x is the sum of three bf16 values (its 24
 // significant bits cut into three 8-bit pieces). So with
 //   P[m][n] = sum over one quantization group's k of x[m][k] (q[n][k] - c)
 // (three MFMAs a fragment pair, float32 sums of exact products), X[m][g] the
@@ -13,6 +13,11 @@
 // (777 rows of 2048 normal values against 12352 columns of 4-bit codes in
 // groups of 64: 1.2e-7 from float64, where the float32 library product of
 // rounded weights is 8.1e-7 off and takes 345 us to this one's 125-129).
+// c is the group's own: the integer nearest to -b / s, the code of the weight
+// nearest to zero, so that |b'| <= |s| / 2 and the two terms of a weight w are
+// at most 3 |w| together (0 for w = 0; with one c for all, an x thousands of
+// times the rest left the rounding of c s x where its weight is 0). Where -b /
+// s lies outside [0, 255], c is the nearer end and the terms have one sign.
 //
 // Two launches (three where K is split): the preparation cuts x, sums its
 // groups and lays s and b' out group-major; the product kernel does the rest.
@@ -50,25 +55,32 @@ GDN_DEV f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 constexpr float kRowMax = 0x1p80f, kRowMin = 0x1p-90f;
 constexpr float kScaleMax = 0x1p16f, kBiasMax = 0x1p24f;
 constexpr int kFlagCols = 64;
+__host__ __device__ constexpr int64_t padded_columns(int64_t n) { return (n + kBN - 1) / kBN * kBN; }
 
 // Blocks 0 .. M - 1: row m of x as bf16 pieces, pieces[m][step][part][64]
 // (part 0 the upper 8 significant bits; truncation, so no piece can round up
 // to infinity), its group sums (in double, rounded once) and its flag. The
-// blocks after them, 64 columns each: s and b' = b + centre s in float32,
-// group-major, and the columns' flag (at flags[M + block]).
+// blocks after them, 64 columns each: s and b' = b + c s in float32,
+// group-major, c as a byte (c_t[group][64-column block][n % 16][n / 16 % 4]: a
+// word for the four columns of a lane of the product) and the columns' flag (at
+// flags[M + block]). The rows of s and c have padded_columns(N) columns; those
+// past N are read for outputs that are not stored.
 __global__ __launch_bounds__(256) void prepare_f32_kernel(
     const float* __restrict__ x, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
     uint16_t* __restrict__ pieces, float* __restrict__ xsum, int* __restrict__ flags, float* __restrict__ s_t,
-    float* __restrict__ b_t, int M, int N, int K, int group_size, float centre) {
+    float* __restrict__ b_t, uint8_t* __restrict__ c_t, int M, int N, int K, int group_size) {
     const int G = K / group_size;
     if (int(blockIdx.x) >= M) {
-        const int64_t n = int64_t(int(blockIdx.x) - M) * kFlagCols + (threadIdx.x & 63);
+        const int block = int(blockIdx.x) - M, lane = threadIdx.x & 63;
+        const int64_t stride = padded_columns(N), n = int64_t(block) * kFlagCols + lane;
         bool far = false;
         for (int g = threadIdx.x >> 6; g < G && n < N; g += 4) {
             const float s = load_any(scales, n * G + g, sb_dtype), b = load_any(biases, n * G + g, sb_dtype);
             far |= !(fabsf(s) < kScaleMax && fabsf(b) < kBiasMax);
-            s_t[int64_t(g) * N + n] = s;
-            b_t[int64_t(g) * N + n] = __builtin_fmaf(centre, s, b);
+            const float c = fminf(fmaxf(rintf(-b / s), 0.f), 255.f);  // s = 0: any, b' = b
+            s_t[g * stride + n] = s;
+            c_t[g * stride + block * kFlagCols + (lane % 16) * 4 + lane / 16] = uint8_t(c);
+            b_t[int64_t(g) * N + n] = __builtin_fmaf(c, s, b);
         }
         far = __syncthreads_or(far);
         if (threadIdx.x == 0) flags[blockIdx.x] = far;
@@ -119,18 +131,27 @@ __global__ __launch_bounds__(256) void prepare_f32_kernel(
 // product
 // ---------------------------------------------------------------------------
 
-// 8 codes less their centre as bf16 (exact: the float's upper half).
+// 8 codes less c as bf16 (exact: the float's upper half). A masked 4-bit code
+// in a byte is the e4m3 value q 2^-9, so one conversion gives two.
 template <int kBits>
-GDN_DEV bf16x8 centred_fragment(const uint32_t* words) {
+GDN_DEV bf16x8 centred_fragment(const uint32_t* words, float c) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    constexpr int kPer = 32 / kBits;
     u32x4 d;
     float f[8];
+    if constexpr (kBits == 4) {
+        const uint32_t half[2] = {words[0] & 0x0F0F0F0Fu, (words[0] >> 4) & 0x0F0F0F0Fu};  // codes 0 2 4 6, 1 3 5 7
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        // flipping a field's top bit makes it the two's complement of q - centre
-        const int32_t v = int32_t(words[j / kPer] ^ (kBits == 4 ? 0x88888888u : 0x80808080u));
-        f[j] = float((v << (32 - kBits * (j % kPer + 1))) >> (32 - kBits));
+        for (int i = 0; i < 2; ++i) {
+            const auto lo = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(half[i], 512.f, false);
+            const auto hi = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(half[i], 512.f, true);
+            f[i] = lo[0] - c;
+            f[2 + i] = lo[1] - c;
+            f[4 + i] = hi[0] - c;
+            f[6 + i] = hi[1] - c;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = float((words[j / 4] >> (8 * (j % 4))) & 255u) - c;
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -165,9 +186,9 @@ GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__
 // 2.1 PFLOP/s: 58 us of 125): with two waves on a SIMD a wave's LDS reads,
 // conversions and scaling are not all covered. A wave in its MFMAs goes before
 // one that loads or converts (131 us without). Fetching the codes two steps
-// ahead, or the next row tile's fragments, spilled or gained nothing, and
-// codes converted by the fp8 instruction (uncentred, a third of the
-// instructions) gained 1 % at 2.5 times the error.
+// ahead, or the next row tile's fragments, spilled or gained nothing. One c for
+// all groups (no c_t, a shift in place of the fp8 conversion and subtraction)
+// takes the same time at this size, 8-bit K = 4096 153 us to 157.
 //
 // kG32: groups of 32 (an MFMA's k), each scaled by itself; else one group (64
 // or half of 128) a step. Lane quarter q = l / 16 holds k 8 q .. of each
@@ -178,9 +199,10 @@ GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__
 template <int kBits, int kTM, bool kG32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void qlinear_f32_kernel(
     const uint16_t* __restrict__ pieces, const float* __restrict__ xsum, const int* __restrict__ flags,
-    const float* __restrict__ s_t, const float* __restrict__ b_t, const float* __restrict__ x,
-    const uint32_t* __restrict__ w, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
-    float* out, const float* residual, int M, int N, int K, int group_size, int mt, int tiles) {
+    const float* __restrict__ s_t, const float* __restrict__ b_t, const uint32_t* __restrict__ c_t,
+    const float* __restrict__ x, const uint32_t* __restrict__ w, const void* __restrict__ scales,
+    const void* __restrict__ biases, int sb_dtype, float* out, const float* residual, int M, int N, int K,
+    int group_size, int mt, int tiles) {
     constexpr int kBM = 16 * kTM;
     constexpr int kPiecesPerRow = kPK / 8;
     constexpr int kXLoads = (kBM * kPiecesPerRow + 255) / 256;
@@ -231,21 +253,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     };
 
     const int64_t wpr = int64_t(K) * kBits / 32;
-    uint32_t wo[kTN], so[kTN];
+    uint32_t wo[kTN];
 #pragma unroll
     for (int b = 0; b < kTN; ++b) {
         wo[b] = (uint32_t(col[b] - n0) * uint32_t(wpr) + lq * (kG32 ? kWords / 2 : kWords)) * 4;
-        so[b] = uint32_t(col[b] - n0) * 4;
     }
-    // a step's codes (words of MFMA block kb at [b][kb kWords / 2 ..]) and scales
+    static_assert(kFlagCols == 16 * kTN, "a wave's columns share a flag and a word of c");
+    const int blocks = (N + kFlagCols - 1) / kFlagCols, wblock = n0 / kFlagCols + wv;
+    const int64_t sstride = padded_columns(N);
+    // a step's codes (words of MFMA block kb at [b][kb kWords / 2 ..]), scales and c
     struct Codes {
         uint32_t wd[kTN][kWords];
         float sc[kTN][kG32 ? 2 : 1];
+        uint32_t centre[kG32 ? 2 : 1];  // a byte a column
     };
     Codes c;
     auto fetch_w = [&](int s) {
         const char* wtile = reinterpret_cast<const char*>(w + n0 * wpr + s * kBK * kBits / 32);
         const int g = s * kBK / group_size;
+#pragma unroll
+        for (int i = 0; i < (kG32 ? 2 : 1); ++i) c.centre[i] = (c_t + ((g + i) * sstride + n0) / 4 + 16 * wv)[lr];
 #pragma unroll
         for (int b = 0; b < kTN; ++b) {
             const uint32_t* src = reinterpret_cast<const uint32_t*>(wtile + wo[b]);
@@ -253,7 +280,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
             for (int i = 0; i < kWords; ++i) c.wd[b][i] = src[kG32 ? i / (kWords / 2) * kBits + i % (kWords / 2) : i];
 #pragma unroll
             for (int i = 0; i < (kG32 ? 2 : 1); ++i)
-                c.sc[b][i] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(s_t + int64_t(g + i) * N + n0) + so[b]);
+                c.sc[b][i] = (s_t + (g + i) * sstride + n0 + 16 * kTN * wv)[lr + 16 * b];
         }
     };
 
@@ -294,10 +321,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 #pragma unroll
         for (int b = 0; b < kTN; ++b) {
 #pragma unroll
-            for (int kb = 0; kb < 2; ++kb) bf[b][kb] = centred_fragment<kBits>(&c.wd[b][kb * kWords / 2]);
+            for (int kb = 0; kb < 2; ++kb)
+                bf[b][kb] = centred_fragment<kBits>(&c.wd[b][kb * kWords / 2], float((c.centre[kG32 ? kb : 0] >> (8 * b)) & 255u));
 #pragma unroll
             for (int i = 0; i < (kG32 ? 2 : 1); ++i) scale[b][i] = c.sc[b][i];
         }
+        __builtin_amdgcn_sched_barrier(0);  // the codes' registers first: fetches hoisted above them spill
         const int next = s < last ? s + 1 : last;  // the last step again, unused
         fetch_x(next);
         fetch_w(next);
@@ -340,13 +369,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 
     // flagged rows, and the wave's own 64 columns when flagged, are left to
     // the loop below
-    static_assert(kFlagCols == 16 * kTN, "a wave's columns share a flag");
-    const int cols = (N + kFlagCols - 1) / kFlagCols, col0 = n0 / kFlagCols;
+    const int col0 = n0 / kFlagCols;
     int any = 0;
     if (tid < kBM) any = flags[m0 + tid < M ? m0 + tid : M - 1];
-    if (tid < kBN / kFlagCols && col0 + tid < cols) any |= flags[M + col0 + tid];
+    if (tid < kBN / kFlagCols && col0 + tid < blocks) any |= flags[M + col0 + tid];
     any = __syncthreads_or(any);
-    const int far = any && col0 + wv < cols ? flags[M + col0 + wv] : 0;
+    const int far = any && wblock < blocks ? flags[M + wblock] : 0;
     float* dst = out + int64_t(blockIdx.y) * M * N;
 #pragma unroll
     for (int a = 0; a < kTM; ++a)
@@ -378,7 +406,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 
 struct F32Plan {
     int tm, splits;
-    int64_t pieces, xsum, flags, s_t, b_t, partial, bytes;  // workspace offsets
+    int64_t pieces, xsum, flags, s_t, b_t, c_t, partial, bytes;  // workspace offsets
 };
 
 // Rows of a workgroup and splits of K: the least time by the matrix cores'
@@ -405,8 +433,9 @@ F32Plan plan_f32(int M, int N, int K, int group_size) {
     p.xsum = up(int64_t(M) * K * kParts * 2);
     p.flags = p.xsum + up(M * G * 4);
     p.s_t = p.flags + up((int64_t(M) + (N + kFlagCols - 1) / kFlagCols) * 4);
-    p.b_t = p.s_t + up(N * G * 4);
-    p.partial = p.b_t + up(N * G * 4);
+    p.b_t = p.s_t + up(padded_columns(N) * G * 4);
+    p.c_t = p.b_t + up(N * G * 4);
+    p.partial = p.c_t + up(padded_columns(N) * G);
     p.bytes = p.partial + (p.splits > 1 ? int64_t(p.splits) * M * N * 4 : 0);
     return p;
 }
@@ -466,18 +495,20 @@ extern "C" int gdn_quantized_matmul_f32(const float* x, const void* w, const voi
     auto* flags = reinterpret_cast<int*>(ws + p.flags);
     auto* s_t = reinterpret_cast<float*>(ws + p.s_t);
     auto* b_t = reinterpret_cast<float*>(ws + p.b_t);
+    auto* c_t = reinterpret_cast<uint8_t*>(ws + p.c_t);
     auto* partial = reinterpret_cast<float*>(ws + p.partial);
     const int64_t sb_blocks = (int64_t(N) + kFlagCols - 1) / kFlagCols;
     hipLaunchKernelGGL(prepare_f32_kernel, dim3(unsigned(M + sb_blocks)), dim3(256), 0, s, x, scales, biases, sb_dtype,
-                       pieces, xsum, flags, s_t, b_t, M, N, K, group_size, bits == 4 ? 8.f : 128.f);
+                       pieces, xsum, flags, s_t, b_t, c_t, M, N, K, group_size);
     if (int rc = check_launch("gdn_quantized_matmul_f32/prepare")) return rc;
 
     const int mt = (M + 16 * p.tm - 1) / (16 * p.tm), tiles = mt * ((N + kBN - 1) / kBN);
     const auto kernel = bits == 4 ? (group_size == 32 ? kernel_of<4, true>(p.tm) : kernel_of<4, false>(p.tm))
                                   : (group_size == 32 ? kernel_of<8, true>(p.tm) : kernel_of<8, false>(p.tm));
     hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8), unsigned(p.splits)), dim3(256), 0, s, pieces, xsum,
-                       flags, s_t, b_t, x, static_cast<const uint32_t*>(w), scales, biases, sb_dtype,
-                       p.splits > 1 ? partial : y, p.splits > 1 ? nullptr : residual, M, N, K, group_size, mt, tiles);
+                       flags, s_t, b_t, reinterpret_cast<const uint32_t*>(c_t), x, static_cast<const uint32_t*>(w),
+                       scales, biases, sb_dtype, p.splits > 1 ? partial : y, p.splits > 1 ? nullptr : residual, M, N,
+                       K, group_size, mt, tiles);
     if (int rc = check_launch(fn)) return rc;
     if (p.splits > 1)
         return launch_split_sum(partial, p.splits, int64_t(M) * N, y, GDN_F32, residual, s, "gdn_quantized_matmul_f32/sum");

@@ -814,3 +814,32 @@ def test_float32_rows_at_the_ends_of_their_range_do_not_overflow(gpu, bits, edge
         np.testing.assert_array_equal(y, np.repeat(want[None], 40, 0).astype(np.float32))
     else:
         assert (np.abs(y - want) <= K * 2.0 ** -24 * K * s * 2 * 2 ** bits * 2.0 ** edge).all()
+
+
+@pytest.mark.parametrize("N,K,bits,gs,exact_zero", [(300, 2048, 4, 64, True), (130, 1024, 8, 64, True),
+                                                    (130, 1024, 4, 32, False), (70, 4096, 8, 128, False)])
+def test_float32_rows_with_outlying_activations_against_small_weights(gpu, N, K, bits, gs, exact_zero):
+    """A few activations 10^9 times the rest where the weights are zero (or the
+    codes nearest to zero): within float32 sums of |x| |w|. A group's two terms
+    s (q - c) and b' = b + c s are at most 3 |w| together for c = round(-b / s)
+    (test_float32_rows_in_three_bf16_pieces counts the sums)."""
+    rng = np.random.default_rng(N + K)
+    M, G = 50, K // gs
+    s = R.bf16_round(rng.uniform(0.005, 0.01, (N, G))) * np.where(rng.random((N, G)) < 0.5, -1, 1)
+    q0 = rng.integers(0, 2 ** bits, (N, G))
+    b = -q0 * s if exact_zero else -(q0 + rng.uniform(-0.5, 0.5, (N, G))) * s
+    s, b = s.astype(np.float32), b.astype(np.float32)
+    q = rng.integers(0, 2 ** bits, (N, K))
+    big = rng.choice(K, 5, replace=False)
+    q[:, big] = q0[:, big // gs]
+    W = {"weight": torch.tensor(Q.pack(q, bits).view(np.int32), device=gpu), "scales": torch.tensor(s, device=gpu),
+         "biases": torch.tensor(b, device=gpu)}
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[:, big] *= np.float32(1e9)
+    w = np.repeat(s, gs, 1).astype(np.float64) * q + np.repeat(b, gs, 1)
+    if exact_zero:
+        assert (w[:, big] == 0).all()
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
+    mass = np.abs(x).astype(np.float64) @ np.abs(w).T
+    bound = (3 * gs + 2 * G + 22) * 2.0 ** -24 * 3 * mass
+    assert (np.abs(y - x.astype(np.float64) @ w.T) <= bound).all()
