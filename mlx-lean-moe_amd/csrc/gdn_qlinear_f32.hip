@@ -48,7 +48,7 @@ GDN_DEV f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 // Rows whose pieces would not be exact (a non-finite x, a row of magnitudes
 // whose last piece leaves bf16's range), and rows and columns whose partial
 // sums could overflow where the products with the weights do not, are
-// multiplied apart (slow_row; flags of rows and of 64 columns). Inside the
+// multiplied apart (float_rows; flags of rows and of 64 columns). Inside the
 // limits no partial sum over K <= 2^20 of a scaled P (|q - c| <= 2^8: 2^20 2^16
 // 2^8 2^80) or of b' X (|b'| <= 2^24 + 2^8 2^16 = 2^25: 2^20 2^25 2^80), nor
 // their sum, reaches 2^127.
@@ -60,15 +60,16 @@ __host__ __device__ constexpr int64_t padded_columns(int64_t n) { return (n + kB
 // Blocks 0 .. M - 1: row m of x as bf16 pieces, pieces[m][step][part][64]
 // (part 0 the upper 8 significant bits; truncation, so no piece can round up
 // to infinity), its group sums (in double, rounded once) and its flag. The
-// blocks after them, 64 columns each: s and b' = b + c s in float32,
+// blocks after them, 64 columns each: s, b (o_t) and b' = b + c s in float32,
 // group-major, c as a byte (c_t[group][64-column block][n % 16][n / 16 % 4]: a
 // word for the four columns of a lane of the product) and the columns' flag (at
-// flags[M + block]). The rows of s and c have padded_columns(N) columns; those
+// flags[M + block]). The rows of s, b and c have padded_columns(N) columns; those
 // past N are read for outputs that are not stored.
 __global__ __launch_bounds__(256) void prepare_f32_kernel(
     const float* __restrict__ x, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
     uint16_t* __restrict__ pieces, float* __restrict__ xsum, int* __restrict__ flags, float* __restrict__ s_t,
-    float* __restrict__ b_t, uint8_t* __restrict__ c_t, int M, int N, int K, int group_size) {
+    float* __restrict__ b_t, float* __restrict__ o_t, uint8_t* __restrict__ c_t, int M, int N, int K,
+    int group_size) {
     const int G = K / group_size;
     if (int(blockIdx.x) >= M) {
         const int block = int(blockIdx.x) - M, lane = threadIdx.x & 63;
@@ -79,6 +80,7 @@ __global__ __launch_bounds__(256) void prepare_f32_kernel(
             far |= !(fabsf(s) < kScaleMax && fabsf(b) < kBiasMax);
             const float c = fminf(fmaxf(rintf(-b / s), 0.f), 255.f);  // s = 0: any, b' = b
             s_t[g * stride + n] = s;
+            o_t[g * stride + n] = b;
             c_t[g * stride + block * kFlagCols + (lane % 16) * 4 + lane / 16] = uint8_t(c);
             b_t[int64_t(g) * N + n] = __builtin_fmaf(c, s, b);
         }
@@ -159,21 +161,73 @@ GDN_DEV bf16x8 centred_fragment(const uint32_t* words, float c) {
     return __builtin_bit_cast(bf16x8, d);
 }
 
-// One flagged row's columns of the workgroup, a thread a column, from the
-// float32 weights: what the pieces cannot carry (infinities, NaN, the ends
-// of the range).
-template <int kBits>
-GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__ w, const void* scales,
-                       const void* biases, int sb_dtype, int64_t n, int K, int group_size) {
+// The workgroup's rows of x (past M - 1 repeating it) by a wave's 64 columns
+// from n0 over the k range [k0, k1), from the float32 weights s q + b on the
+// float32 matrix cores: what the pieces and group sums cannot carry
+// (infinities, NaN, the ends of the range). Lane (lr, lq) holds row or column
+// lr and k 4 lq .. of each 16, the next 16's operands in registers meanwhile.
+// All of 777 rows flagged, 2048 -> 12352, take 612 us, one row 383, ordinary
+// rows 130 (a thread a column and a serial chain a row took 234 ms and 950 us).
+template <int kBits, int kTM>
+GDN_DEV void float_rows(const float* __restrict__ x, const uint32_t* __restrict__ w, const float* __restrict__ s_t,
+                        const float* __restrict__ o_t, int m0, int n0, int M, int N, int K, int group_size, int k0,
+                        int k1, int lr, int lq, f32x4 (&v)[kTM][kTN]) {
     constexpr int kPer = 32 / kBits;
-    const int64_t G = K / group_size;
-    float v = 0.f;
-    for (int k = 0; k < K; ++k) {
-        const uint32_t q = (w[n * (K / kPer) + k / kPer] >> (kBits * (k % kPer))) & ((1u << kBits) - 1u);
-        const int64_t gi = n * G + k / group_size;
-        v = __builtin_fmaf(x[k], __builtin_fmaf(load_any(scales, gi, sb_dtype), float(q), load_any(biases, gi, sb_dtype)), v);
+    const int64_t stride = padded_columns(N);
+    const float* xr[kTM];
+    const uint32_t* wr[kTN];
+#pragma unroll
+    for (int a = 0; a < kTM; ++a) {
+        const int64_t m = m0 + 16 * a + lr;
+        xr[a] = x + (m < M ? m : M - 1) * K + 4 * lq;
+#pragma unroll
+        for (int b = 0; b < kTN; ++b) v[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
-    return v;
+#pragma unroll
+    for (int b = 0; b < kTN; ++b) {
+        const int64_t n = n0 + 16 * b + lr;
+        wr[b] = w + (n < N ? n : N - 1) * (K / kPer);
+    }
+    struct Operands {
+        f32x4 x[kTM];
+        uint32_t wd[kTN];
+        float s[kTN], o[kTN];
+    };
+    const auto fetch = [&](int k) {
+        Operands p;
+        const int kl = k + 4 * lq;
+        const int64_t at = kl / group_size * stride + n0 + lr;
+#pragma unroll
+        for (int a = 0; a < kTM; ++a) p.x[a] = *reinterpret_cast<const f32x4*>(xr[a] + k);
+#pragma unroll
+        for (int b = 0; b < kTN; ++b) {
+            p.wd[b] = wr[b][kl / kPer];
+            p.s[b] = s_t[at + 16 * b];
+            p.o[b] = o_t[at + 16 * b];
+        }
+        return p;
+    };
+    Operands p = fetch(k0);
+#pragma unroll 1
+    for (int k = k0; k < k1; k += 16) {
+        const Operands next = fetch(k + 16 < k1 ? k + 16 : k);
+        f32x4 wf[kTN];
+#pragma unroll
+        for (int b = 0; b < kTN; ++b)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t q = p.wd[b] >> (kBits * ((4 * lq) % kPer) + kBits * j) & ((1u << kBits) - 1u);
+                wf[b][j] = __builtin_fmaf(p.s[b], float(q), p.o[b]);
+            }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int a = 0; a < kTM; ++a)
+#pragma unroll
+                for (int b = 0; b < kTN; ++b)
+                    v[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(p.x[a][j], wf[b][j], v[a][b], 0, 0, 0);
+        p = next;
+    }
 }
 
 // A workgroup holds 16 kTM rows by 256 columns, each of its 4 waves all the
@@ -199,10 +253,9 @@ GDN_DEV float slow_row(const float* __restrict__ x, const uint32_t* __restrict__
 template <int kBits, int kTM, bool kG32>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void qlinear_f32_kernel(
     const uint16_t* __restrict__ pieces, const float* __restrict__ xsum, const int* __restrict__ flags,
-    const float* __restrict__ s_t, const float* __restrict__ b_t, const uint32_t* __restrict__ c_t,
-    const float* __restrict__ x, const uint32_t* __restrict__ w, const void* __restrict__ scales,
-    const void* __restrict__ biases, int sb_dtype, float* out, const float* residual, int M, int N, int K,
-    int group_size, int mt, int tiles) {
+    const float* __restrict__ s_t, const float* __restrict__ b_t, const float* __restrict__ o_t,
+    const uint32_t* __restrict__ c_t, const float* __restrict__ x, const uint32_t* __restrict__ w, float* out,
+    const float* residual, int M, int N, int K, int group_size, int mt, int tiles) {
     constexpr int kBM = 16 * kTM;
     constexpr int kPiecesPerRow = kPK / 8;
     constexpr int kXLoads = (kBM * kPiecesPerRow + 255) / 256;
@@ -368,7 +421,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
     }
 
     // flagged rows, and the wave's own 64 columns when flagged, are left to
-    // the loop below
+    // float_rows below
     const int col0 = n0 / kFlagCols;
     int any = 0;
     if (tid < kBM) any = flags[m0 + tid < M ? m0 + tid : M - 1];
@@ -390,14 +443,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
                 dst[e] = acc[a][b][i] + (residual ? residual[e] : 0.f);
             }
         }
-    if (any && n0 + tid < N) {  // thread tid's column lies in its own wave's 64
-        for (int r = 0; r < kBM && m0 + r < M; ++r) {
-            if (!far && !flags[m0 + r]) continue;
-            const int64_t m = m0 + r, n = n0 + tid, e = m * N + n;
-            const float v = blockIdx.y == 0 ? slow_row<kBits>(x + m * K, w, scales, biases, sb_dtype, n, K, group_size) : 0.f;
-            dst[e] = v + (residual ? residual[e] : 0.f);
+    if (!any || wblock >= blocks) return;
+    float_rows<kBits, kTM>(x, w, s_t, o_t, m0, n0 + 16 * kTN * wv, M, N, K, group_size, step0 * kBK, (last + 1) * kBK,
+                           lr, lq, acc);
+#pragma unroll
+    for (int a = 0; a < kTM; ++a)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + 16 * a + 4 * lq + i;
+            if (m >= M || !(far || flags[m])) continue;
+#pragma unroll
+            for (int b = 0; b < kTN; ++b) {
+                const int n = n0 + 16 * kTN * wv + 16 * b + lr;
+                if (n >= N) continue;
+                const int64_t e = int64_t(m) * N + n;
+                dst[e] = acc[a][b][i] + (residual ? residual[e] : 0.f);
+            }
         }
-    }
 }
 
 // ---------------------------------------------------------------------------
@@ -406,7 +468,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 
 struct F32Plan {
     int tm, splits;
-    int64_t pieces, xsum, flags, s_t, b_t, c_t, partial, bytes;  // workspace offsets
+    int64_t pieces, xsum, flags, s_t, b_t, o_t, c_t, partial, bytes;  // workspace offsets
 };
 
 // Rows of a workgroup and splits of K: the least time by the matrix cores'
@@ -434,7 +496,8 @@ F32Plan plan_f32(int M, int N, int K, int group_size) {
     p.flags = p.xsum + up(M * G * 4);
     p.s_t = p.flags + up((int64_t(M) + (N + kFlagCols - 1) / kFlagCols) * 4);
     p.b_t = p.s_t + up(padded_columns(N) * G * 4);
-    p.c_t = p.b_t + up(N * G * 4);
+    p.o_t = p.b_t + up(N * G * 4);
+    p.c_t = p.o_t + up(padded_columns(N) * G * 4);
     p.partial = p.c_t + up(padded_columns(N) * G);
     p.bytes = p.partial + (p.splits > 1 ? int64_t(p.splits) * M * N * 4 : 0);
     return p;
@@ -495,20 +558,21 @@ extern "C" int gdn_quantized_matmul_f32(const float* x, const void* w, const voi
     auto* flags = reinterpret_cast<int*>(ws + p.flags);
     auto* s_t = reinterpret_cast<float*>(ws + p.s_t);
     auto* b_t = reinterpret_cast<float*>(ws + p.b_t);
+    auto* o_t = reinterpret_cast<float*>(ws + p.o_t);
     auto* c_t = reinterpret_cast<uint8_t*>(ws + p.c_t);
     auto* partial = reinterpret_cast<float*>(ws + p.partial);
     const int64_t sb_blocks = (int64_t(N) + kFlagCols - 1) / kFlagCols;
     hipLaunchKernelGGL(prepare_f32_kernel, dim3(unsigned(M + sb_blocks)), dim3(256), 0, s, x, scales, biases, sb_dtype,
-                       pieces, xsum, flags, s_t, b_t, c_t, M, N, K, group_size);
+                       pieces, xsum, flags, s_t, b_t, o_t, c_t, M, N, K, group_size);
     if (int rc = check_launch("gdn_quantized_matmul_f32/prepare")) return rc;
 
     const int mt = (M + 16 * p.tm - 1) / (16 * p.tm), tiles = mt * ((N + kBN - 1) / kBN);
     const auto kernel = bits == 4 ? (group_size == 32 ? kernel_of<4, true>(p.tm) : kernel_of<4, false>(p.tm))
                                   : (group_size == 32 ? kernel_of<8, true>(p.tm) : kernel_of<8, false>(p.tm));
     hipLaunchKernelGGL(kernel, dim3(unsigned((tiles + 7) / 8 * 8), unsigned(p.splits)), dim3(256), 0, s, pieces, xsum,
-                       flags, s_t, b_t, reinterpret_cast<const uint32_t*>(c_t), x, static_cast<const uint32_t*>(w),
-                       scales, biases, sb_dtype, p.splits > 1 ? partial : y, p.splits > 1 ? nullptr : residual, M, N,
-                       K, group_size, mt, tiles);
+                       flags, s_t, b_t, o_t, reinterpret_cast<const uint32_t*>(c_t), x,
+                       static_cast<const uint32_t*>(w), p.splits > 1 ? partial : y, p.splits > 1 ? nullptr : residual,
+                       M, N, K, group_size, mt, tiles);
     if (int rc = check_launch(fn)) return rc;
     if (p.splits > 1)
         return launch_split_sum(partial, p.splits, int64_t(M) * N, y, GDN_F32, residual, s, "gdn_quantized_matmul_f32/sum");

@@ -843,3 +843,62 @@ def test_float32_rows_with_outlying_activations_against_small_weights(gpu, N, K,
     mass = np.abs(x).astype(np.float64) @ np.abs(w).T
     bound = (3 * gs + 2 * G + 22) * 2.0 ** -24 * 3 * mass
     assert (np.abs(y - x.astype(np.float64) @ w.T) <= bound).all()
+
+
+@pytest.mark.parametrize("M,N,K,bits,gs,sb", [
+    (33, 300, 512, 4, 64, "bf16"),      # ragged rows and columns
+    (81, 257, 384, 8, 128, "f32"),      # one row past five tiles
+    (200, 2048, 4096, 4, 64, "bf16"),   # K split
+    (50, 96, 1024, 4, 32, "f16"),
+    (16, 40, 64, 8, 32, "f32"),         # a single step
+])
+def test_whole_prompts_of_float32_rows_outside_the_pieces_range(gpu, M, N, K, bits, gs, sb):
+    """Every row (and one column block) out of the pieces' range: infinities,
+    NaN, and rows of 2^85 (at most 2^2 of them a value, times 2^28 and 128 of
+    the column block's weights: below 2^127) and 2^-125, whose products are
+    subnormal, within float32 sums of the float64 product."""
+    rng = np.random.default_rng(M + N)
+    words, s, b = _weights(rng, N, K, bits, gs, sb)
+    if sb == "f32":
+        s[0, 0], b[0, 0] = np.float32(2.0 ** 20), np.float32(-3 * 2.0 ** 20)
+    W = _dev_weights(gpu, words, s, b, sb)
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    x[0::4] *= np.float32(2.0 ** 85)
+    x[1::4] *= np.float32(2.0 ** -125)
+    x[2::4, 3] = np.inf
+    x[3::4, 5] = np.nan
+    w = Q.dequantize(words, s, b, bits, gs, out="f32").astype(np.float64)
+    with np.errstate(invalid="ignore"):
+        ref = x.astype(np.float64) @ w.T
+        mass = np.abs(x).astype(np.float64) @ np.abs(w).T
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
+    np.testing.assert_array_equal(y[2::4], ref[2::4].astype(np.float32))
+    for rows in (slice(0, None, 4), slice(1, None, 4)):
+        assert (np.abs(y[rows] - ref[rows]) <= 2 * K * 2.0 ** -24 * mass[rows] + K * 2.0 ** -149).all()
+
+
+def test_float32_rows_outside_the_pieces_range_cost_a_bounded_multiple(gpu):
+    """A prompt whose rows all hold an infinity takes about 4 times an ordinary
+    one's time (the float32 matrix cores have a quarter of the bf16 ones' rate
+    for a piece), not a serial chain a row: 20 times leaves room for noise."""
+    M, N, K = 300, 2048, 2048
+    rng = np.random.default_rng(1)
+    words, s, b = _weights(rng, N, K, 4, 64, "bf16")
+    W = _dev_weights(gpu, words, s, b, "bf16")
+    x = torch.randn(M, K, device=gpu)
+    far = x.clone()
+    far[:, 3] = float("inf")
+    times = []
+    for t in (x, far):
+        best = float("inf")
+        for _ in range(5):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                gdn.quantized_linear(t, W, gdn.QuantScheme(4, 64))
+            end.record()
+            end.synchronize()
+            best = min(best, start.elapsed_time(end))
+        times.append(best)
+    assert times[1] < 20 * times[0], times
