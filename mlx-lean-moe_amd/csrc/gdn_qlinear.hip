@@ -1425,7 +1425,7 @@ __global__ __launch_bounds__(256) void dequantize_scheme_kernel(
     const uint32_t* __restrict__ w, const void* __restrict__ scales, const void* __restrict__ biases,
     int sb_dtype, void* __restrict__ out, int out_dtype, int N, int K, int group_size, bool wide) {
     const int chunks = K / 8;
-    const int64_t t = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t t = (int64_t(blockIdx.y) * gridDim.x + blockIdx.x) * 256 + threadIdx.x;
     if (t >= int64_t(N) * chunks) return;
     const int64_t n = t / chunks, row_words = int64_t(K) * kBits / 32;
     const int k0 = int(t % chunks) * 8;
@@ -1932,9 +1932,11 @@ extern "C" int gdn_dequantize(const void* w, const void* scales, const void* bia
                 "gdn_dequantize: K=%d must be a multiple of group_size and fill whole words", K);
     GDN_REQUIRE(w && scales && (mode != GDN_QUANT_AFFINE || biases), "gdn_dequantize: null weight, scales or biases");
     GDN_REQUIRE(mode != GDN_QUANT_AFFINE || valid_dtype(sb_dtype), "gdn_dequantize: bad scales/biases dtype");
-    const int64_t threads = int64_t(N) * ((K + 31) / 32);
-    GDN_REQUIRE(threads < (int64_t(1) << 31), "gdn_dequantize: %lld elements exceed the grid",
+    GDN_REQUIRE(int64_t(N) * ((K + 31) / 32) < (int64_t(1) << 31), "gdn_dequantize: %lld elements exceed the grid",
                 (long long)N * K);
+    // rows of at most 2^23 blocks: a grid dimension holds less than 2^32 threads
+    const int64_t blocks = (int64_t(N) * (K / 8) + 255) / 256, row = int64_t(1) << 23;
+    const dim3 grid(unsigned(blocks < row ? blocks : row), unsigned((blocks + row - 1) / row));
     auto kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 2>;
     switch (mode) {
         case GDN_QUANT_MXFP4: kernel = dequantize_scheme_kernel<GDN_QUANT_MXFP4, 4>; break;
@@ -1945,7 +1947,7 @@ extern "C" int gdn_dequantize(const void* w, const void* scales, const void* bia
             if (bits == 5) kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 5>;
             if (bits == 6) kernel = dequantize_scheme_kernel<GDN_QUANT_AFFINE, 6>;
     }
-    hipLaunchKernelGGL(kernel, dim3(unsigned((int64_t(N) * (K / 8) + 255) / 256)), dim3(256), 0, s,
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s,
                        static_cast<const uint32_t*>(w), scales, biases, sb_dtype, out, out_dtype, N, K, group_size,
                        reinterpret_cast<uintptr_t>(out) % 16 == 0);
     return check_launch("gdn_dequantize");

@@ -902,3 +902,20 @@ def test_float32_rows_outside_the_pieces_range_cost_a_bounded_multiple(gpu):
             best = min(best, start.elapsed_time(end))
         times.append(best)
     assert times[1] < 20 * times[0], times
+
+
+def test_dequantize_of_more_threads_than_a_grid_dimension_holds(gpu):
+    """2^35 2-bit codes, 8 a thread: 2^32 threads, the first count that one grid
+    dimension does not hold, checked in blocks over the whole output."""
+    N, K, gs = 1 << 20, 1 << 15, 128
+    if torch.cuda.mem_get_info(gpu)[0] < 100 << 30:
+        pytest.skip("needs 75 GB of device memory")
+    w = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 16), dtype=torch.int32, device=gpu)
+    s = torch.rand(N, K // gs, device=gpu).to(torch.bfloat16)
+    out = gdn.dequantize({"weight": w, "scales": s, "biases": s}, gdn.QuantScheme(2, gs), torch.bfloat16)
+    shifts = torch.arange(0, 32, 2, device=gpu, dtype=torch.int32)
+    for n0 in range(0, N, N // 64):
+        for n in (n0, n0 + N // 64 - 8):
+            q = ((w[n:n + 8, :, None] >> shifts) & 3).reshape(8, K).float()
+            sc = s[n:n + 8].float().repeat_interleave(gs, 1)
+            assert torch.equal(out[n:n + 8], (sc * q + sc).to(torch.bfloat16)), n
