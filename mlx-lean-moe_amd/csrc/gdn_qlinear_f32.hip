@@ -514,9 +514,12 @@ auto kernel_of(int tm) {
 }
 
 bool f32_sizes_ok(int64_t M, int64_t N, int64_t K, int group_size) {
-    // 32-bit lane offsets and grid sizes
-    return M <= (1 << 24) && N <= (1 << 24) && K <= (1 << 20) && (group_size == 32 || group_size == 64 || group_size == 128) &&
-           K % kBK == 0 && K % group_size == 0;
+    // 32-bit lane offsets; grids of less than 2^32 threads (256 a block): the
+    // preparation's rows and column blocks, the product's smallest tiles
+    constexpr int64_t kBlocks = 1 << 24;
+    return M <= kBlocks && N <= kBlocks && K <= (1 << 20) && M + (N + kFlagCols - 1) / kFlagCols < kBlocks &&
+           ((M + 31) / 32) * ((N + kBN - 1) / kBN) < kBlocks - 8 &&
+           (group_size == 32 || group_size == 64 || group_size == 128) && K % kBK == 0 && K % group_size == 0;
 }
 
 }  // namespace
@@ -538,7 +541,8 @@ extern "C" int gdn_quantized_matmul_f32(const float* x, const void* w, const voi
     GDN_REQUIRE(valid_dtype(sb_dtype), "%s: bad scales/biases dtype", fn);
     if (bits != 4 && bits != 8) return fail(GDN_EUNSUPPORTED, "%s: %d-bit weights (4 and 8 are implemented)", fn, bits);
     GDN_REQUIRE(f32_sizes_ok(M, N, K, group_size),
-                "%s: group_size must be 32, 64 or 128 and K=%d a multiple of 64 and of it", fn, K);
+                "%s: group_size must be 32, 64 or 128, K=%d a multiple of 64 and of it, and M=%d N=%d fit the grid", fn,
+                K, M, N);
     if (M == 0) return 0;
     GDN_REQUIRE(x && y, "%s: null x or y", fn);
     GDN_REQUIRE((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) |

@@ -194,3 +194,18 @@ def test_scheme_matmul_argument_checks():
     assert size(1, 96, 512) == 0               # 16 blocks of 32 k: too few to split
     assert size(1, 96, 2048) == 4 * 96 * 4     # 64 blocks: 4 splits of 16
     assert size(65, 2048, 4096) == 0 and size(1, 2048, 4080) == 0
+
+
+def test_float32_quantized_matmul_sizes_fit_its_grids():
+    """Sizes whose launches would need 2^32 threads or more are refused (size 0
+    and EINVAL) before anything is launched; the largest below are taken."""
+    lib = _lib.load()
+    size = lib.gdn_quantized_matmul_f32_workspace_size
+    assert size((1 << 24) - 2, 64, 64, 4, 64) > 0                 # 2^24 - 2 row blocks and one of 64 columns
+    assert size((1 << 24) - 1, 64, 64, 4, 64) == 0
+    assert size(1 << 24, 64, 64, 4, 64) == 0
+    assert size(1 << 15, 1 << 22, 64, 4, 64) == 0                 # 2^10 x 2^14 product tiles
+    assert size(1 << 14, 1 << 22, 64, 4, 64) > 0
+    one = ctypes.c_void_p(16)
+    assert lib.gdn_quantized_matmul_f32(one, one, one, one, _lib.GDN_BF16, one, None, 1 << 24, 64, 64, 4, 64, one,
+                                        1 << 40, None) == _lib.GDN_EINVAL
