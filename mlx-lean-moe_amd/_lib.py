@@ -16,7 +16,7 @@ import torch
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(HERE, "libgdn.so")
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 GDN_F32, GDN_BF16, GDN_F16 = 0, 1, 2
 GDN_EINVAL, GDN_EUNSUPPORTED = -1, -2
@@ -56,11 +56,19 @@ _SIGNATURES = {
                                      _c_int, _c_i64, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p,
                                      _c_void_p, _c_int, _c_void_p, _c_int, _c_i64, _c_int,
                                      _c_int, _c_int, _c_int, _c_void_p, _c_i64, _c_void_p]),
+    "gdn_prefill_chunked_runs": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p,
+                                          _c_int, _c_i64, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_void_p,
+                                          _c_void_p, _c_int, _c_void_p, _c_int, _c_i64, _c_int,
+                                          _c_int, _c_int, _c_int, _c_void_p, _c_i64, _c_i64, _c_void_p]),
     "gdn_prefill_fused_workspace_size": (_c_i64, [_c_int, _c_i64, _c_int, _c_int, _c_int, _c_int]),
     "gdn_prefill_fused": (_c_int, [_c_void_p, _c_i64, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int,
                                    _c_void_p, _c_void_p, _c_int, _c_i64, _c_void_p, _c_void_p,
                                    _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_i64,
                                    _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_i64, _c_void_p]),
+    "gdn_prefill_fused_runs": (_c_int, [_c_void_p, _c_i64, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int,
+                                        _c_void_p, _c_void_p, _c_int, _c_i64, _c_void_p, _c_void_p,
+                                        _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_i64,
+                                        _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_i64, _c_i64, _c_void_p]),
     "gdn_gated_rmsnorm": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_int, _c_i64, _c_int, _c_void_p, _c_float,
                                    _c_void_p, _c_int, _c_i64, _c_int, _c_void_p]),
     "gdn_quantized_matmul": (_c_int, [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_int,

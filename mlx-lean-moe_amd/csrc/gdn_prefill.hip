@@ -694,8 +694,8 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // (kUpper = false) fetch and multiply only their first 32 columns.
 constexpr int kStateThreads = 512;
 // A state-pass workgroup holds its CU to itself (256 registers a thread, the
-// prefetch ring three chunks deep), which suits a grid of one a CU: the chain
-// of chunk steps is all there is to hide. With more workgroups than CUs a
+// prefetch ring two or three chunks deep), which suits a grid of one a CU: the
+// chain of chunk steps is all there is to hide. With more workgroups than CUs a
 // second one on the CU hides more than the deep ring does: calls above 256
 // workgroups take prefill_state_shared_kernel (128 registers and 76-78 KB of
 // LDS, the same bits). Whole calls, us, one a CU against two, bf16: 3 runs of
@@ -704,7 +704,16 @@ constexpr int kStateThreads = 512;
 // 87 -> 52, 16 packed runs of 67 128 tokens in all at 32 heads 2232 -> 2054;
 // float32 in the same order 193 -> 171, 192 -> 172, 145 -> 131, 99 -> 84, and
 // 8 packed runs of 300 to 1000 tokens at 32 heads 315 -> 287.
-constexpr int kStateSharedAbove = 256;
+// Where one run is nearly all of the work (known only to a caller that has the
+// offsets on the host), its chain runs alone on the CU after the others' end
+// and the deep ring is the better again: from kStateLongRun tokens on, those of
+// a CU's share have to be 1.1 times the longest run's. 32 heads, one a CU against two, bf16 / float32:
+// 8192 + 64 tokens 296 and 312 / 459 and 501, 8192 + 3 x 64 302 and 314 / 473
+// and 507, 8192 + 15 x 64 (1.12 times) 378 and 346 / 543 and 537, 4096 + 512
+// (1.13) 169 and 164 / 264 and 263, 4096 + 2048 217 and 212 / 332 and 308, 4096
+// + 64 160 and 160 / 245 and 253, but 2048 + 64 111 and 108 / 156 and 156, 1000
+// + 64 81 and 78 / 105 and 103.
+constexpr int kStateSharedAbove = 256, kStateLongRun = 4096;
 
 // Chunk operands of state wave w, fetched by output wave w. They pass
 // through registers on the way to LDS, so each load covers whole rows (full
@@ -1416,12 +1425,18 @@ prefill_state_shared_kernel(GDN_STATE_ARGS) {
 }
 #undef GDN_STATE_ARGS
 
+// Whether the longest run (0: not known) is long and nearly all of a CU's share.
+bool one_run_dominates(int64_t T_total, int Hv, int64_t longest) {
+    return longest >= kStateLongRun && T_total * Hv * kSlices * 10 < longest * kStateSharedAbove * 11;
+}
+
 // The state pass over every (run, value head, slice).
 template <class Y, bool kF32>
 int launch_state(const void* q, const void* k, const void* v, const float* state_in, float* state_out, void* y,
-                 const RunLayout& rl, const char* records, int Hk, int Hv, hipStream_t s, const char* what) {
+                 const RunLayout& rl, const char* records, int Hk, int Hv, bool one_run, hipStream_t s,
+                 const char* what) {
     const int64_t wgs = int64_t(rl.N) * Hv * kSlices;
-    const auto kernel = wgs > kStateSharedAbove ? prefill_state_shared_kernel<Y, kF32> : prefill_state_kernel<Y, kF32>;
+    const auto kernel = wgs > kStateSharedAbove && !one_run ? prefill_state_shared_kernel<Y, kF32> : prefill_state_kernel<Y, kF32>;
     hipLaunchKernelGGL(kernel, dim3(unsigned(wgs)), dim3(kStateThreads), 0, s, q, k, v, state_in, state_out,
                        static_cast<typename Y::storage*>(y), rl, records, Hk, Hv);
     return check_launch(what);
@@ -1437,13 +1452,12 @@ extern "C" int64_t gdn_prefill_workspace_size(int N, int64_t T_total, int Hk, in
     return records_offset(N) + chunks_bound(T_total, N) * Hv * kRecBytes;
 }
 
-extern "C" int gdn_prefill_chunked(const void* q, const void* k, const void* v, int qkv_dtype, const void* ga,
-                                   const void* gb, int gb_dtype, int64_t gate_stride, const float* A_log,
-                                   const float* dt_bias, int gate_mode, const float* state_in,
-                                   float* state_out, void* y, int y_dtype,
-                                   const int32_t* cu_seqlens, int N, int64_t T_total, int Hk,
-                                   int Hv, int Dk, int Dv, void* workspace,
-                                   int64_t workspace_bytes, void* stream) {
+extern "C" int gdn_prefill_chunked_runs(const void* q, const void* k, const void* v, int qkv_dtype, const void* ga,
+                                        const void* gb, int gb_dtype, int64_t gate_stride, const float* A_log,
+                                        const float* dt_bias, int gate_mode, const float* state_in, float* state_out,
+                                        void* y, int y_dtype, const int32_t* cu_seqlens, int N, int64_t T_total,
+                                        int Hk, int Hv, int Dk, int Dv, void* workspace, int64_t workspace_bytes,
+                                        int64_t longest_run, void* stream) {
     GDN_REQUIRE(N > 0 && T_total >= 0 && Hk > 0 && Hv > 0 && Hv % Hk == 0,
                 "gdn_prefill_chunked: bad sizes");
     if (Dk != kHD || Dv != kHD)
@@ -1458,6 +1472,7 @@ extern "C" int gdn_prefill_chunked(const void* q, const void* k, const void* v, 
     GDN_REQUIRE(gate_mode == 1 || (A_log && dt_bias), "gdn_prefill_chunked: gate_mode 0 needs A_log, dt_bias");
     GDN_REQUIRE(cu_seqlens || T_total % N == 0, "gdn_prefill_chunked: T_total not divisible by N");
     GDN_REQUIRE(T_total < (int64_t(1) << 31), "gdn_prefill_chunked: token count must fit int32");
+    GDN_REQUIRE(longest_run >= 0 && longest_run <= T_total, "gdn_prefill_chunked: bad longest run");
     GDN_REQUIRE(state_out, "gdn_prefill_chunked: null state_out");
     GDN_REQUIRE(T_total == 0 || (q && k && v && ga && gb && y), "gdn_prefill_chunked: null pointer");
     GDN_REQUIRE((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
@@ -1502,7 +1517,8 @@ extern "C" int gdn_prefill_chunked(const void* q, const void* k, const void* v, 
                        gb_dtype, gate_stride, A_log, dt_bias, gate_mode, rl, records, Hk, Hv);
     if (int rc = check_launch("gdn_prefill_chunked/chunk")) return rc;
     const auto launch = [&](auto kernel) {
-        return kernel(q, k, v, state_in, state_out, y, rl, records, Hk, Hv, s, "gdn_prefill_chunked/state");
+        return kernel(q, k, v, state_in, state_out, y, rl, records, Hk, Hv,
+                      one_run_dominates(T_total, Hv, longest_run), s, "gdn_prefill_chunked/state");
     };
     if (f32) {
         if (y_dtype == GDN_F32) return launch(launch_state<ActF32, true>);
@@ -1512,6 +1528,16 @@ extern "C" int gdn_prefill_chunked(const void* q, const void* k, const void* v, 
     if (y_dtype == GDN_F32) return launch(launch_state<ActF32, false>);
     if (y_dtype == GDN_BF16) return launch(launch_state<ActBF16, false>);
     return launch(launch_state<ActF16, false>);
+}
+
+extern "C" int gdn_prefill_chunked(const void* q, const void* k, const void* v, int qkv_dtype, const void* ga,
+                                   const void* gb, int gb_dtype, int64_t gate_stride, const float* A_log,
+                                   const float* dt_bias, int gate_mode, const float* state_in, float* state_out,
+                                   void* y, int y_dtype, const int32_t* cu_seqlens, int N, int64_t T_total, int Hk,
+                                   int Hv, int Dk, int Dv, void* workspace, int64_t workspace_bytes, void* stream) {
+    return gdn_prefill_chunked_runs(q, k, v, qkv_dtype, ga, gb, gb_dtype, gate_stride, A_log, dt_bias, gate_mode,
+                                    state_in, state_out, y, y_dtype, cu_seqlens, N, T_total, Hk, Hv, Dk, Dv, workspace,
+                                    workspace_bytes, 0, stream);
 }
 
 namespace {
@@ -1531,13 +1557,13 @@ extern "C" int64_t gdn_prefill_fused_workspace_size(int N, int64_t T_total, int 
     return fused_qkv_offset(N, T_total, Hv) + T_total * (2LL * Hk + Hv) * kHD * 2;
 }
 
-extern "C" int gdn_prefill_fused(const void* qkv, int64_t qkv_stride, const void* conv_state_in,
-                                 void* conv_state_out, int conv_dtype, const float* conv_weight, int K,
-                                 const void* a, const void* b, int gate_dtype, int64_t gate_stride,
-                                 const float* A_log, const float* dt_bias, const float* state_in,
-                                 float* state_out, void* y, int y_dtype, const int32_t* cu_seqlens, int N,
-                                 int64_t T_total, int Hk, int Hv, int Dk, int Dv, void* workspace,
-                                 int64_t workspace_bytes, void* stream) {
+extern "C" int gdn_prefill_fused_runs(const void* qkv, int64_t qkv_stride, const void* conv_state_in,
+                                      void* conv_state_out, int conv_dtype, const float* conv_weight, int K,
+                                      const void* a, const void* b, int gate_dtype, int64_t gate_stride,
+                                      const float* A_log, const float* dt_bias, const float* state_in,
+                                      float* state_out, void* y, int y_dtype, const int32_t* cu_seqlens, int N,
+                                      int64_t T_total, int Hk, int Hv, int Dk, int Dv, void* workspace,
+                                      int64_t workspace_bytes, int64_t longest_run, void* stream) {
     GDN_REQUIRE(N > 0 && T_total >= 0 && Hk > 0 && Hv > 0 && Hv % Hk == 0, "gdn_prefill_fused: bad sizes");
     if (Dk != kHD || Dv != kHD || K != 4)
         return fail(GDN_EUNSUPPORTED, "gdn_prefill_fused: specialised for Dk=Dv=128, K=4 (got %d, %d, %d)",
@@ -1549,6 +1575,7 @@ extern "C" int gdn_prefill_fused(const void* qkv, int64_t qkv_stride, const void
                 Hv);
     GDN_REQUIRE(cu_seqlens || T_total % N == 0, "gdn_prefill_fused: T_total not divisible by N");
     GDN_REQUIRE(T_total < (int64_t(1) << 31), "gdn_prefill_fused: token count must fit int32");
+    GDN_REQUIRE(longest_run >= 0 && longest_run <= T_total, "gdn_prefill_fused: bad longest run");
     const int64_t C = (2LL * Hk + Hv) * kHD;
     GDN_REQUIRE(qkv_stride >= C && qkv_stride % 8 == 0,
                 "gdn_prefill_fused: qkv_stride %lld must be at least conv_dim %lld and a multiple of 8",
@@ -1616,9 +1643,22 @@ extern "C" int gdn_prefill_fused(const void* qkv, int64_t qkv_stride, const void
         if (int rc = check_launch("gdn_prefill_fused/conv_state")) return rc;
     }
     const auto launch = [&](auto kernel) {
-        return kernel(cv.qo, cv.ko, cv.vo, state_in, state_out, y, rl, records, Hk, Hv, s, "gdn_prefill_fused/state");
+        return kernel(cv.qo, cv.ko, cv.vo, state_in, state_out, y, rl, records, Hk, Hv,
+                      one_run_dominates(T_total, Hv, longest_run), s, "gdn_prefill_fused/state");
     };
     if (y_dtype == GDN_F32) return launch(launch_state<ActF32, false>);
     if (y_dtype == GDN_BF16) return launch(launch_state<ActBF16, false>);
     return launch(launch_state<ActF16, false>);
+}
+
+extern "C" int gdn_prefill_fused(const void* qkv, int64_t qkv_stride, const void* conv_state_in,
+                                 void* conv_state_out, int conv_dtype, const float* conv_weight, int K,
+                                 const void* a, const void* b, int gate_dtype, int64_t gate_stride,
+                                 const float* A_log, const float* dt_bias, const float* state_in,
+                                 float* state_out, void* y, int y_dtype, const int32_t* cu_seqlens, int N,
+                                 int64_t T_total, int Hk, int Hv, int Dk, int Dv, void* workspace,
+                                 int64_t workspace_bytes, void* stream) {
+    return gdn_prefill_fused_runs(qkv, qkv_stride, conv_state_in, conv_state_out, conv_dtype, conv_weight, K, a, b,
+                                  gate_dtype, gate_stride, A_log, dt_bias, state_in, state_out, y, y_dtype,
+                                  cu_seqlens, N, T_total, Hk, Hv, Dk, Dv, workspace, workspace_bytes, 0, stream);
 }

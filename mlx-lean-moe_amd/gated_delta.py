@@ -169,17 +169,30 @@ def prefill_workspace_bytes(N: int, T: int, Hk: int, Hv: int, Dk: int, Dv: int) 
 
 
 def _launch_prefill(q, k, v, ga, gb, A_log, dt_bias, gate_mode, state_in, state_out, y, cu, N, T,
-                    Hk, Hv, Dk, Dv, device, workspace=None, gate_stride=None):
+                    Hk, Hv, Dk, Dv, device, workspace=None, gate_stride=None, longest=0):
     nbytes = prefill_workspace_bytes(N, T, Hk, Hv, Dk, Dv)
     if workspace is None or workspace.numel() < nbytes:
         workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    _lib.call("gdn_prefill_chunked", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v),
+    name, hint = _with_longest("gdn_prefill_chunked", T, longest)
+    _lib.call(name, _lib.ptr(q), _lib.ptr(k), _lib.ptr(v),
               _lib.dtype_code(q.dtype), _lib.ptr(ga),
               _lib.ptr(gb), _lib.dtype_code(gb.dtype), Hv if gate_stride is None else gate_stride,
               _lib.ptr(A_log), _lib.ptr(dt_bias),
               gate_mode, _lib.ptr(state_in), _lib.ptr(state_out), _lib.ptr(y),
               _lib.dtype_code(y.dtype), _lib.ptr(cu), N, T, Hk, Hv, Dk, Dv,
-              _lib.ptr(workspace), workspace.numel(), _stream(device))
+              _lib.ptr(workspace), workspace.numel(), *hint, _stream(device))
+
+
+def _longest_run(offsets: list[int]) -> int:
+    return max(b - a for a, b in zip(offsets, offsets[1:]))
+
+
+def _with_longest(name: str, T: int, longest: int) -> tuple[str, tuple]:
+    """A prefill entry point and its hint: packed runs of which one holds most
+    of the tokens are handed over with its length (the library has the offsets
+    on the device only)."""
+
+    return (name + "_runs", (longest,)) if 2 * longest > T else (name, ())
 
 
 def _prefill_eligible(q, k, v, tokens_per_run: float) -> bool:
@@ -335,7 +348,8 @@ def gated_delta_update(q, k, v, a, b, A_log, dt_bias, state=None, *, cu_seqlens=
             if not rows_ok:
                 a, b = _c(a), _c(b)
             _launch_prefill(q, k, v, a, b, _c(A_log.float()), _c(dt_bias.float()), 0, state_in,
-                            state_out, y, cu, N, T, Hk, Hv, Dk, Dv, device, gate_stride=a.stride(0))
+                            state_out, y, cu, N, T, Hk, Hv, Dk, Dv, device, gate_stride=a.stride(0),
+                            longest=_longest_run(offsets) if packed and N > 1 else 0)
         else:
             g, beta = _gates(_c(a), _c(b), A_log, dt_bias)
             name = "gdn_scan" if use_kernel and Dk in (32, 64, 128, 256) else "gdn_scan_reference"

@@ -29,8 +29,8 @@ import torch
 
 from . import _lib
 from .config import LinearAttentionDims
-from .gated_delta import (PREFILL_MIN_TOKENS, _as, _c, _check_cu_seqlens, _check_out, _require_device,
-                          _stream, gated_delta_update)
+from .gated_delta import (PREFILL_MIN_TOKENS, _as, _c, _check_cu_seqlens, _check_out, _longest_run,
+                          _require_device, _stream, _with_longest, gated_delta_update)
 from .quant import (LinearWeights, QuantScheme, concat_quantized, quantized_linear,
                     quantized_linear_split)
 from .recurrent_cache import RecurrentCache, RecurrentStatePool
@@ -87,7 +87,7 @@ def conv_frontend(qkv: torch.Tensor, conv_state: torch.Tensor, conv_weight: torc
     K = dims.conv_kernel_dim
     if C != dims.conv_dim or tuple(conv_state.shape[1:]) != (K - 1, C):
         raise ValueError("qkv/conv_state do not match the layer's conv_dim and kernel")
-    cu_seqlens = _runs_on_device(cu_seqlens, N, T, device)
+    cu_seqlens, _ = _runs_on_device(cu_seqlens, N, T, device)
     act = qkv.dtype
     if act not in (torch.float32, torch.bfloat16):
         raise ValueError(f"activations must be float32 or bfloat16, got {act}")
@@ -163,7 +163,7 @@ def prefill_fused(qkv, a, b, conv_state, ssm_state, conv_weight, A_log, dt_bias,
         raise ValueError("prefill_fused needs bf16 activations, Dk = Dv = 128, K = 4, a bf16 or "
                          "float32 conv state, a float32 ssm state and runs of at least "
                          f"{PREFILL_MIN_TOKENS} tokens on average")
-    cu = _runs_on_device(cu_seqlens, N, T, device)
+    cu, longest = _runs_on_device(cu_seqlens, N, T, device)
     if not (qkv.stride(1) == 1 and qkv.stride(0) >= C and qkv.stride(0) % 8 == 0
             and qkv.data_ptr() % 16 == 0):
         qkv = qkv.contiguous()
@@ -184,31 +184,33 @@ def prefill_fused(qkv, a, b, conv_state, ssm_state, conv_weight, A_log, dt_bias,
     if nbytes < 0:
         raise RuntimeError("gdn_prefill_fused_workspace_size: " + _lib.load().gdn_last_error().decode())
     workspace = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
-    _lib.call("gdn_prefill_fused", _lib.ptr(qkv), qkv.stride(0), _lib.ptr(conv_state),
+    name, hint = _with_longest("gdn_prefill_fused", T, longest)
+    _lib.call(name, _lib.ptr(qkv), qkv.stride(0), _lib.ptr(conv_state),
               _lib.ptr(conv_out), _lib.dtype_code(conv_state.dtype), _lib.ptr(w), K, _lib.ptr(a),
               _lib.ptr(b), _lib.dtype_code(a.dtype), a.stride(0), _lib.ptr(_c(A_log.float())),
               _lib.ptr(_c(dt_bias.float())), _lib.ptr(ssm_in), _lib.ptr(state_out), _lib.ptr(y),
               _lib.dtype_code(y.dtype), _lib.ptr(cu), N, T, Hk, Hv, D, D, _lib.ptr(workspace),
-              workspace.numel(), _stream(device))
+              workspace.numel(), *hint, _stream(device))
     return y, conv_out, state_out
 
 
-def _runs_on_device(cu_seqlens, N: int, T: int, device) -> torch.Tensor | None:
+def _runs_on_device(cu_seqlens, N: int, T: int, device) -> tuple[torch.Tensor | None, int]:
     """Checked run offsets as an int32 device tensor (None: N equal runs,
-    T a multiple of N)."""
+    T a multiple of N), and the longest of several runs (else 0)."""
 
     if cu_seqlens is None:
         if N <= 0 or T % N:
             raise ValueError(f"{T} tokens do not split into {N} equal runs; pass cu_seqlens")
-        return None
+        return None, 0
     offsets = _check_cu_seqlens(cu_seqlens, T)
     if len(offsets) != N + 1:
         raise ValueError(f"cu_seqlens must hold {N + 1} offsets (one more than the "
                          f"{N} conv states), got {len(offsets)}")
+    longest = _longest_run(offsets) if N > 1 else 0
     if (isinstance(cu_seqlens, torch.Tensor) and cu_seqlens.device == device
             and cu_seqlens.dtype == torch.int32 and cu_seqlens.is_contiguous()):
-        return cu_seqlens
-    return torch.tensor(offsets, dtype=torch.int32).to(device)
+        return cu_seqlens, longest
+    return torch.tensor(offsets, dtype=torch.int32).to(device), longest
 
 
 def _fused_decode_ok(dims: LinearAttentionDims, act: torch.dtype) -> bool:

@@ -13,7 +13,7 @@ import pytest
 import torch
 
 import mlx_lean_moe_amd as gdn
-from mlx_lean_moe_amd import gated_delta
+from mlx_lean_moe_amd import _lib, gated_delta
 from oracle import cref
 from oracle import gated_delta_ref as R
 from tests.helpers import max_rel
@@ -427,3 +427,31 @@ def test_prefill_runs_sharing_a_cu_equal_each_run_alone(gpu, lens, dtype):
                 assert torch.equal(y[o], y1) and torch.equal(s[r], s1[0]), (r, n)
             elif n == 0:
                 assert torch.equal(s[r], state[r])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("lens,Hv", [([4100, 64], 32), ([65, 1, 4200, 64], 16), ([5000] + [64] * 3, 16)])
+def test_runs_with_one_long_one_take_the_deep_prefetch_with_the_same_bits(gpu, dtype, lens, Hv, monkeypatch):
+    """Packed runs of which one is nearly all of the work: gated_delta_update
+    hands the library that run's length, which chooses the state pass of one
+    workgroup a CU where the run count alone (no length given) chooses the
+    shared one; the two give the same bits."""
+    rng = np.random.default_rng(sum(lens))
+    T, N, Hk = sum(lens), len(lens), 16
+    f = lambda *s: torch.tensor(rng.standard_normal(s), dtype=torch.float32, device=gpu)
+    unit = lambda t: t / t.norm(dim=-1, keepdim=True)
+    q, k, v = (unit(f(T, Hk, 128)) * 128 ** -0.5).to(dtype), unit(f(T, Hk, 128)).to(dtype), f(T, Hv, 128).to(dtype)
+    a, b = f(T, Hv).to(dtype), f(T, Hv).to(dtype)
+    A_log, dt_bias = f(Hv).abs(), f(Hv)
+    state = f(N, Hv, 128, 128) * 0.05
+    cu = [0] + np.cumsum(lens).tolist()
+    assert N * Hv * 8 > 256
+    names = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *args: (names.append((name, args[-2])), call(name, *args))[1])
+    y, s = gated_delta.gated_delta_update(q, k, v, a, b, A_log, dt_bias, state, cu_seqlens=cu)
+    assert names == [("gdn_prefill_chunked_runs", max(lens))]
+    monkeypatch.setattr(gated_delta, "_longest_run", lambda offsets: 0)
+    y0, s0 = gated_delta.gated_delta_update(q, k, v, a, b, A_log, dt_bias, state, cu_seqlens=cu)
+    assert names[1][0] == "gdn_prefill_chunked"
+    assert torch.equal(y, y0) and torch.equal(s, s0)

@@ -123,3 +123,23 @@ def test_layer_prompt_path_takes_the_fused_call(gpu, monkeypatch):
     out_ref = linear_attention.gated_rms_norm(y_ref, z, norm_w, 1e-6, out_dtype=z.dtype)
     assert torch.equal(out, out_ref.reshape(512, d.value_dim))
     assert torch.equal(conv, conv_ref) and torch.equal(ssm, ssm_ref)
+
+
+def test_fused_prefill_of_one_long_run_and_short_ones_gives_the_same_bits(gpu, monkeypatch):
+    """Runs of which one is nearly all of the work go to gdn_prefill_fused_runs
+    with that run's length (the state pass of one workgroup a CU); without it,
+    and through the unfused pair, the bits are the same."""
+    lens = [64, 4500, 1, 100]
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32), device=gpu)
+    c = _case(gpu, 3, sum(lens), len(lens), 16, 16)
+    args = (c["qkv"], c["a"], c["b"], c["conv"], c["ssm"], c["w"], c["A_log"], c["dt_bias"], c["dims"], cu)
+    names = []
+    call = gdn._lib.call
+    monkeypatch.setattr(gdn._lib, "call", lambda name, *a: (names.append(name), call(name, *a))[1])
+    told = gdn.prefill_fused(*args, y_dtype=torch.bfloat16)
+    monkeypatch.setattr(gdn.linear_attention, "_longest_run", lambda offsets: 0)
+    untold = gdn.prefill_fused(*args, y_dtype=torch.bfloat16)
+    assert names == ["gdn_prefill_fused_runs", "gdn_prefill_fused"]
+    y, conv, ssm = _unfused(c, cu, torch.bfloat16)
+    for got in (told, untold):
+        assert torch.equal(got[0], y) and torch.equal(got[1], conv) and torch.equal(got[2], ssm)
