@@ -425,7 +425,12 @@ def test_prefill_runs_sharing_a_cu_equal_each_run_alone(gpu, lens, dtype):
                 y1, s1 = gated_delta.gated_delta_update(q[o], k[o], v[o], a[o], b[o], A_log, dt, state[r:r + 1],
                                                cu_seqlens=[0, n], y_dtype=y_dtype)
                 assert torch.equal(y[o], y1) and torch.equal(s[r], s1[0]), (r, n)
-            elif n == 0:
+            elif n:  # alone gated_delta_update would scan it: the chunked launch directly
+                y1, s1 = torch.empty_like(y[o]), torch.empty_like(state[r:r + 1])
+                gated_delta._launch_prefill(q[o], k[o], v[o], a[o], b[o], A_log, dt, 0, state[r:r + 1], s1, y1, None,
+                                            1, n, Hk, Hv, 128, 128, gpu)
+                assert torch.equal(y[o], y1) and torch.equal(s[r], s1[0]), (r, n)
+            else:
                 assert torch.equal(s[r], state[r])
 
 

@@ -41,8 +41,8 @@ def _decode_kernel_takes(M, K, bits, gs, sb):
     (64, 12352, 2048, 4, 64, "bf16"),   # the layer's stacked input projection at decode
     (33, 2048, 4096, 4, 64, "bf16"),    # out_proj at decode (value_dim 4096 -> hidden)
     (5, 70, 1024, 8, 32, "f16"),
-    (200, 130, 512, 8, 128, "f32"),
-    (300, 2048, 1024, 4, 64, "bf16"),   # large-M tiles, partial edge tiles
+    (200, 130, 512, 8, 128, "f32"),     # quantized_linear: dense; the ABI: the kernel for 65-511 rows
+    (300, 2048, 1024, 4, 64, "bf16"),   # the same, ragged last row tile
     (2, 78, 256, 4, 64, "bf16"),        # decode kernel: 4 groups per column, last block partial
     (3, 77, 256, 4, 64, "bf16"),        # scales span not whole 16-byte pieces: tiled kernel
     (16, 200, 1024, 4, 32, "f32"),      # decode kernel with float32 scales
@@ -325,8 +325,8 @@ def test_layer_with_quantized_projections_matches_dense_weights(gpu, T):
     (1, 2048, 4096, 64, "bf16"),      # the one-row matrix-vector kernel
     (16, 2048, 4096, 64, "bf16"),     # decode kernel, K split (sum kernel stores)
     (32, 12352, 2048, 64, "f32"),     # decode kernel, float32 x and result
-    (100, 300, 512, 64, "bf16"),      # tiled kernel
-    (600, 256, 512, 64, "bf16"),      # quantized_linear: dequantize + BLAS, then the add
+    (100, 300, 512, 64, "bf16"),      # dequantize + BLAS, then the add
+    (600, 256, 512, 64, "bf16"),      # the same
 ])
 def test_residual_is_the_unfused_add(gpu, M, N, K, gs, dt):
     """residual + x W^T, the product rounded to the result dtype first: bit
@@ -634,7 +634,7 @@ def test_rows_above_the_decode_sizes(gpu, M, N, K, bits, gs, sb):
     assert nbytes > 0 or N != 2048
     for ws in (None, torch.empty(nbytes, dtype=torch.uint8, device=gpu) if nbytes else None):
         y = torch.empty(M, N, device=gpu)
-        _lib.call("gdn_quantized_matmul", _lib.ptr(xt), _lib.GDN_BF16, _lib.ptr(W["weight"]), _lib.ptr(W["scales"]),
+        _lib.call("gdn_quantized_matmul_rows", _lib.ptr(xt), _lib.GDN_BF16, _lib.ptr(W["weight"]), _lib.ptr(W["scales"]),
                   _lib.ptr(W["biases"]), _lib.dtype_code(W["scales"].dtype), _lib.ptr(y), _lib.GDN_F32, None, M, N, K,
                   bits, gs, _lib.ptr(ws), nbytes if ws is not None else 0, _lib.stream_ptr(xt.device))
         assert (np.abs(y.cpu().numpy() - ref) <= bound).all()
@@ -919,3 +919,58 @@ def test_dequantize_of_more_threads_than_a_grid_dimension_holds(gpu):
             q = ((w[n:n + 8, :, None] >> shifts) & 3).reshape(8, K).float()
             sc = s[n:n + 8].float().repeat_interleave(gs, 1)
             assert torch.equal(out[n:n + 8], (sc * q + sc).to(torch.bfloat16)), n
+
+
+@pytest.mark.parametrize("M,N,K,bits,gs,sb", [
+    # the 128 x 128 tiles: K not in steps of 256 (quantized_linear sends N >= 4096 there)
+    (100, 300, 320, 4, 64, "bf16"),
+    (130, 4100, 320, 8, 64, "f32"),
+    (129, 4160, 1088, 4, 32, "f16"),
+    (511, 4097, 192, 8, 32, "bf16"),
+    # the same where the 112-row tiles would need a second round of workgroups
+    (256, 12352, 256, 4, 64, "bf16"),
+    (385, 12352, 512, 8, 128, "bf16"),
+    (449, 12352, 1024, 8, 32, "bf16"),
+    # the 112-row tiles, up to their last row count; two rounds of them
+    (225, 1000, 512, 4, 64, "bf16"),
+    (300, 4096, 256, 8, 32, "f16"),
+    (511, 700, 768, 8, 128, "f32"),
+    (300, 12352, 1024, 4, 128, "bf16"),
+    # K split over the grid
+    (448, 2048, 4096, 4, 64, "bf16"),
+    (511, 1000, 4096, 8, 64, "f16"),
+])
+def test_every_kernel_of_65_to_511_rows(gpu, M, N, K, bits, gs, sb):
+    """x times the bf16-rounded weights, whichever kernel takes the rows: the
+    float32 result within K + 20 roundings of the magnitudes added, a float16 and
+    a bfloat16 one with a residual in y itself as the unfused add of the rounded
+    product, and quantized_linear's with the residual bit for bit that add."""
+    rng = np.random.default_rng(M + N + K)
+    words, s, b = _weights(rng, N, K, bits, gs, sb)
+    W = _dev_weights(gpu, words, s, b, sb)
+    x = R.bf16_round(rng.standard_normal((M, K)))
+    xt = torch.tensor(x, dtype=torch.float32, device=gpu).to(torch.bfloat16)
+    w = torch.tensor(Q.dequantize(words, s, b, bits, gs, out="bf16"), dtype=torch.float64, device=gpu)
+    ref = xt.double() @ w.T
+    bound = (K + 20) * 2.0 ** -24 * (xt.double().abs() @ w.abs().T)
+    lib = _lib.load()
+    nbytes = lib.gdn_quantized_matmul_rows_workspace_size(_lib.dtype_code(_TORCH[sb]), M, N, K, bits, gs)
+    ws = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=gpu)
+
+    def run(y, residual=None):
+        _lib.call("gdn_quantized_matmul_rows", _lib.ptr(xt), _lib.GDN_BF16, _lib.ptr(W["weight"]),
+                  _lib.ptr(W["scales"]), _lib.ptr(W["biases"]), _lib.dtype_code(_TORCH[sb]), _lib.ptr(y),
+                  _lib.dtype_code(y.dtype), _lib.ptr(residual), M, N, K, bits, gs, _lib.ptr(ws), nbytes,
+                  _lib.stream_ptr(gpu))
+        return y
+
+    y32 = run(torch.empty(M, N, device=gpu))
+    assert ((y32.double() - ref).abs() <= bound).all()
+    for dt in (torch.float16, torch.bfloat16):
+        r = torch.randn(M, N, device=gpu).to(dt)
+        y = r.clone()
+        assert torch.equal(run(y, y), y32.to(dt) + r)
+    q = gdn.QuantScheme(bits, gs)
+    y = gdn.quantized_linear(xt, W, q)
+    assert ((y.double() - ref).abs() <= bound + 2.0 ** -8 * ref.abs()).all()
+    assert torch.equal(gdn.quantized_linear(xt, W, q, residual=r), y + r)

@@ -159,8 +159,9 @@ def test_dense_path_choice_follows_the_measured_crossovers():
     from mlx_lean_moe_amd.quant import _dense_rows
 
     assert not _dense_rows(64, 2048, 4096)       # decode sizes: quantized kernels
+    # where the kernel for 65-511 rows does not take the shape, or a copy is kept
     assert _dense_rows(65, 2048, 4096)           # out_proj above 64 rows: dense
-    assert not _dense_rows(300, 12352, 2048)     # the stacked input projection: tiled kernel
+    assert not _dense_rows(300, 12352, 2048)     # the stacked input projection: quantized kernels
     assert _dense_rows(512, 12352, 2048)         # prefill sizes: dense for every shape
     assert _dense_rows(200, 12352, 4096)         # deep weights
     assert _dense_rows(100, 300, 512)            # narrow weights
