@@ -684,12 +684,13 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // recurrence (S K^T -> R -> Tb R -> state update) and touch only LDS and
 // their accumulators. Waves 4-7 compute the output (Q S^T, P D, y) and fetch
 // every chunk operand from global memory for both halves: those of the
-// state waves (K, V, Tb, the decay factors) two chunks ahead into registers,
-// then into LDS one chunk ahead, and their own Q rows, straight into MFMA
-// A fragments two chunks ahead. Issuing the loads is what the state
-// recurrence cannot afford (the vector-memory queue stalls the issuing
-// wave); the output waves have slack. Both halves meet at the same three
-// barriers per chunk. Output wave w fetches the rows state wave w consumes;
+// state waves (K, V, Tb, the decay factors) into registers, three chunks ahead
+// with bf16 input and two with float32 (one, or phases, where two workgroups
+// share the CU), then into LDS one chunk ahead, and their own Q rows, straight
+// into MFMA A fragments. Issuing the loads is what the state recurrence cannot
+// afford (the vector-memory queue stalls the issuing wave); the output waves
+// have slack. Both halves meet at the same three barriers per chunk (four where
+// a single K tile is held). Output wave w fetches the rows state wave w consumes;
 // Tb and P are lower triangular, so the waves of token rows 0-31
 // (kUpper = false) fetch and multiply only their first 32 columns.
 constexpr int kStateThreads = 512;
@@ -707,12 +708,12 @@ constexpr int kStateThreads = 512;
 // Where one run is nearly all of the work (known only to a caller that has the
 // offsets on the host), its chain runs alone on the CU after the others' end
 // and the deep ring is the better again: from kStateLongRun tokens on, those of
-// a CU's share have to be 1.1 times the longest run's. 32 heads, one a CU against two, bf16 / float32:
-// 8192 + 64 tokens 296 and 312 / 459 and 501, 8192 + 3 x 64 302 and 314 / 473
-// and 507, 8192 + 15 x 64 (1.12 times) 378 and 346 / 543 and 537, 4096 + 512
-// (1.13) 169 and 164 / 264 and 263, 4096 + 2048 217 and 212 / 332 and 308, 4096
-// + 64 160 and 160 / 245 and 253, but 2048 + 64 111 and 108 / 156 and 156, 1000
-// + 64 81 and 78 / 105 and 103.
+// a CU's share have to be 1.1 times the longest run's. 32 heads, one a CU
+// against two, bf16 / float32: 8192 + 64 tokens 296 and 312 / 459 and 501, 8192 +
+// 3 x 64 302 and 314 / 473 and 507, 8192 + 15 x 64 (1.12 times) 378 and 346 / 543
+// and 537, 4096 + 512 (1.13) 169 and 164 / 264 and 263, 4096 + 2048 217 and 212 /
+// 332 and 308, 4096 + 64 160 and 160 / 245 and 253, but 2048 + 64 111 and 108 /
+// 156 and 156, 1000 + 64 81 and 78 / 105 and 103.
 constexpr int kStateSharedAbove = 256, kStateLongRun = 4096;
 
 // Chunk operands of state wave w, fetched by output wave w. They pass
@@ -1129,8 +1130,9 @@ GDN_DEV void output_store(const OutputOperands& op, f32x4 yacc, const StatePassL
     }
 }
 
-// Chunk c: [S] B1 [R | Q S^T] B2 [D | Q, K, V(c+1), fetch c+2] B3
-// [update | Tb(c+1), y]. Both loops are straight-line code (wave-uniform
+// Chunk c: [S] B1 [R | Q S^T] B2 [D | K, V(c+1), fetches] B3 [update | Tb(c+1),
+// y]; with a single K tile [R | Q S^T, fetches] B2 [D | ] B3 [update | Tb(c+1),
+// y] B4 [ | K, V(c+1)]. Both loops are straight-line code (wave-uniform
 // roles), so the compiler's waits for loaded operands are exact and never
 // cover a later prefetch; both steps of the unrolled body are unconditional
 // (an odd last chunk runs after the loop), because a conditional second step

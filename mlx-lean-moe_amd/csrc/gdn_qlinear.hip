@@ -1388,16 +1388,9 @@ extern "C" int gdn_quantized_matmul_noalloc(const void* x, int x_dtype, const vo
 namespace gdn {
 namespace {
 
-// The microscaling float codes (OCP MX formats): e2m1 (fp4: sign, 2-bit
-// exponent of bias 1, 1-bit mantissa; exponent 0 is 0 or 0.5), e4m3 (fp8:
-// sign, 4-bit exponent of bias 7, 3-bit mantissa; exponent 0 subnormal,
-// 0x7F / 0xFF NaN) and e8m0 (a power of two, 2^(c - 127); 255 NaN).
-GDN_DEV float e2m1_value(uint32_t c) {
-    const int e = int(c >> 1) & 3;
-    const float mag = e == 0 ? 0.5f * float(c & 1) : ldexpf(1.f + 0.5f * float(c & 1), e - 1);
-    return (c & 8) ? -mag : mag;
-}
-
+// The microscaling float formats' scale codes (OCP MX): e4m3 (fp8: sign, 4-bit
+// exponent of bias 7, 3-bit mantissa; exponent 0 subnormal, 0x7F / 0xFF NaN)
+// and e8m0 (a power of two, 2^(c - 127); 255 NaN).
 GDN_DEV float e4m3_value(uint32_t c) {
     const int e = int(c >> 3) & 15, m = int(c & 7);
     if (e == 15 && m == 7) return __builtin_nanf("");

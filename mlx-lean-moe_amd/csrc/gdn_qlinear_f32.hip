@@ -236,8 +236,8 @@ GDN_DEV void float_rows(const float* __restrict__ x, const uint32_t* __restrict_
 // workgroup. A step is 64 k: x's pieces through two LDS tiles (one barrier a
 // step), the next step's pieces, codes and scales in registers meanwhile. Two
 // workgroups share a CU (256 registers a thread). At 777 rows, 2048 -> 12352,
-// the matrix cores are busy half the time (118 TFLOP of bf16 products against
-// 2.1 PFLOP/s: 58 us of 125): with two waves on a SIMD a wave's LDS reads,
+// the matrix cores are busy half the time (118 GFLOP of bf16 products against
+// 2.1 PFLOP/s: 56 us of 125): with two waves on a SIMD a wave's LDS reads,
 // conversions and scaling are not all covered. A wave in its MFMAs goes before
 // one that loads or converts (131 us without). Fetching the codes two steps
 // ahead, or the next row tile's fragments, spilled or gained nothing. One c for
