@@ -55,34 +55,52 @@ GDN_DEV f32x4 mfma_bf16(bf16x8 a, bf16x8 b, f32x4 c) {
 constexpr float kRowMax = 0x1p80f, kRowMin = 0x1p-90f;
 constexpr float kScaleMax = 0x1p16f, kBiasMax = 0x1p24f;
 constexpr int kFlagCols = 64;
+constexpr int kFlagGroups = 32;  // quantization groups of a column flag
+__host__ __device__ constexpr int flag_chunks(int groups) { return (groups + kFlagGroups - 1) / kFlagGroups; }
 __host__ __device__ constexpr int64_t padded_columns(int64_t n) { return (n + kBN - 1) / kBN * kBN; }
 
 // Blocks 0 .. M - 1: row m of x as bf16 pieces, pieces[m][step][part][64]
 // (part 0 the upper 8 significant bits; truncation, so no piece can round up
 // to infinity), its group sums (in double, rounded once) and its flag. The
-// blocks after them, 64 columns each: s, b (o_t) and b' = b + c s in float32,
-// group-major, c as a byte (c_t[group][64-column block][n % 16][n / 16 % 4]: a
-// word for the four columns of a lane of the product) and the columns' flag (at
-// flags[M + block]). The rows of s, b and c have padded_columns(N) columns; those
-// past N are read for outputs that are not stored.
+// blocks after them, 64 columns by 32 groups each (a thread 8 consecutive ones
+// of a column, all loads in flight: a thread walking all of its column's groups
+// took 18 us for 128 rows and 1024 columns of 128 groups, this 8): s, b (o_t) and b' = b + c s in
+// float32, group-major, c as a byte (c_t[group][64-column block][n % 16][n / 16
+// % 4]: a word for the four columns of a lane of the product) and the flag (at
+// flags[M + column block * chunks + chunk]). The rows of s, b and c have
+// padded_columns(N) columns; those past N are read for outputs that are not
+// stored.
+template <class SB>
 __global__ __launch_bounds__(256) void prepare_f32_kernel(
-    const float* __restrict__ x, const void* __restrict__ scales, const void* __restrict__ biases, int sb_dtype,
-    uint16_t* __restrict__ pieces, float* __restrict__ xsum, int* __restrict__ flags, float* __restrict__ s_t,
-    float* __restrict__ b_t, float* __restrict__ o_t, uint8_t* __restrict__ c_t, int M, int N, int K,
-    int group_size) {
+    const float* __restrict__ x, const typename SB::storage* __restrict__ scales,
+    const typename SB::storage* __restrict__ biases, uint16_t* __restrict__ pieces, float* __restrict__ xsum,
+    int* __restrict__ flags, float* __restrict__ s_t, float* __restrict__ b_t, float* __restrict__ o_t,
+    uint8_t* __restrict__ c_t, int M, int N, int K, int group_size) {
     const int G = K / group_size;
     if (int(blockIdx.x) >= M) {
-        const int block = int(blockIdx.x) - M, lane = threadIdx.x & 63;
+        constexpr int kPer = kFlagGroups / 4;  // groups of a thread
+        const int at = int(blockIdx.x) - M, block = at / flag_chunks(G), lane = threadIdx.x & 63;
+        const int g0 = at % flag_chunks(G) * kFlagGroups + int(threadIdx.x >> 6) * kPer;
         const int64_t stride = padded_columns(N), n = int64_t(block) * kFlagCols + lane;
+        const int64_t row = (n < N ? n : N - 1) * G;
+        float s[kPer], b[kPer];
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int g = g0 + i < G ? g0 + i : G - 1;
+            s[i] = SB::load(scales, row + g);
+            b[i] = SB::load(biases, row + g);
+        }
         bool far = false;
-        for (int g = threadIdx.x >> 6; g < G && n < N; g += 4) {
-            const float s = load_any(scales, n * G + g, sb_dtype), b = load_any(biases, n * G + g, sb_dtype);
-            far |= !(fabsf(s) < kScaleMax && fabsf(b) < kBiasMax);
-            const float c = fminf(fmaxf(rintf(-b / s), 0.f), 255.f);  // s = 0: any, b' = b
-            s_t[g * stride + n] = s;
-            o_t[g * stride + n] = b;
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+            const int64_t g = g0 + i;
+            if (n >= N || g >= G) continue;
+            far |= !(fabsf(s[i]) < kScaleMax && fabsf(b[i]) < kBiasMax);
+            const float c = fminf(fmaxf(rintf(-b[i] / s[i]), 0.f), 255.f);  // s = 0: any, b' = b
+            s_t[g * stride + n] = s[i];
+            o_t[g * stride + n] = b[i];
             c_t[g * stride + block * kFlagCols + (lane % 16) * 4 + lane / 16] = uint8_t(c);
-            b_t[int64_t(g) * N + n] = __builtin_fmaf(c, s, b);
+            b_t[g * N + n] = __builtin_fmaf(c, s[i], b[i]);
         }
         far = __syncthreads_or(far);
         if (threadIdx.x == 0) flags[blockIdx.x] = far;
@@ -422,12 +440,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void q
 
     // flagged rows, and the wave's own 64 columns when flagged, are left to
     // float_rows below
-    const int col0 = n0 / kFlagCols;
+    const int col0 = n0 / kFlagCols, chunks = flag_chunks(G);
     int any = 0;
     if (tid < kBM) any = flags[m0 + tid < M ? m0 + tid : M - 1];
-    if (tid < kBN / kFlagCols && col0 + tid < blocks) any |= flags[M + col0 + tid];
+    for (int i = tid; i < kBN / kFlagCols * chunks && col0 + i / chunks < blocks; i += 256)
+        any |= flags[M + col0 * chunks + i];
     any = __syncthreads_or(any);
-    const int far = any && wblock < blocks ? flags[M + wblock] : 0;
+    int far = 0;
+    if (any && wblock < blocks)
+        for (int i = 0; i < chunks; ++i) far |= flags[M + wblock * chunks + i];
     float* dst = out + int64_t(blockIdx.y) * M * N;
 #pragma unroll
     for (int a = 0; a < kTM; ++a)
@@ -494,7 +515,7 @@ F32Plan plan_f32(int M, int N, int K, int group_size) {
     const int64_t G = K / group_size;
     p.xsum = up(int64_t(M) * K * kParts * 2);
     p.flags = p.xsum + up(M * G * 4);
-    p.s_t = p.flags + up((int64_t(M) + (N + kFlagCols - 1) / kFlagCols) * 4);
+    p.s_t = p.flags + up((int64_t(M) + int64_t(N + kFlagCols - 1) / kFlagCols * flag_chunks(int(G))) * 4);
     p.b_t = p.s_t + up(padded_columns(N) * G * 4);
     p.o_t = p.b_t + up(N * G * 4);
     p.c_t = p.o_t + up(padded_columns(N) * G * 4);
@@ -517,9 +538,10 @@ bool f32_sizes_ok(int64_t M, int64_t N, int64_t K, int group_size) {
     // 32-bit lane offsets; grids of less than 2^32 threads (256 a block): the
     // preparation's rows and column blocks, the product's smallest tiles
     constexpr int64_t kBlocks = 1 << 24;
-    return M <= kBlocks && N <= kBlocks && K <= (1 << 20) && M + (N + kFlagCols - 1) / kFlagCols < kBlocks &&
-           ((M + 31) / 32) * ((N + kBN - 1) / kBN) < kBlocks - 8 &&
-           (group_size == 32 || group_size == 64 || group_size == 128) && K % kBK == 0 && K % group_size == 0;
+    return (group_size == 32 || group_size == 64 || group_size == 128) && K % kBK == 0 && K % group_size == 0 &&
+           M <= kBlocks && N <= kBlocks && K <= (1 << 20) &&
+           M + (N + kFlagCols - 1) / kFlagCols * flag_chunks(int(K) / group_size) < kBlocks &&
+           ((M + 31) / 32) * ((N + kBN - 1) / kBN) < kBlocks - 8;
 }
 
 }  // namespace
@@ -565,9 +587,17 @@ extern "C" int gdn_quantized_matmul_f32(const float* x, const void* w, const voi
     auto* o_t = reinterpret_cast<float*>(ws + p.o_t);
     auto* c_t = reinterpret_cast<uint8_t*>(ws + p.c_t);
     auto* partial = reinterpret_cast<float*>(ws + p.partial);
-    const int64_t sb_blocks = (int64_t(N) + kFlagCols - 1) / kFlagCols;
-    hipLaunchKernelGGL(prepare_f32_kernel, dim3(unsigned(M + sb_blocks)), dim3(256), 0, s, x, scales, biases, sb_dtype,
-                       pieces, xsum, flags, s_t, b_t, o_t, c_t, M, N, K, group_size);
+    const int64_t sb_blocks = (int64_t(N) + kFlagCols - 1) / kFlagCols * flag_chunks(K / group_size);
+    const auto prepare = [&](auto sb) {
+        using SB = decltype(sb);
+        using St = typename SB::storage;
+        hipLaunchKernelGGL(prepare_f32_kernel<SB>, dim3(unsigned(M + sb_blocks)), dim3(256), 0, s, x,
+                           static_cast<const St*>(scales), static_cast<const St*>(biases), pieces, xsum, flags, s_t,
+                           b_t, o_t, c_t, M, N, K, group_size);
+    };
+    if (sb_dtype == GDN_F32) prepare(ActF32{});
+    else if (sb_dtype == GDN_BF16) prepare(ActBF16{});
+    else prepare(ActF16{});
     if (int rc = check_launch("gdn_quantized_matmul_f32/prepare")) return rc;
 
     const int mt = (M + 16 * p.tm - 1) / (16 * p.tm), tiles = mt * ((N + kBN - 1) / kBN);
