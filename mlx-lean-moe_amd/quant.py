@@ -103,17 +103,25 @@ def _runs_dense(rows: int, N: int, K: int, quant: QuantScheme, sb_dtype: torch.d
     against kernel, us: 4096 -> 2048 at 66 rows 10 and 15, 200 rows 14 and 20,
     384 rows 18 and 26; 4096 -> 12352 at 200 rows 42 and 51)."""
 
-    dense = _dense_rows(rows, N, K)
-    if not _mid_rows(rows, N, K, quant.group_size, sb_dtype) or (dense and (kept or _transformed(*operands))):
-        return dense
-    if N * K <= 1 << 20:
-        return dense
-    if workspace_bytes(torch.bfloat16, sb_dtype, rows, N, K, quant.bits, quant.group_size):
+    if rows <= 64:
         return False
+    fallback, dense = _route(rows, N, K, quant.bits, quant.group_size, sb_dtype)
+    return dense or (fallback and (kept or _transformed(*operands)))
+
+
+@functools.lru_cache(maxsize=2048)
+def _route(rows: int, N: int, K: int, bits: int, group_size: int, sb_dtype: torch.dtype) -> tuple[bool, bool]:
+    """_dense_rows and _runs_dense of more than 64 rows by the sizes alone."""
+
+    fallback = _dense_rows(rows, N, K)
+    if not _mid_rows(rows, N, K, group_size, sb_dtype) or N * K <= 1 << 20:
+        return fallback, fallback
+    if workspace_bytes(torch.bfloat16, sb_dtype, rows, N, K, bits, group_size):
+        return fallback, False
     if N < 4096:
-        return True
+        return fallback, True
     tiles = -(-rows // _MID_TILE_ROWS) * -(-N // _MID_TILE_COLUMNS)
-    return K >= 2048 and tiles > _CUS
+    return fallback, K >= 2048 and tiles > _CUS
 
 
 def _transformed(*operands: torch.Tensor | None) -> bool:
