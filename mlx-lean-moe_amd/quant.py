@@ -13,7 +13,7 @@ scale (e8m0, e4m3 for nvfp4), no biases. Affine 4- and 8-bit projections of
 bf16 activations run on ``gdn_quantized_matmul``; the other schemes and
 activation dtypes dequantize on the GPU (``gdn_dequantize``) and multiply on
 the vendor BLAS, except that float32 rows times affine 4- and 8-bit codes run
-on ``gdn_quantized_matmul_f32``. Dense projections are ``x @ W.T``.
+on ``gdn_quantized_matmul_f32`` (small weights aside). Dense projections are ``x @ W.T``.
 """
 
 from __future__ import annotations
@@ -122,6 +122,20 @@ def _route(rows: int, N: int, K: int, bits: int, group_size: int, sb_dtype: torc
         return fallback, True
     tiles = -(-rows // _MID_TILE_ROWS) * -(-N // _MID_TILE_COLUMNS)
     return fallback, K >= 2048 and tiles > _CUS
+
+
+def _f32_rows(rows: int, N: int, K: int) -> bool:
+    """Whether float32 rows beyond the decode kernel's run on
+    gdn_quantized_matmul_f32 rather than on dequantized weights and the vendor
+    BLAS. Small weights are a few launches' time either way, and the kernel's
+    three launches lose (device time from graphs, us, kernel and library: 1024
+    -> 256 at 128 rows 18 and 11, 4096 rows 45 and 26; 4096 -> 256 22 and 14, 84
+    and 74; 1024 -> 2048 at 128 rows 23 and 16, 300 rows 36 and 24, 777 rows 39
+    and 42; 512 -> 4096 at 64 rows 22 and 16, 300 rows 24 and 23; but 4096 ->
+    1024 at 96 rows 27 and 27, 777 rows 65 and 76, and 256 -> 12352 at 128 rows
+    18 and 25)."""
+
+    return N * K > 1 << 21 or (N * K > 1 << 20 and rows > 512)
 
 
 def _transformed(*operands: torch.Tensor | None) -> bool:
@@ -320,7 +334,7 @@ def quantized_linear(x: torch.Tensor, tensors, quant: QuantScheme | None = None,
         return with_residual(x @ wd.to(x.dtype).T)
     x_f32 = (x.dtype == torch.float32 and rows <= 32
              and decode_kernel_takes(rows, K, quant.bits, quant.group_size, scales.dtype))
-    if (x.dtype == torch.float32 and not x_f32 and not _transformed(x, residual)
+    if (x.dtype == torch.float32 and not x_f32 and _f32_rows(rows, N, K) and not _transformed(x, residual)
             and f32_workspace_bytes(min(rows, _F32_ROWS), N, K, quant.bits, quant.group_size)):
         return _f32_matmul(x, w, scales, biases, quant, N, K, residual)
     if x.dtype != torch.bfloat16 and not x_f32:

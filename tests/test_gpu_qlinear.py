@@ -10,7 +10,7 @@ import torch
 
 import mlx_lean_moe_amd as gdn
 from mlx_lean_moe_amd import _lib
-from mlx_lean_moe_amd.quant import decode_kernel_takes, quantized_linear_split
+from mlx_lean_moe_amd.quant import _f32_matmul, decode_kernel_takes, quantized_linear_split
 from oracle import quant_ref as Q
 from oracle import gated_delta_ref as R
 from tests.helpers import assert_bf16_out_close, layer_inputs, layer_params
@@ -539,6 +539,12 @@ def test_scheme_matmul_special_scale_codes(gpu, mode, gs, M):
     assert (err <= 2.0 ** -20 * np.abs(ref[:, ok]) + 1e-5 * np.abs(ref[:, ok]).max()).all(), err.max()
 
 
+def _f32_kernel(x, W, q, residual=None):
+    """gdn_quantized_matmul_f32 as quantized_linear calls it, whatever the size
+    (small weights stay on the library there)."""
+    return _f32_matmul(x, W["weight"], W["scales"], W["biases"], q, W["weight"].shape[0], x.shape[-1], residual)
+
+
 def _f32_bound(x, words, s, b, bits, gs):
     """Worst-case rounding of gdn_quantized_matmul_f32: its products are
     exact, and every value passes at most 3 gs + 2 float32 sums inside a group
@@ -569,11 +575,11 @@ def test_float32_rows_in_three_bf16_pieces(gpu, M, N, K, bits, gs, sb):
     x = (rng.standard_normal((M, K)) * np.exp(rng.uniform(-6, 6, (M, K))) + 0.5).astype(np.float32)
     ref = Q.quantized_matmul(x, words, s, b, bits, gs, w_round="f32")
     assert _lib.load().gdn_quantized_matmul_f32_workspace_size(M, N, K, bits, gs) > 0
-    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs))
+    y = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs))
     assert y.dtype == torch.float32
     assert (np.abs(y.cpu().numpy() - ref) <= _f32_bound(x, words, s, b, bits, gs) + 1e-30).all()
     r = torch.tensor(rng.standard_normal((M, N)), dtype=torch.float32, device=gpu)
-    got = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs), residual=r)
+    got = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs), residual=r)
     assert torch.equal(got, y + r)
 
 
@@ -597,7 +603,7 @@ def test_float32_rows_outside_the_pieces_range(gpu, N, K):
     w = Q.dequantize(words, s, b, 4, 64, out="f32").astype(np.float64)
     with np.errstate(invalid="ignore"):
         ref = x.astype(np.float64) @ w.T
-    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
+    y = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
     finite = np.isfinite(x).all(axis=1)
     mass = np.abs(x[finite]).astype(np.float64) @ np.abs(w).T
     assert (np.abs(y[finite] - ref[finite]) <= 2 * K * 2.0 ** -24 * mass + 1e-38 * K).all()
@@ -717,7 +723,7 @@ def test_float32_rows_times_scales_out_of_range(gpu, N, K):
     with np.errstate(all="ignore"):
         w = (np.repeat(s, 64, 1).astype(np.float64) * q + np.repeat(b, 64, 1)).astype(np.float32).astype(np.float64)
         ref = x.astype(np.float64) @ w.T
-    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
+    y = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
     np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
     np.testing.assert_array_equal(np.isposinf(y), np.isposinf(ref))
     np.testing.assert_array_equal(np.isneginf(y), np.isneginf(ref))
@@ -806,7 +812,7 @@ def test_float32_rows_at_the_ends_of_their_range_do_not_overflow(gpu, bits, edge
     x = np.ldexp(np.where(rng.random((40, K)) < 0.3, -1.0, 1.0), edge).astype(np.float32)
     x[::2] = np.abs(x[::2])
     x[:, 5] = np.ldexp(1.0, edge - 20)
-    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
+    y = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
     want = np.ldexp(np.where(q0 == top, -1.0, 1.0), edge - 5)
     # float32 sums of the cancelling terms |q0| s |x| of each of K elements
     assert np.isfinite(y).all()
@@ -839,7 +845,7 @@ def test_float32_rows_with_outlying_activations_against_small_weights(gpu, N, K,
     w = np.repeat(s, gs, 1).astype(np.float64) * q + np.repeat(b, gs, 1)
     if exact_zero:
         assert (w[:, big] == 0).all()
-    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
+    y = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
     mass = np.abs(x).astype(np.float64) @ np.abs(w).T
     bound = (3 * gs + 2 * G + 22) * 2.0 ** -24 * 3 * mass
     assert (np.abs(y - x.astype(np.float64) @ w.T) <= bound).all()
@@ -871,7 +877,7 @@ def test_whole_prompts_of_float32_rows_outside_the_pieces_range(gpu, M, N, K, bi
     with np.errstate(invalid="ignore"):
         ref = x.astype(np.float64) @ w.T
         mass = np.abs(x).astype(np.float64) @ np.abs(w).T
-    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
+    y = _f32_kernel(torch.tensor(x, device=gpu), W, gdn.QuantScheme(bits, gs)).cpu().numpy()
     np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
     np.testing.assert_array_equal(y[2::4], ref[2::4].astype(np.float32))
     for rows in (slice(0, None, 4), slice(1, None, 4)):
@@ -896,7 +902,7 @@ def test_float32_rows_outside_the_pieces_range_cost_a_bounded_multiple(gpu):
             start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             start.record()
             for _ in range(4):
-                gdn.quantized_linear(t, W, gdn.QuantScheme(4, 64))
+                _f32_kernel(t, W, gdn.QuantScheme(4, 64))
             end.record()
             end.synchronize()
             best = min(best, start.elapsed_time(end))
@@ -974,3 +980,19 @@ def test_every_kernel_of_65_to_511_rows(gpu, M, N, K, bits, gs, sb):
     y = gdn.quantized_linear(xt, W, q)
     assert ((y.double() - ref).abs() <= bound + 2.0 ** -8 * ref.abs()).all()
     assert torch.equal(gdn.quantized_linear(xt, W, q, residual=r), y + r)
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(100, 256, 1024, False), (513, 2048, 1024, True), (512, 2048, 1024, False),
+                                          (40, 1024, 4096, True)])
+def test_float32_rows_take_the_kernel_by_the_weights_size(gpu, M, N, K, kernel, monkeypatch):
+    rng = np.random.default_rng(M)
+    words, s, b = _weights(rng, N, K, 4, 64, "bf16")
+    W = _dev_weights(gpu, words, s, b, "bf16")
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    calls = []
+    call = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (calls.append(name), call(name, *a))[1])
+    y = gdn.quantized_linear(torch.tensor(x, device=gpu), W, gdn.QuantScheme(4, 64)).cpu().numpy()
+    assert calls == ["gdn_quantized_matmul_f32" if kernel else "gdn_dequantize"]
+    w = Q.dequantize(words, s, b, 4, 64, out="f32").astype(np.float64)
+    assert (np.abs(y - x.astype(np.float64) @ w.T) <= K * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T)).all()

@@ -114,3 +114,15 @@ def test_transforms_are_seen_through_public_interfaces(monkeypatch):
     assert seen == [(True, True, False)] * 6
     with torch.no_grad():
         assert not _transformed(x.clone().requires_grad_())
+
+
+def test_float32_rows_of_small_weights_stay_on_the_library():
+    """Where gdn_quantized_matmul_f32's three launches are more than the
+    dequantization and product they replace."""
+    from mlx_lean_moe_amd.quant import _f32_rows
+
+    for rows, N, K in ((33, 256, 1024), (4096, 256, 1024), (4096, 256, 4096), (33, 2048, 1024), (512, 2048, 1024),
+                       (64, 4096, 512)):
+        assert not _f32_rows(rows, N, K), (rows, N, K)
+    for rows, N, K in ((777, 2048, 1024), (33, 12352, 256), (33, 1024, 4096), (1, 12352, 2048)):
+        assert _f32_rows(rows, N, K), (rows, N, K)
