@@ -61,15 +61,15 @@ __host__ __device__ constexpr int64_t padded_columns(int64_t n) { return (n + kB
 
 // Blocks 0 .. M - 1: row m of x as bf16 pieces, pieces[m][step][part][64]
 // (part 0 the upper 8 significant bits; truncation, so no piece can round up
-// to infinity), its group sums (in double, rounded once) and its flag. The
-// blocks after them, 64 columns by 32 groups each (a thread 8 consecutive ones
-// of a column, all loads in flight: a thread walking all of its column's groups
-// took 18 us for 128 rows and 1024 columns of 128 groups, this 8): s, b (o_t) and b' = b + c s in
-// float32, group-major, c as a byte (c_t[group][64-column block][n % 16][n / 16
-// % 4]: a word for the four columns of a lane of the product) and the flag (at
-// flags[M + column block * chunks + chunk]). The rows of s, b and c have
-// padded_columns(N) columns; those past N are read for outputs that are not
-// stored.
+// to infinity), its group sums (in double, rounded once) and its flag.
+// The blocks after them, 64 columns by 32 groups each, a thread 8 consecutive
+// ones of a column with all its loads in flight (a thread walking all of its
+// column's groups took 18 us for 128 rows and 1024 columns of 128 groups, this
+// 8): s, b (o_t) and b' = b + c s in float32, group-major, c as a byte
+// (c_t[group][64-column block][n % 16][n / 16 % 4]: a word for the four columns
+// of a lane of the product) and the flag (at flags[M + column block * chunks +
+// chunk]). The rows of s, b and c have padded_columns(N) columns; those past N
+// are read for outputs that are not stored.
 template <class SB>
 __global__ __launch_bounds__(256) void prepare_f32_kernel(
     const float* __restrict__ x, const typename SB::storage* __restrict__ scales,
